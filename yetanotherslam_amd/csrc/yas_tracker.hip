@@ -17,23 +17,33 @@
 //   update   one workgroup folds the partial rows in a fixed order, solves
 //            the 6x6 system in FP64 (the reference's Eigen LDLT, restated),
 //            applies T <- exp(xi) T in FP64 and keeps the best pose.
-// A full solve takes each update but the last at the start of the next
-// pass 1 instead: every workgroup of that pass folds the same rows and takes
-// the same step, one launch fewer per iteration with the same values.
+// A full solve runs all of its iterations in one launch (k_solve,
+// yas_solve_dev.hpp) where its workgroups can be resident at once; otherwise
+// it takes each update but the last at the start of the next pass 1: every
+// workgroup of that pass folds the same rows and takes the same step, one
+// launch fewer per iteration.  The values are the same either way.
 // Results are deterministic run to run.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "yas_internal.hpp"
 #include "yas_tracker_dev.hpp"
+#include "yas_solve_dev.hpp"
 #include "yas_server_dev.hpp"
 
 using namespace yas;
+
+constexpr int kMaxSolveDevices = 64;
+constexpr long long kSolveMaxPixels = 1 << 26;  // 32-bit byte offsets in yas_solve_dev.hpp
+// 20 ms: a solve takes under 0.5 ms, and its workgroups wait for a CU at
+// most as long as other streams' kernels hold one.
+constexpr unsigned long long kSolveWaitTicks = 2000000ull;
 
 namespace {
 
@@ -113,6 +123,21 @@ template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_step_pass1(Level L, TrackBufs B, StepArgs a, float* part_icp,
                                                     float* part_res, float angle_th, float dist_th) {
   pass1_at<ICP, RGB, true, true>(L, B, nullptr, part_icp, part_res, angle_th, dist_th, blockIdx.x, gridDim.x, &a);
+}
+// The whole solve in one launch (yas_solve_dev.hpp).  1024 threads a
+// workgroup, so 128 registers a lane; one workgroup per CU.  Bound by the
+// chain of an iteration (20 us at 640x480, 16.5 us at any small size): pixel
+// terms 3-5 us (VALU issue, four wavefronts a SIMD), statistics 1.5 us, three
+// messages between workgroups of about 1.3 us each, the step 4.3 us.  The
+// launch-per-pass iteration took 27 us (24 us at small sizes).
+template <bool ICP, bool RGB>
+__global__ void __launch_bounds__(kSolveThreads) k_solve(SolveArgs a) {
+  solve_body<ICP, RGB>(solve_lds(), a);
+}
+// Takes a solve whose workgroups did not meet; nothing to do otherwise.
+template <bool ICP, bool RGB>
+__global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a) {
+  solve_rescue<ICP, RGB>(a);
 }
 // A frame's tracker inputs in levels + 1 launches instead of seven per
 // level: the pointwise products of level l from level l - 1 (or from the
@@ -217,6 +242,8 @@ struct yas_tracker {
   TrackState* st;
   TrackState* st2;  // a solve's steps alternate between st and st2
   TrackState* host_st;
+  SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
+  unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
   float angle_th, dist_th;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
   float* raw_image;  // intensity uploaded by the host-image setters
@@ -315,7 +342,7 @@ static int launch_iteration(yas_tracker* t, int l, bool icp, bool rgb, bool do_s
 // saves one launch per iteration.  Step i reads the state buffer of step
 // i - 1 and writes the other one, and the ICP partial rows alternate the
 // same way, since that pass 1 reads the previous rows while writing its own.
-int yas_tracker_solve_async(yas_tracker* t) {
+static int solve_by_passes(yas_tracker* t) {
   const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
   hipStream_t s = t->ctx->stream;
   TrackState* S[2] = {t->st, t->st2};
@@ -366,6 +393,110 @@ int yas_tracker_solve_async(yas_tracker* t) {
     }
   if (i > 0) hipLaunchKernelGGL(k_update_into, dim3(1), dim3(256), 0, s, (const TrackState*)S[(i - 1) & 1], t->st, a);
   YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+
+// Whether this solve may run as one launch (k_solve): every workgroup must
+// find a CU at once, so only one stream's solves do at a time.  A stream
+// other than the last one's takes over once that one is idle; until then its
+// solves run as separate passes.  So do solves recorded into a graph, whose
+// replays nothing here orders.
+static std::mutex g_solve_mu;
+static struct {
+  bool used;
+  hipStream_t stream;
+} g_solve_last[kMaxSolveDevices];
+
+void yas_solve_forget_stream(int device, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(g_solve_mu);
+  if (device >= 0 && device < kMaxSolveDevices && g_solve_last[device].used && g_solve_last[device].stream == s)
+    g_solve_last[device].used = false;
+}
+
+static bool solve_fits(int device, const void* kernel, int grid) {
+  static std::mutex mu;
+  static int room[kMaxSolveDevices][3];  // workgroups that fit at once, + 1; 0 = not asked yet
+  int per_cu = 0, cus = 0;
+  const int k = kernel == (const void*)k_solve<true, true> ? 0 : kernel == (const void*)k_solve<true, false> ? 1 : 2;
+  std::lock_guard<std::mutex> lk(mu);
+  int& r = room[device][k];
+  if (r == 0) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kSolveThreads, 0) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+      (void)hipGetLastError();
+      per_cu = cus = 0;
+    }
+    r = per_cu * cus + 1;
+  }
+  return grid <= r - 1;
+}
+
+static bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+int yas_tracker_solve_async(yas_tracker* t) {
+  const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
+  hipStream_t s = t->ctx->stream;
+  const int device = t->ctx->device;
+  int grid = 0;
+  for (int l = t->P.levels - 1; l >= 0; --l)
+    if (t->P.iters[l] > 0) grid = groups_for(t->lv[l]);
+  if (grid == 0) return YAS_OK;  // no iteration at any level
+  const void* kernel = icp && rgb ? (const void*)k_solve<true, true>
+                                  : icp ? (const void*)k_solve<true, false> : (const void*)k_solve<false, true>;
+  if (device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels || is_capturing(s) ||
+      !solve_fits(device, kernel, grid)) return solve_by_passes(t);
+  std::lock_guard<std::mutex> lk(g_solve_mu);
+  auto& last = g_solve_last[device];
+  if (last.used && last.stream != s && (is_capturing(last.stream) || hipStreamQuery(last.stream) != hipSuccess)) {
+    (void)hipGetLastError();  // hipErrorNotReady is no failure
+    return solve_by_passes(t);
+  }
+  last.used = true;
+  last.stream = s;
+  SolveArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.levels = t->P.levels;
+  for (int l = 0; l < t->P.levels; ++l) {
+    a.lv[l] = t->lv[l];
+    a.tb[l] = bufs(t, l);
+    a.iters[l] = t->P.iters[l];
+    a.groups[l] = groups_for(t->lv[l]);
+  }
+  a.mode = t->P.mode;
+  a.angle_th = t->angle_th;
+  a.dist_th = t->dist_th;
+  a.wrh = t->P.w_rgb_h; a.wrb = t->P.w_rgb_b; a.wih = t->P.w_icp_h; a.wib = t->P.w_icp_b;
+  a.st = t->st;
+  a.x = t->xchg;
+  a.part_icp = t->part_icp; a.part_res = t->part_res; a.part_rgb = t->part_rgb;
+  a.wait_ticks = t->wait_ticks;
+  if (icp && rgb) {
+    hipLaunchKernelGGL((k_solve<true, true>), dim3(grid), dim3(kSolveThreads), 0, s, a);
+    hipLaunchKernelGGL((k_solve_rescue<true, true>), dim3(1), dim3(256), 0, s, a);
+  } else if (icp) {
+    hipLaunchKernelGGL((k_solve<true, false>), dim3(grid), dim3(kSolveThreads), 0, s, a);
+    hipLaunchKernelGGL((k_solve_rescue<true, false>), dim3(1), dim3(256), 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_solve<false, true>), dim3(grid), dim3(kSolveThreads), 0, s, a);
+    hipLaunchKernelGGL((k_solve_rescue<false, true>), dim3(1), dim3(256), 0, s, a);
+  }
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+
+// The bound of the one-launch solve's waits, for tests that want one to run
+// out: 0 makes every wait that finds its words missing at the first look
+// give up.
+extern "C" int yas_tracker_set_wait_ticks(yas_tracker* t, unsigned long long ticks) {
+  YAS_REQUIRE(t, "null tracker");
+  t->wait_ticks = ticks;
   return YAS_OK;
 }
 
@@ -476,6 +607,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   // RGBDTracking.cu:432-433: sin(20 deg) computed in float, 1 cm.
   t->angle_th = (float)std::sin(20.f * 3.14159254f / 180.f);
   t->dist_th = 0.01f;
+  t->wait_ticks = kSolveWaitTicks;
   hipError_t e = hipSuccess;
   auto alloc = [&](void** p, size_t bytes) {
     if (e == hipSuccess) e = hipMalloc(p, bytes);
@@ -506,6 +638,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   alloc((void**)&t->part_rgb, sizeof(float) * 32 * kRedGroups);
   alloc((void**)&t->st, sizeof(TrackState));
   alloc((void**)&t->st2, sizeof(TrackState));
+  alloc((void**)&t->xchg, sizeof(SolveXchg));
   if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_st, sizeof(TrackState), hipHostMallocDefault);
   if (e != hipSuccess) {
     yas_set_error("yas_tracker_create: %s", hipGetErrorString(e));
@@ -524,6 +657,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   }
   YAS_HIP(hipMemsetAsync(t->st, 0, sizeof(TrackState), ctx->stream));
   YAS_HIP(hipMemsetAsync(t->st2, 0, sizeof(TrackState), ctx->stream));
+  YAS_HIP(hipMemsetAsync(t->xchg, 0, sizeof(SolveXchg), ctx->stream));
   int rc = yas_tracker_init_identity_async(t);
   if (rc) {
     yas_tracker_destroy(t);
@@ -549,6 +683,7 @@ int yas_tracker_destroy(yas_tracker* t) {
   hipFree(t->part_rgb);
   hipFree(t->st);
   hipFree(t->st2);
+  hipFree(t->xchg);
   hipFree(t->raw_depth);
   hipFree(t->raw_image);
   if (t->host_st) hipHostFree(t->host_st);

@@ -461,8 +461,7 @@ __device__ inline float bilerp(const float* m, int w, float x, float y) {
 // ImageProc.cu:42-61: reference pixel k at its inverse depth, moved by the
 // warp (RK, t); w = -1 where the inverse depth is 0.  Both passes evaluate it
 // (the same operations, so the same floats) instead of storing it.
-__device__ inline float4 warp_ref(const Level& L, const float* wp, int k, float iz) {
-  const int y = k / L.w, x = k - y * L.w;
+__device__ inline float4 warp_ref_xy(const float* wp, int x, int y, float iz) {
   float4 p = make_float4(0.f, 0.f, 0.f, -1.f);
   if (iz > 0.0f) {
     float z = 1.0f / iz;
@@ -472,6 +471,10 @@ __device__ inline float4 warp_ref(const Level& L, const float* wp, int k, float 
     p = make_float4(px, py, pz, 1.0f);
   }
   return p;
+}
+__device__ inline float4 warp_ref(const Level& L, const float* wp, int k, float iz) {
+  const int y = k / L.w;
+  return warp_ref_xy(wp, k - y * L.w, y, iz);
 }
 
 // TrackingUtils.h:73-151 with the warp of ImageProc.cu:42-61 fused in; the
@@ -842,33 +845,35 @@ __device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* 
   constexpr int n = 6;
   const int lane = threadIdx.x & 63;
   const int r = lane < n ? lane : n - 1;
-  double d[n];
+  // the pivots, from the diagonal as floats (the same order as the doubles')
+  float d[n];
   int p[n];
 #pragma unroll
   for (int i = 0; i < n; ++i) {
-    d[i] = (double)H[i * n + i];
+    d[i] = fabsf(H[i * n + i]);
     p[i] = i;
   }
   bool stop = false;
 #pragma unroll
-  for (int k = 0; k < n; ++k) {
+  for (int k = 0; k < n - 1; ++k) {
     int big = k;
-    double bv = fabs(d[k]);
+    float bv = d[k];
 #pragma unroll
-    for (int i = k + 1; i < n; ++i)
-      if (fabs(d[i]) > bv) {
-        bv = fabs(d[i]);
-        big = i;
-      }
+    for (int i = k + 1; i < n; ++i) {
+      const bool gt = d[i] > bv;
+      bv = gt ? d[i] : bv;
+      big = gt ? i : big;
+    }
+    if (k == 0) stop = !(bv > 0.0f);  // no pivot at all
+    const float dk = d[k];
+    const int pk = p[k];
 #pragma unroll
     for (int i = k + 1; i < n; ++i) {
       const bool sw = i == big;
-      swap_if(sw, d[k], d[i]);
-      const int pk = p[k], pi = p[i];
-      p[k] = sw ? pi : pk;
-      p[i] = sw ? pk : pi;
+      p[k] = sw ? p[i] : p[k];
+      d[i] = sw ? dk : d[i];
+      p[i] = sw ? pk : p[i];
     }
-    if (k == 0 && !(fabs(d[0]) > 0.0)) stop = true;
   }
   if (stop) {
 #pragma unroll
@@ -923,9 +928,22 @@ __device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* 
   for (int i = 0; i < n; ++i) x[i] = scratch[i];
 }
 
-// SE(3) exponential, twist (rho, omega), Rodrigues' formula.
-__device__ inline void se3_exp(const double* xi, double* T) {
+// SE(3) exponential, twist (rho, omega), Rodrigues' formula, by a whole
+// wavefront: lane 4 i + j < 16 writes element (i, j) of the 4x4 result to E
+// (LDS).  Lanes 0..8 first leave W = [omega]x in `w9` (LDS) and the result's
+// elements are formed one per lane, W^2, R = I + A W + B W^2 and
+// V = I + B W + C W^2 each summed left to right; in every lane alike they
+// were 130 double operations and 72 registers.
+__device__ inline void se3_exp_wave(const double* xi, double* w9, double* E) {
+  const int lane = threadIdx.x & 63;
   const double* w = xi + 3;
+  if (lane < 9) {
+    const int i = lane / 3, j = lane - 3 * i;
+    const int axis = 3 - i - j;  // of the off-diagonal element (i, j)
+    const double v = axis == 0 ? w[0] : axis == 1 ? w[1] : w[2];
+    const bool neg = (i == 0 && j == 1) || (i == 1 && j == 2) || (i == 2 && j == 0);
+    w9[lane] = i == j ? 0.0 : neg ? -v : v;
+  }
   double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
   double th = sqrt(th2);
   double A, B, C;
@@ -934,25 +952,38 @@ __device__ inline void se3_exp(const double* xi, double* T) {
     B = 0.5 - th2 / 24.0;
     C = 1.0 / 6.0 - th2 / 120.0;
   } else {
-    A = sin(th) / th;
-    B = (1.0 - cos(th)) / th2;
-    C = (th - sin(th)) / (th2 * th);
+    // A = sin / th, B = (1 - cos) / th2, C = (th - sin) / (th2 th): one
+    // division, each quotient in a lane of its own
+    const double sn = sin(th), cs = cos(th);
+    const double num = lane == 0 ? sn : lane == 1 ? 1.0 - cs : th - sn;
+    const double den = lane == 0 ? th : lane == 1 ? th2 : th2 * th;
+    const double quo = num / den;
+    A = lane_value(quo, 0);
+    B = lane_value(quo, 1);
+    C = lane_value(quo, 2);
   }
-  double W[9] = {0, -w[2], w[1], w[2], 0, -w[0], -w[1], w[0], 0};
-  double W2[9], Rm[9], V[9];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) W2[3 * i + j] = W[3 * i] * W[j] + W[3 * i + 1] * W[3 + j] + W[3 * i + 2] * W[6 + j];
-  for (int i = 0; i < 9; ++i) {
-    double I = (i % 4 == 0) ? 1.0 : 0.0;
-    Rm[i] = I + A * W[i] + B * W2[i];
-    V[i] = I + B * W[i] + C * W2[i];
+  wave_lds_sync();
+  if (lane < 16) {
+    const int i = lane >> 2, j = lane & 3;
+    double e = i == j ? 1.0 : 0.0;
+    if (i < 3) {
+      const double r0 = w9[3 * i], r1 = w9[3 * i + 1], r2 = w9[3 * i + 2];
+      // the translation's lane (j = 3) needs all of V's row, the others one element
+      double v[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int c = j < 3 ? j : k;
+        const double W = c == 0 ? r0 : c == 1 ? r1 : r2;
+        const double W2 = r0 * w9[c] + r1 * w9[3 + c] + r2 * w9[6 + c];
+        const double I = c == i ? 1.0 : 0.0;
+        const double p = j < 3 ? A : B, q = j < 3 ? B : C;
+        v[k] = I + p * W + q * W2;
+      }
+      e = j < 3 ? v[0] : v[0] * xi[0] + v[1] * xi[1] + v[2] * xi[2];
+    }
+    E[lane] = e;
   }
-  for (int i = 0; i < 3; ++i) {
-    for (int j = 0; j < 3; ++j) T[4 * i + j] = Rm[3 * i + j];
-    T[4 * i + 3] = V[3 * i] * xi[0] + V[3 * i + 1] * xi[1] + V[3 * i + 2] * xi[2];
-  }
-  T[12] = T[13] = T[14] = 0.0;
-  T[15] = 1.0;
+  wave_lds_sync();
 }
 
 // RankUpdateHessian<6,7> (TrackingUtils.h:45-58).
@@ -972,8 +1003,8 @@ __device__ inline void unpack29(const float* s, float* H, float* b) {
 // est_out (each when not null).  Each value is formed by the operations of
 // the serial form, in its order: H and b one element per lane
 // (RankUpdateHessian's packing, the RGB term weighted first), the solve by
-// ldlt_solve6_wave, the exponential in every lane alike, and E * est one
-// element per lane for lanes 0..15.  lds_H (36), lds_b (6), lds_x (6) and
+// ldlt_solve6_wave, the exponential by se3_exp_wave, and E * est one element
+// per lane for lanes 0..15.  lds_H (36), lds_b (6), lds_x (6), lds_W (9) and
 // lds_E (16) are LDS.
 __device__ __attribute__((always_inline)) inline void gn_step_wave0(const float (*sums)[32], const double* s_est,
                                                                     int s_good, float s_last_err, TrackState* st,
@@ -981,7 +1012,7 @@ __device__ __attribute__((always_inline)) inline void gn_step_wave0(const float 
                                                                     int first_of_level, int do_step, int record,
                                                                     float wrh, float wrb, float wih, float wib,
                                                                     float* lds_H, float* lds_b, double* lds_x,
-                                                                    double* lds_E) {
+                                                                    double* lds_W, double* lds_E) {
   const int lane = threadIdx.x & 63;
   if (st && lane == 0 && record && gi) st->icp_inliers = (int)sums[0][28];
   if (st && lane == 0 && record && gr) st->rgb_inliers = (int)sums[1][28];
@@ -1025,13 +1056,7 @@ __device__ __attribute__((always_inline)) inline void gn_step_wave0(const float 
     if (st && lane == 0) st->good = 0;
     return;
   }
-  double E[16];
-  se3_exp(xi, E);
-  if (lane < 16) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) lds_E[q] = E[q];
-  }
-  wave_lds_sync();
+  se3_exp_wave(xi, lds_W, lds_E);
   if (lane < 16) {
     const int i = lane >> 2, j = lane & 3;
     const double t = lds_E[4 * i] * s_est[j] + lds_E[4 * i + 1] * s_est[4 + j] + lds_E[4 * i + 2] * s_est[8 + j] +
@@ -1061,7 +1086,7 @@ __device__ __attribute__((always_inline)) inline void gn_update(const TrackState
   __shared__ int s_good;
   __shared__ float s_last_err;
   __shared__ float s_H[36], s_b[6];  // wavefront 0's step
-  __shared__ double s_x[6], s_E[16];
+  __shared__ double s_x[6], s_W[9], s_E[16];
   // the state the step reads, loaded alongside the partial rows
   if (threadIdx.x < 16) s_est[threadIdx.x] = st_in->est[threadIdx.x];
   if (threadIdx.x == 16) s_good = st_in->good;
@@ -1104,7 +1129,7 @@ __device__ __attribute__((always_inline)) inline void gn_update(const TrackState
   if (threadIdx.x >= 64) return;
   if (est_out && threadIdx.x < 16) est_out[threadIdx.x] = s_est[threadIdx.x];  // the pose where no step is taken
   gn_step_wave0(sums, s_est, s_good, s_last_err, write ? st_out : nullptr, est_out, gi, gr, mode, first_of_level,
-                do_step, record, wrh, wrb, wih, wib, s_H, s_b, s_x, s_E);
+                do_step, record, wrh, wrb, wih, wib, s_H, s_b, s_x, s_W, s_E);
 }
 __device__ inline void update_at(TrackState* st, const float* part_icp, int gi, const float* part_rgb, int gr,
                                  int mode, int first_of_level, int do_step, int record, float wrh, float wrb, float wih,

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <vector>
 
+#include "yas_frame_dev.hpp"
 #include "yas_internal.hpp"
 #include "yas_raycast_dev.hpp"
 #include "yas_server_dev.hpp"
@@ -29,26 +30,27 @@ TrackState* yas_tracker_state_dev(yas_tracker* t);
 int yas_tracker_solve_async(yas_tracker* t);
 const double* yas_tracker_result_dev(yas_tracker* t);
 const int* yas_tracker_good_dev(yas_tracker* t);
-int yas_tracker_set_tracking_image_dev(yas_tracker* t, const float* g, size_t pitch);
-int yas_tracker_prepare_frame_dev(yas_tracker* t, const float* vmap, size_t vpitch, const float* g, size_t gpitch,
-                                  const float* d, size_t dpitch);
-int yas_tracker_set_tracking_depth_dev(yas_tracker* t, const float* d, size_t pitch);
+int yas_tracker_frame_args(yas_tracker* t, ImageArgs<SrcRgb>& im, DepthArgs<SrcU16>& d);
+int yas_tracker_coarse_levels(yas_tracker* t);
+int yas_tracker_set_model_dev(yas_tracker* t, const float* vmap, size_t pitch);
 int yas_tracker_unswap_copies(yas_tracker* t, RefRestore& r);
 
 namespace {
 
-// The start of a frame in one launch of 64x4-pixel workgroups: depth in
-// metres and the gray image; from the first workgroup the map's float pose
-// pair of T_last with its visible counter cleared (for the ray cast, or the
-// first frame's fusion) and the tracker's state reset to identity; from the
-// first ncell threads the ray caster's z-range cells reset.
+// The start of a frame in one launch: depth in metres (64x4-pixel tiles);
+// from the first workgroup the map's float pose pair of T_last with its
+// visible counter cleared (for the ray cast, or the first frame's fusion) and
+// the tracker's state reset to identity; from the first ncell threads the ray
+// caster's z-range cells reset.  On the first frame also the gray image;
+// on later ones the tracker's image and depth levels, straight from the
+// camera's images.
 struct FrameBegin {
   const uint16_t* depth_in;
   size_t dpitch;
   const uint8_t* rgb;
   size_t cpitch;
   float* depth;  // pitch fpitch
-  float* gray;   // pitch fpitch
+  float* gray;   // pitch fpitch; null after the first frame
   size_t fpitch;
   float scale;
   int W, H, gray_mode;
@@ -59,15 +61,23 @@ struct FrameBegin {
   unsigned* zmin;
   unsigned* zmax;
   int ncell;
+  int tiles_x, tiles;  // of the depth conversion
+  int image_tiles, depth_tiles;  // of the levels (0 on the first frame)
+  ImageArgs<SrcRgb> im;
+  DepthArgs<SrcU16> d;
 };
 
+// Workgroups: the image tiles first (the longest), then the conversion's,
+// then the depth levels'.
 __global__ void __launch_bounds__(256) k_frame_begin(FrameBegin a) {
-  const int gid = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+  __shared__ ImageLds S;
+  int b = blockIdx.x;
+  const int gid = b * blockDim.x + threadIdx.x;
   if (gid < a.ncell) {
     a.zmin[gid] = __float_as_uint(kZrangeFar);
     a.zmax[gid] = 0u;
   }
-  if (blockIdx.x == 0 && blockIdx.y == 0) {
+  if (b == 0) {
     if (threadIdx.x == 0) {
       PosePair p;
       pose_pair_from(a.T_last, p);
@@ -76,12 +86,22 @@ __global__ void __launch_bounds__(256) k_frame_begin(FrameBegin a) {
     }
     track_init_identity_at(a.st);
   }
-  const int x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (x < a.W && y < a.H) {
-    const uint16_t d = ((const uint16_t*)((const char*)a.depth_in + (size_t)y * a.dpitch))[x];
-    ((float*)((char*)a.depth + (size_t)y * a.fpitch))[x] = (float)d * a.scale;
+  if (b < a.image_tiles) {
+    image_tile(a.im, b, S);
+    return;
   }
-  rgb_to_gray_at(a.rgb, a.cpitch, a.gray, a.fpitch, a.W, a.H, a.gray_mode, blockIdx.x, blockIdx.y);
+  b -= a.image_tiles;
+  if (b < a.tiles) {
+    const int bx = b % a.tiles_x, by = b / a.tiles_x;
+    const int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
+    if (x < a.W && y < a.H) {
+      const uint16_t d = ((const uint16_t*)((const char*)a.depth_in + (size_t)y * a.dpitch))[x];
+      ((float*)((char*)a.depth + (size_t)y * a.fpitch))[x] = (float)d * a.scale;
+    }
+    if (a.gray) rgb_to_gray_at(a.rgb, a.cpitch, a.gray, a.fpitch, a.W, a.H, a.gray_mode, bx, by);
+    return;
+  }
+  depth_tile(a.d, b - a.tiles);
 }
 
 // The frame's outcome (one thread), which then writes the map's pose pair
@@ -328,7 +348,7 @@ int yas_pipeline_step(yas_pipeline* p, const uint16_t* depth, size_t dpitch, con
     a.rgb = rgb;
     a.cpitch = cpitch;
     a.depth = p->depth;
-    a.gray = p->gray;
+    a.gray = p->frames == 0 ? p->gray : nullptr;
     a.fpitch = fp;
     a.scale = (float)(1.0 / (double)p->depth_scale);
     a.W = W;
@@ -339,7 +359,17 @@ int yas_pipeline_step(yas_pipeline* p, const uint16_t* depth, size_t dpitch, con
     a.ctr = yas_map_view(p->map).ctr;
     a.st = yas_tracker_state_dev(p->trk);
     yas_raycaster_zrange_dev(p->rc, &a.zmin, &a.zmax, &a.ncell);
-    hipLaunchKernelGGL(k_frame_begin, dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, s, a);
+    a.tiles_x = (W + 63) / 64;
+    a.tiles = a.tiles_x * ((H + 3) / 4);
+    a.image_tiles = a.depth_tiles = 0;
+    if (p->frames > 0) {
+      yas_tracker_frame_args(p->trk, a.im, a.d);
+      a.im.src = SrcRgb{rgb, cpitch, p->gray_mode};
+      a.d.src = SrcU16{depth, dpitch, a.scale};
+      a.image_tiles = a.im.tiles;
+      a.depth_tiles = a.d.t.first[a.d.t.n];
+    }
+    hipLaunchKernelGGL(k_frame_begin, dim3(a.image_tiles + a.tiles + a.depth_tiles), dim3(256), 0, s, a);
     YAS_LAUNCH_CHECK();
   }
   if ((rc = mark(1))) return rc;
@@ -357,8 +387,8 @@ int yas_pipeline_step(yas_pipeline* p, const uint16_t* depth, size_t dpitch, con
     // TrackRGBD (Tracking.cpp:162-197)
     if ((rc = yas_raycast_prepared(p->rc, p->map, detail ? ev[2] : nullptr, kpair(0)))) return rc;
     if ((rc = mark(3))) return rc;
-    if ((rc = yas_tracker_prepare_frame_dev(p->trk, (const float*)yas_raycaster_vmap_dev(p->rc), (size_t)W * 16,
-                                            p->gray, fp, p->depth, fp)))
+    if ((rc = yas_tracker_coarse_levels(p->trk))) return rc;
+    if ((rc = yas_tracker_set_model_dev(p->trk, (const float*)yas_raycaster_vmap_dev(p->rc), (size_t)W * 16)))
       return rc;
     if ((rc = mark(4))) return rc;
     if ((rc = yas_tracker_solve_async(p->trk))) return rc;

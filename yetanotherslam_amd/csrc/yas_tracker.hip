@@ -33,6 +33,8 @@
 #include <vector>
 
 #include "yas_internal.hpp"
+#include "yas_frame_dev.hpp"
+#include "yas_frame_host.hpp"
 #include "yas_tracker_dev.hpp"
 #include "yas_solve_dev.hpp"
 #include "yas_server_dev.hpp"
@@ -46,10 +48,6 @@ constexpr long long kSolveMaxPixels = 1 << 26;  // 32-bit byte offsets in yas_so
 constexpr unsigned long long kSolveWaitTicks = 2000000ull;
 
 namespace {
-
-__global__ void __launch_bounds__(256) k_copy_f32(const float* src, size_t sp, float* dst, int W, int H) {
-  copy_f32_at(src, sp, dst, W, H, blockIdx.x, blockIdx.y);
-}
 
 __global__ void __launch_bounds__(256) k_rgb_to_gray(const uint8_t* rgb, size_t sp, float* dst, size_t dp, int W,
                                                      int H, int mode) {
@@ -74,14 +72,6 @@ __global__ void __launch_bounds__(256) k_pyrdown_depth(const float* s, size_t sp
   pyrdown_depth_at(s, sp, o, dp, W, H, blockIdx.x, blockIdx.y);
 }
 
-__global__ void __launch_bounds__(256) k_pyrdown_vmap(const float4* s, size_t sp, float4* o, size_t dp, int W, int H) {
-  pyrdown_vmap_at(s, sp, o, dp, W, H, blockIdx.x, blockIdx.y);
-}
-
-__global__ void __launch_bounds__(256) k_copy_f4(const float4* s, size_t sp, float4* o, int W, int H) {
-  copy_f4_at(s, sp, o, W, H, blockIdx.x, blockIdx.y);
-}
-
 __global__ void __launch_bounds__(256) k_vertex(const float* inv, size_t sp, float4* v, size_t dp, int W, int H,
                                                 float invfx, float invfy, float cx, float cy, float cut) {
   vertex_at(inv, sp, v, dp, W, H, invfx, invfy, cx, cy, cut, blockIdx.x, blockIdx.y);
@@ -89,10 +79,6 @@ __global__ void __launch_bounds__(256) k_vertex(const float* inv, size_t sp, flo
 
 __global__ void __launch_bounds__(256) k_normal(const float4* v, size_t sp, float4* n, size_t dp, int W, int H) {
   normal_at(v, sp, n, dp, W, H, blockIdx.x, blockIdx.y);
-}
-
-__global__ void __launch_bounds__(256) k_icp_point(const float4* v, float4* o, int W, int H) {
-  icp_point_at(v, (size_t)W * 16, o, W, H, blockIdx.x, blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256) k_vmap_to_depth(const float4* v, size_t sp, float* d, size_t dp, int W, int H) {
@@ -139,83 +125,13 @@ template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a) {
   solve_rescue<ICP, RGB>(a);
 }
-// A frame's tracker inputs in levels + 1 launches instead of seven per
-// level: the pointwise products of level l from level l - 1 (or from the
-// frame at level 0): intensity, inverse depth and vertices of the current
-// frame, and the model's vertices; and the neighbourhood products of level
-// l: gradients and both ICP point maps (vertex and normal), which need the
-// products of level l but nothing of level l + 1, so they share a launch
-// with those.  Each pixel gets the value the separate kernels give it.
-struct FrameLevel {
-  int l, w, h, pw, ph;  // level, its size, the size of level l - 1
-  float invfx, invfy, cx, cy;
-  const float* gray;   // level 0 sources
-  size_t gp;
-  const float* depth;
-  size_t dp;
-  const float4* vmap;
-  size_t vp;
-  const float* int_prev;  // level l - 1
-  const float* inv_prev;
-  const float4* refv_prev;
-  float* cur_int;  // level l
-  float* cur_inv;
-  float4* cur_v;
-  float4* ref_v;
-  float* gx;
-  float* gy;
-  float4* cur_p;  // ICP point maps
-  float4* ref_p;
-};
-__device__ inline void frame_level_px(const FrameLevel& a, int x, int y) {
-  if (x >= a.w || y >= a.h) return;
-  const size_t k = (size_t)y * a.w + x;
-  float in, iv;
-  float4 rv;
-  if (a.l == 0) {
-    in = ld(a.gray, a.gp, x, y);
-    iv = invdepth_of(ld(a.depth, a.dp, x, y));
-    rv = ((const float4*)((const char*)a.vmap + (size_t)y * a.vp))[x];
-  } else {
-    in = pyrdown_gauss_px(a.int_prev, (size_t)a.pw * 4, a.pw, a.ph, x, y);
-    iv = pyrdown_depth_px(a.inv_prev, (size_t)a.pw * 4, a.w, a.h, x, y);
-    rv = pyrdown_vmap_px(a.refv_prev, (size_t)a.pw * 16, a.w, a.h, x, y);
-  }
-  a.cur_int[k] = in;
-  a.cur_inv[k] = iv;
-  a.cur_v[k] = vertex_of(iv, x, y, a.invfx, a.invfy, a.cx, a.cy, 3.0f);
-  a.ref_v[k] = rv;
+// All levels of an image, a depth image or a model in one launch (yas_frame_dev.hpp).
+__global__ void __launch_bounds__(256) k_image_levels(ImageArgs<SrcF32> a) {
+  __shared__ ImageLds S;
+  image_tile(a, blockIdx.x, S);
 }
-__device__ inline void frame_level_nb_px(const FrameLevel& a, int x, int y) {
-  if (x >= a.w || y >= a.h) return;
-  const size_t k = (size_t)y * a.w + x;
-  float gxv, gyv;
-  gradient_px(a.cur_int, (size_t)a.w * 4, a.w, a.h, x, y, gxv, gyv);
-  a.gx[k] = gxv;
-  a.gy[k] = gyv;
-  store_icp_point(a.cur_p, a.w * a.h, (int)k, icp_point_px(a.cur_v, (size_t)a.w * 16, a.w, a.h, x, y));
-  store_icp_point(a.ref_p, a.w * a.h, (int)k, icp_point_px(a.ref_v, (size_t)a.w * 16, a.w, a.h, x, y));
-}
-__global__ void __launch_bounds__(256) k_frame_level(FrameLevel a) {
-  frame_level_px(a, blockIdx.x * 64 + (threadIdx.x & 63), blockIdx.y * 4 + (threadIdx.x >> 6));
-}
-__global__ void __launch_bounds__(256) k_frame_level_nb(FrameLevel a) {
-  frame_level_nb_px(a, blockIdx.x * 64 + (threadIdx.x & 63), blockIdx.y * 4 + (threadIdx.x >> 6));
-}
-// Level l's pointwise products and level l - 1's neighbourhood products,
-// which do not depend on each other, in one launch: the first `nprod`
-// workgroups take the products' 64x4 tiles, the others the neighbourhood
-// products'.
-__global__ void __launch_bounds__(256) k_frame_level_pair(FrameLevel prod, FrameLevel nb, int nprod) {
-  const int b = blockIdx.x;
-  if (b < nprod) {
-    const int tx = (prod.w + 63) >> 6;
-    frame_level_px(prod, (b % tx) * 64 + (threadIdx.x & 63), (b / tx) * 4 + (threadIdx.x >> 6));
-  } else {
-    const int tx = (nb.w + 63) >> 6, c = b - nprod;
-    frame_level_nb_px(nb, (c % tx) * 64 + (threadIdx.x & 63), (c / tx) * 4 + (threadIdx.x >> 6));
-  }
-}
+__global__ void __launch_bounds__(256) k_depth_levels(DepthArgs<SrcF32> a) { depth_tile(a, blockIdx.x); }
+__global__ void __launch_bounds__(256) k_model_levels(ModelArgs a) { model_tile(a, blockIdx.x); }
 __global__ void k_track_init(TrackState* st, Mat44 T) { track_init_at(st, T.m); }
 __global__ void k_track_init_identity(TrackState* st) { track_init_identity_at(st); }
 
@@ -251,49 +167,37 @@ struct yas_tracker {
 
 static int image_pyramid(yas_tracker* t, const float* g, size_t pitch, float** pyr, bool grads) {
   hipStream_t s = t->ctx->stream;
-  hipLaunchKernelGGL(k_copy_f32, grid64x4(t->W, t->H), dim3(256), 0, s, g, pitch, pyr[0], t->W, t->H);
-  for (int l = 1; l < t->P.levels; ++l) {
-    const Level& a = t->lv[l - 1];
-    const Level& b = t->lv[l];
-    hipLaunchKernelGGL(k_pyrdown_gauss, dim3((b.w + 15) / 16, (b.h + 15) / 16), dim3(256), 0, s, pyr[l - 1],
-                       (size_t)a.w * 4, a.w, a.h, pyr[l], (size_t)b.w * 4, b.w, b.h);
+  // three levels a launch; the next launch starts at the last of them
+  for (int base = 0; base == 0 || base + 1 < t->P.levels; base += kImageLevels - 1) {
+    ImageArgs<SrcF32> a;
+    if (base == 0) a.src = SrcF32{g, pitch};
+    else a.src = SrcF32{pyr[base], (size_t)t->lv[base].w * 4};
+    fill_image(a, t->lv, t->P.levels, base, pyr, grads ? t->gx : nullptr, grads ? t->gy : nullptr);
+    hipLaunchKernelGGL(k_image_levels, dim3(a.tiles), dim3(256), 0, s, a);
   }
-  if (grads)
-    for (int l = 0; l < t->P.levels; ++l) {
-      const Level& a = t->lv[l];
-      hipLaunchKernelGGL(k_gradient, grid64x4(a.w, a.h), dim3(256), 0, s, pyr[l], (size_t)a.w * 4, t->gx[l], t->gy[l],
-                         (size_t)a.w * 4, a.w, a.h);
-    }
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
 static int depth_pyramid(yas_tracker* t, const float* d, size_t pitch, float** inv, float4** v, float4** pt) {
-  hipStream_t s = t->ctx->stream;
-  for (int l = 0; l < t->P.levels; ++l) {
-    const Level& a = t->lv[l];
-    if (l == 0)
-      hipLaunchKernelGGL(k_invdepth, grid64x4(a.w, a.h), dim3(256), 0, s, d, pitch, inv[0], (size_t)a.w * 4, a.w, a.h);
-    else
-      hipLaunchKernelGGL(k_pyrdown_depth, grid64x4(a.w, a.h), dim3(256), 0, s, inv[l - 1], (size_t)t->lv[l - 1].w * 4,
-                         inv[l], (size_t)a.w * 4, a.w, a.h);
-    hipLaunchKernelGGL(k_vertex, grid64x4(a.w, a.h), dim3(256), 0, s, inv[l], (size_t)a.w * 4, v[l], (size_t)a.w * 16,
-                       a.w, a.h, a.invfx, a.invfy, a.cx, a.cy, 3.0f);
-    hipLaunchKernelGGL(k_icp_point, grid64x4(a.w, a.h), dim3(256), 0, s, v[l], pt[l], a.w, a.h);
-  }
+  DepthArgs<SrcF32> a;
+  a.src = SrcF32{d, pitch};
+  fill_depth(a, t->lv, t->P.levels, inv, v, pt);
+  hipLaunchKernelGGL(k_depth_levels, dim3(a.t.first[a.t.n]), dim3(256), 0, t->ctx->stream, a);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
-static int model_pyramid(yas_tracker* t) {
-  hipStream_t s = t->ctx->stream;
+static int model_pyramid(yas_tracker* t, const float* vmap, size_t pitch) {
+  ModelArgs a;
+  a.src = (const float4*)vmap;
+  a.pitch = pitch;
+  fill_tiles(a.t, t->lv, t->P.levels);
   for (int l = 0; l < t->P.levels; ++l) {
-    const Level& a = t->lv[l];
-    if (l > 0)
-      hipLaunchKernelGGL(k_pyrdown_vmap, grid64x4(a.w, a.h), dim3(256), 0, s, t->ref_v[l - 1],
-                         (size_t)t->lv[l - 1].w * 16, t->ref_v[l], (size_t)a.w * 16, a.w, a.h);
-    hipLaunchKernelGGL(k_icp_point, grid64x4(a.w, a.h), dim3(256), 0, s, t->ref_v[l], t->ref_p[l], a.w, a.h);
+    a.v[l] = t->ref_v[l];
+    a.p[l] = t->ref_p[l];
   }
+  hipLaunchKernelGGL(k_model_levels, dim3(a.t.first[a.t.n]), dim3(256), 0, t->ctx->stream, a);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
@@ -534,52 +438,26 @@ const int* yas_tracker_good_dev(yas_tracker* t) { return &t->st->good; }
 // The state a solve starts from (the pipeline resets it in its first launch).
 TrackState* yas_tracker_state_dev(yas_tracker* t) { return t->st; }
 
-int yas_tracker_set_tracking_image_dev(yas_tracker* t, const float* g, size_t pitch) {
-  return image_pyramid(t, g, pitch, t->cur_int, true);
+// The current frame's image and depth levels from the camera's own images,
+// for the pipeline's first launch.  Levels past the third follow from
+// yas_tracker_coarse_levels.
+int yas_tracker_frame_args(yas_tracker* t, ImageArgs<SrcRgb>& im, DepthArgs<SrcU16>& d) {
+  fill_image(im, t->lv, t->P.levels, 0, t->cur_int, t->gx, t->gy);
+  fill_depth(d, t->lv, t->P.levels, t->cur_inv, t->cur_v, t->cur_p);
+  return YAS_OK;
 }
-int yas_tracker_set_tracking_depth_dev(yas_tracker* t, const float* d, size_t pitch) {
-  return depth_pyramid(t, d, pitch, t->cur_inv, t->cur_v, t->cur_p);
-}
-
-// The pipeline's per-frame tracker inputs: the model from a ray-cast vertex
-// map and the current frame from its intensity and depth, as
-// set_reference_model + set_tracking_image + set_tracking_depth give them.
-int yas_tracker_prepare_frame_dev(yas_tracker* t, const float* vmap, size_t vpitch, const float* g, size_t gpitch,
-                                  const float* d, size_t dpitch) {
-  YAS_REQUIRE(t && vmap && g && d && vpitch >= (size_t)t->W * 16, "yas_tracker_prepare_frame_dev: bad argument");
-  hipStream_t s = t->ctx->stream;
-  FrameLevel a[kMaxLevels];
-  for (int l = 0; l < t->P.levels; ++l) {
-    FrameLevel& f = a[l];
-    const Level& v = t->lv[l];
-    f.l = l;
-    f.w = v.w;
-    f.h = v.h;
-    f.pw = l > 0 ? t->lv[l - 1].w : 0;
-    f.ph = l > 0 ? t->lv[l - 1].h : 0;
-    f.invfx = v.invfx; f.invfy = v.invfy; f.cx = v.cx; f.cy = v.cy;
-    f.gray = g; f.gp = gpitch;
-    f.depth = d; f.dp = dpitch;
-    f.vmap = (const float4*)vmap; f.vp = vpitch;
-    f.int_prev = l > 0 ? t->cur_int[l - 1] : nullptr;
-    f.inv_prev = l > 0 ? t->cur_inv[l - 1] : nullptr;
-    f.refv_prev = l > 0 ? t->ref_v[l - 1] : nullptr;
-    f.cur_int = t->cur_int[l]; f.cur_inv = t->cur_inv[l]; f.cur_v = t->cur_v[l]; f.ref_v = t->ref_v[l];
-    f.gx = t->gx[l]; f.gy = t->gy[l]; f.cur_p = t->cur_p[l]; f.ref_p = t->ref_p[l];
+int yas_tracker_coarse_levels(yas_tracker* t) {
+  for (int base = kImageLevels - 1; base + 1 < t->P.levels; base += kImageLevels - 1) {
+    ImageArgs<SrcF32> a;
+    a.src = SrcF32{t->cur_int[base], (size_t)t->lv[base].w * 4};
+    fill_image(a, t->lv, t->P.levels, base, t->cur_int, t->gx, t->gy);
+    hipLaunchKernelGGL(k_image_levels, dim3(a.tiles), dim3(256), 0, t->ctx->stream, a);
   }
-  // level 0's products; then level l's products beside level l - 1's
-  // neighbourhood products; then the coarsest level's neighbourhood products
-  hipLaunchKernelGGL(k_frame_level, grid64x4(a[0].w, a[0].h), dim3(256), 0, s, a[0]);
-  for (int l = 1; l < t->P.levels; ++l) {
-    const dim3 gp = grid64x4(a[l].w, a[l].h), gn = grid64x4(a[l - 1].w, a[l - 1].h);
-    const int nprod = (int)(gp.x * gp.y);
-    hipLaunchKernelGGL(k_frame_level_pair, dim3(nprod + gn.x * gn.y), dim3(256), 0, s, a[l], a[l - 1], nprod);
-  }
-  hipLaunchKernelGGL(k_frame_level_nb, grid64x4(a[t->P.levels - 1].w, a[t->P.levels - 1].h), dim3(256), 0, s,
-                     a[t->P.levels - 1]);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
+// The model's levels from a ray-cast vertex map, as set_reference_model.
+int yas_tracker_set_model_dev(yas_tracker* t, const float* vmap, size_t pitch) { return model_pyramid(t, vmap, pitch); }
 
 int yas_rgb_to_gray_async(yas_ctx* ctx, const uint8_t* rgb, size_t sp, float* dst, size_t dp, int W, int H, int mode) {
   hipLaunchKernelGGL(k_rgb_to_gray, grid64x4(W, H), dim3(256), 0, ctx->stream, rgb, sp, dst, dp, W, H, mode);
@@ -806,10 +684,7 @@ int yas_tracker_write_debug_images(yas_tracker* t, const char* dir) {
 
 int yas_tracker_set_reference_model(yas_tracker* t, const float* vmap, size_t pitch) {
   YAS_REQUIRE(t && vmap && pitch >= (size_t)t->W * 16, "yas_tracker_set_reference_model: bad argument");
-  hipLaunchKernelGGL(k_copy_f4, grid64x4(t->W, t->H), dim3(256), 0, t->ctx->stream, (const float4*)vmap, pitch,
-                     t->ref_v[0], t->W, t->H);
-  YAS_LAUNCH_CHECK();
-  return model_pyramid(t);
+  return model_pyramid(t, vmap, pitch);
 }
 
 }  // extern "C"

@@ -192,21 +192,17 @@ __device__ inline float ld(const float* p, size_t pitch, int x, int y) {
   return ((const float*)((const char*)p + (size_t)y * pitch))[x];
 }
 
-__device__ inline void copy_f32_at(const float* src, size_t sp, float* dst, int W, int H, int bx, int by) {
-  int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
-  if (x < W && y < H) dst[(size_t)y * W + x] = ld(src, sp, x, y);
-}
-
 // mode 0: 0.299R + 0.587G + 0.114B (float); mode 1: 8-bit fixed point.
+__device__ inline float gray_of(int r, int g, int b, int mode) {
+  return mode == 0 ? 0.299f * (float)r + 0.587f * (float)g + 0.114f * (float)b
+                   : (float)((r * 4899 + g * 9617 + b * 1868 + (1 << 13)) >> 14);
+}
 __device__ inline void rgb_to_gray_at(const uint8_t* rgb, size_t sp, float* dst, size_t dp, int W,
                                                      int H, int mode, int bx, int by) {
   int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
   if (x >= W || y >= H) return;
   const uint8_t* p = rgb + (size_t)y * sp + 3 * x;
-  int r = p[0], g = p[1], b = p[2];
-  float v = mode == 0 ? 0.299f * (float)r + 0.587f * (float)g + 0.114f * (float)b
-                      : (float)((r * 4899 + g * 9617 + b * 1868 + (1 << 13)) >> 14);
-  ((float*)((char*)dst + (size_t)y * dp))[x] = v;
+  ((float*)((char*)dst + (size_t)y * dp))[x] = gray_of(p[0], p[1], p[2], mode);
 }
 
 // OpenCV pyrDown restated: binomial [1 4 6 4 1]/16 per axis (vertical sums of
@@ -216,8 +212,8 @@ __device__ inline int reflect101(int i, int n) {
   if (i >= n) i = 2 * n - 2 - i;
   return i;
 }
-__device__ __attribute__((always_inline)) inline float pyrdown_gauss_px(const float* src, size_t sp, int sw, int sh,
-                                                                       int x, int y) {
+template <class At>
+__device__ __attribute__((always_inline)) inline float pyrdown_gauss_from(At at, int sw, int sh, int x, int y) {
   const float k[5] = {0.0625f, 0.25f, 0.375f, 0.25f, 0.0625f};
   int rows[5];
 #pragma unroll
@@ -226,15 +222,19 @@ __device__ __attribute__((always_inline)) inline float pyrdown_gauss_px(const fl
 #pragma unroll
   for (int j = 0; j < 5; ++j) {
     int sx = reflect101(2 * x + j - 2, sw);
-    float acc = k[0] * ld(src, sp, sx, rows[0]);
+    float acc = k[0] * at(sx, rows[0]);
 #pragma unroll
-    for (int i = 1; i < 5; ++i) acc = acc + k[i] * ld(src, sp, sx, rows[i]);
+    for (int i = 1; i < 5; ++i) acc = acc + k[i] * at(sx, rows[i]);
     col[j] = acc;
   }
   float acc = k[0] * col[0];
 #pragma unroll
   for (int j = 1; j < 5; ++j) acc = acc + k[j] * col[j];
   return acc;
+}
+__device__ __attribute__((always_inline)) inline float pyrdown_gauss_px(const float* src, size_t sp, int sw, int sh,
+                                                                       int x, int y) {
+  return pyrdown_gauss_from([&](int sx, int sy) { return ld(src, sp, sx, sy); }, sw, sh, x, y);
 }
 __device__ __attribute__((always_inline)) inline void pyrdown_gauss_at(const float* src, size_t sp, int sw, int sh,
                                                                        float* dst, size_t dp, int dw, int dh, int bx,
@@ -288,17 +288,6 @@ __device__ inline float4 pyrdown_vmap_px(const float4* s, size_t sp, int W, int 
   if (x < W - 1 && y < H - 1) v = ((const float4*)((const char*)s + (size_t)(2 * y) * sp))[2 * x];
   return v;
 }
-__device__ inline void pyrdown_vmap_at(const float4* s, size_t sp, float4* o, size_t dp, int W, int H, int bx, int by) {
-  int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
-  if (x >= W || y >= H) return;
-  ((float4*)((char*)o + (size_t)y * dp))[x] = pyrdown_vmap_px(s, sp, W, H, x, y);
-}
-
-__device__ inline void copy_f4_at(const float4* s, size_t sp, float4* o, int W, int H, int bx, int by) {
-  int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
-  if (x < W && y < H) o[(size_t)y * W + x] = ((const float4*)((const char*)s + (size_t)y * sp))[x];
-}
-
 // ImageProc.cu:189-209.
 __device__ inline float4 vertex_of(float iz, int x, int y, float invfx, float invfy, float cx, float cy, float cut) {
   float z = 1.0f / iz;
@@ -314,25 +303,27 @@ __device__ inline void vertex_at(const float* inv, size_t sp, float4* v, size_t 
 }
 
 // ImageProc.cu:222-249.
-__device__ inline float4 normal_px(const float4* v, size_t sp, int W, int H, int x, int y) {
+// The normal of vertex a with its neighbours b at (x + 1, y) and c at (x, y + 1).
+__device__ inline float4 normal_of(const float4& a, const float4& b, const float4& c) {
   float4 o = make_float4(0.f, 0.f, 0.f, -1.f);
-  if (x != W - 1 && y != H - 1) {
-    const float4 a = ((const float4*)((const char*)v + (size_t)y * sp))[x];
-    const float4 b = ((const float4*)((const char*)v + (size_t)y * sp))[x + 1];
-    const float4 c = ((const float4*)((const char*)v + (size_t)(y + 1) * sp))[x];
-    if (a.w > 0.f && b.w > 0.f && c.w > 0.f) {
-      float p0 = c.x - a.x, p1 = c.y - a.y, p2 = c.z - a.z;
-      float q0 = b.x - a.x, q1 = b.y - a.y, q2 = b.z - a.z;
-      float r0 = p1 * q2 - p2 * q1, r1 = p2 * q0 - p0 * q2, r2 = p0 * q1 - p1 * q0;
-      float n2 = r0 * r0 + r1 * r1 + r2 * r2;
-      if (n2 > 0.0f) {
-        float nn = sqrtf(n2);
-        r0 = r0 / nn; r1 = r1 / nn; r2 = r2 / nn;
-      }
-      o = make_float4(r0, r1, r2, 1.0f);
+  if (a.w > 0.f && b.w > 0.f && c.w > 0.f) {
+    float p0 = c.x - a.x, p1 = c.y - a.y, p2 = c.z - a.z;
+    float q0 = b.x - a.x, q1 = b.y - a.y, q2 = b.z - a.z;
+    float r0 = p1 * q2 - p2 * q1, r1 = p2 * q0 - p0 * q2, r2 = p0 * q1 - p1 * q0;
+    float n2 = r0 * r0 + r1 * r1 + r2 * r2;
+    if (n2 > 0.0f) {
+      float nn = sqrtf(n2);
+      r0 = r0 / nn; r1 = r1 / nn; r2 = r2 / nn;
     }
+    o = make_float4(r0, r1, r2, 1.0f);
   }
   return o;
+}
+__device__ inline float4 normal_px(const float4* v, size_t sp, int W, int H, int x, int y) {
+  if (x == W - 1 || y == H - 1) return make_float4(0.f, 0.f, 0.f, -1.f);
+  const float4* r0 = (const float4*)((const char*)v + (size_t)y * sp);
+  const float4* r1 = (const float4*)((const char*)v + (size_t)(y + 1) * sp);
+  return normal_of(r0[x], r0[x + 1], r1[x]);
 }
 __device__ inline void normal_at(const float4* v, size_t sp, float4* n, size_t dp, int W, int H, int bx, int by) {
   int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
@@ -363,21 +354,21 @@ __device__ inline void store_icp_point(float4* m, int n, int k, const IcpPoint& 
   m[k] = make_float4(p.vx, p.vy, p.vz, p.nx);
   reinterpret_cast<float2*>(m + n)[k] = make_float2(p.ny, p.nz);
 }
-__device__ inline IcpPoint icp_point_px(const float4* v, size_t sp, int W, int H, int x, int y) {
-  const float4 a = ((const float4*)((const char*)v + (size_t)y * sp))[x];
-  const float4 n = normal_px(v, sp, W, H, x, y);
+// Of vertex a and the neighbours normal_of takes; `nb`: the pixel has them.
+__device__ inline IcpPoint icp_point_of(const float4& a, const float4& b, const float4& c, bool nb) {
+  const float4 n = nb ? normal_of(a, b, c) : make_float4(0.f, 0.f, 0.f, -1.f);
   IcpPoint p;
   p.vx = n.w > 0.0f ? a.x : __builtin_nanf("");
   p.vy = a.y; p.vz = a.z;
   p.nx = n.x; p.ny = n.y; p.nz = n.z;
   return p;
 }
-__device__ inline void icp_point_at(const float4* v, size_t sp, float4* o, int W, int H, int bx, int by) {
-  int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);
-  if (x >= W || y >= H) return;
-  store_icp_point(o, W * H, y * W + x, icp_point_px(v, sp, W, H, x, y));
+__device__ inline IcpPoint icp_point_px(const float4* v, size_t sp, int W, int H, int x, int y) {
+  const float4* r0 = (const float4*)((const char*)v + (size_t)y * sp);
+  const bool nb = x != W - 1 && y != H - 1;
+  const float4 a = r0[x];
+  return nb ? icp_point_of(a, r0[x + 1], ((const float4*)((const char*)r0 + sp))[x], true) : icp_point_of(a, a, a, false);
 }
-
 // ImageProc.cu:262-275.
 __device__ inline void vmap_to_depth_at(const float4* v, size_t sp, float* d, size_t dp, int W, int H, int bx, int by) {
   int x = bx * 64 + (threadIdx.x & 63), y = by * 4 + (threadIdx.x >> 6);

@@ -82,13 +82,9 @@ __global__ void __launch_bounds__(256) k_balloc(const BatchItem* items, const Po
   constexpr int TH = 256 / TW;
   const int t = b - ws[lo];
   const int tiles_x = (it.W + TW - 1) / TW;
-  __shared__ int walked;
-  if (threadIdx.x == 0) walked = 0;
-  __syncthreads();
-  alloc_walk(it.m, DepthU16{it.depth, it.pitch, it.depth_scale}, it.W, it.H, it.K, pp[lo].T,
-             (t % tiles_x) * TW + (int)(threadIdx.x % TW), (t / tiles_x) * TH + (int)(threadIdx.x / TW), &walked);
-  __syncthreads();
-  if (threadIdx.x == 0 && walked) atomicAdd(&it.m.ctr[kCtrWalk], walked);
+  __shared__ AllocLds lds;
+  alloc_group(it.m, DepthU16{it.depth, it.pitch, it.depth_scale}, it.W, it.H, it.K, pp[lo].T,
+              (t % tiles_x) * TW + (int)(threadIdx.x % TW), (t / tiles_x) * TH + (int)(threadIdx.x / TW), &lds);
 }
 
 __global__ void __launch_bounds__(256) k_bvisible(const BatchItem* items, const PosePair* pp, const int* cur, int n) {

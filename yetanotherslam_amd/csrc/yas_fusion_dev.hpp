@@ -21,9 +21,18 @@ struct DepthF32 {
     return *(const float*)((const char*)p + ((unsigned)y * (unsigned)pitch + (unsigned)x * 4u));
   }
 };
-inline bool depth_span_fits(size_t pitch, int W, int H) {
-  return pitch < (1ull << 32) && (unsigned long long)(H - 1) * pitch + (unsigned long long)W * 4u <= 0xFFFFFFFFull;
+inline bool depth_span_fits(size_t pitch, int W, int H, unsigned bytes = 4u) {
+  return pitch < (1ull << 32) && (unsigned long long)(H - 1) * pitch + (unsigned long long)W * bytes <= 0xFFFFFFFFull;
 }
+// The same for raw uint16 depth (spans below 4 GiB).
+struct DepthU16Near {
+  const uint16_t* p;
+  size_t pitch;
+  float scale;
+  __device__ inline float at(int x, int y) const {
+    return (float)*(const uint16_t*)((const char*)p + ((unsigned)y * (unsigned)pitch + (unsigned)x * 2u)) * scale;
+  }
+};
 struct DepthU16 {
   const uint16_t* p;
   size_t pitch;
@@ -48,11 +57,11 @@ __device__ inline void pixel_block(int x, int y, float z, const Intr& K, const P
 // K3 (VoxelMap.cu:517-652) for pixel (x, y): every block on the integer 3D
 // Bresenham walk between the blocks of depth-mu/2 and depth+mu/2 along the
 // pixel ray.  All lanes of the wavefront must call it (the insertion is a
-// wavefront operation); lanes outside the image pass no blocks.  The walk
-// length is added to *walked (LDS).
+// wavefront operation); lanes outside the image pass no blocks.  New blocks
+// go to `list` (wave_insert).  The walk length is added to *walked (LDS).
 template <class D>
 __device__ inline void alloc_walk(const MapView& m, const D& depth, int W, int H, const Intr& K, const PoseF& T, int x,
-                                  int y, int* walked) {
+                                  int y, int* walked, InsertList* list) {
   const float vs = m.voxel_size;
   int px = 0, py = 0, pz = 0;          // current block
   int dax = 0, day = 0, daz = 0;       // unit step along the dominant axis
@@ -101,7 +110,7 @@ __device__ inline void alloc_walk(const MapView& m, const D& depth, int W, int H
     uint64_t key = ok ? pack_key(px, py, pz) : 0ull;
     int home = ok ? ref_hash(px, py, pz, m.num_buckets) : 0;
     if (lane_id() == __ffsll(act) - 1) atomicAdd(walked, __popcll(act));
-    wave_insert(m, key, ok, home);
+    wave_insert(m, key, ok, home, list);
     if (has) {
       --remaining;
       if (remaining > 0) {
@@ -113,6 +122,31 @@ __device__ inline void alloc_walk(const MapView& m, const D& depth, int W, int H
       }
     }
   }
+}
+
+// A workgroup's part of the allocation: alloc_walk of its pixels, its new
+// blocks' pool indices, and its walk steps added to the map's counter (one
+// atomic each for the workgroup).
+struct AllocLds {
+  int walked;
+  InsertList list;
+};
+template <class D>
+__device__ inline void alloc_group(const MapView& m, const D& depth, int W, int H, const Intr& K, const PoseF& T, int x,
+                                   int y, AllocLds* lds) {
+  if (threadIdx.x == 0) lds->walked = 0;
+  start_inserts(&lds->list);
+  alloc_walk(m, depth, W, H, K, T, x, y, &lds->walked, &lds->list);
+  finish_inserts(m, &lds->list);
+  if (threadIdx.x == 0 && lds->walked) atomicAdd(&m.ctr[kCtrWalk], lds->walked);
+}
+// The pixel of this thread in a 32x32 tile of 1024 threads, 8x8 a wavefront:
+// a wavefront's rays share blocks most when its patch is square.
+constexpr int kAllocThreads = 1024;
+__device__ inline void alloc_pixel(int bx, int by, int& x, int& y) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  x = bx * 32 + (wave & 3) * 8 + (lane & 7);
+  y = by * 32 + (wave >> 2) * 8 + (lane >> 3);
 }
 
 // VoxelStructUtils.h:112-147.

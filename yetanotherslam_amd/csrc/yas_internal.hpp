@@ -423,9 +423,37 @@ __device__ inline float wave_sum(float v) {
   return v;
 }
 
+// New blocks of a workgroup, gathered in LDS: they take their pool indices
+// together, with one atomic on the map's counter for the whole workgroup
+// (finish_inserts).  That counter is one address for all XCDs, and atomics on
+// it follow one another at 20-30 ns each: with one per wavefront and walk
+// step they were most of a first frame's allocation.
+constexpr int kInsertList = 512;
+struct InsertList {
+  int n;     // blocks won by the workgroup (entries past kInsertList are not kept here)
+  int base;  // their first pool index
+  unsigned long long key[kInsertList];
+  int slot[kInsertList];
+};
+
+// Block `key`, whose table slot this caller claimed, becomes pool block idx.
+__device__ inline void take_pool_index(const MapView& m, unsigned long long key, int slot, int idx) {
+  if (idx < m.num_blocks) {
+    m.block_keys[idx] = key;
+    m.block_slot[idx] = slot;
+    m.slots[slot].flags = kBlockUnobserved;
+    m.slots[slot].val = idx;
+  } else {
+    m.slots[slot].val = -1;
+    atomicOr(&m.ctr[kCtrFlags], kFlagPoolOverflow);
+  }
+}
+
 // Insert the keys held by the lanes with `has`, one CAS per distinct key of
-// the wavefront; new blocks get consecutive pool indices from one atomic.
-__device__ inline void wave_insert(const MapView& m, uint64_t key, bool has, int home) {
+// the wavefront.  New blocks go to `list` (LDS), which the workgroup empties
+// with finish_inserts; those that find it full take consecutive pool indices
+// from an atomic of their wavefront.
+__device__ inline void wave_insert(const MapView& m, uint64_t key, bool has, int home, InsertList* list) {
   bool pending = has;
   bool leader = false;
   for (;;) {
@@ -456,25 +484,37 @@ __device__ inline void wave_insert(const MapView& m, uint64_t key, bool has, int
     }
     if (p == lim) atomicOr(&m.ctr[kCtrFlags], kFlagProbeLimit);
   }
+  if (won) {
+    const int at = atomicAdd(&list->n, 1);
+    if (at < kInsertList) {
+      list->key[at] = key;
+      list->slot[at] = slot;
+      won = false;
+    }
+  }
   unsigned long long wm = __ballot(won);
   if (wm) {
     int first = __ffsll(wm) - 1;
     int base = 0;
     if (lane_id() == first) base = atomicAdd(&m.ctr[kCtrAlloc], __popcll(wm));
     base = __shfl(base, first);
-    if (won) {
-      int idx = base + __popcll(wm & lane_mask_lt());
-      if (idx < m.num_blocks) {
-        m.block_keys[idx] = key;
-        m.block_slot[idx] = slot;
-        m.slots[slot].flags = kBlockUnobserved;
-        m.slots[slot].val = idx;
-      } else {
-        m.slots[slot].val = -1;
-        atomicOr(&m.ctr[kCtrFlags], kFlagPoolOverflow);
-      }
-    }
+    if (won) take_pool_index(m, key, slot, base + __popcll(wm & lane_mask_lt()));
   }
+}
+
+// Before the first wave_insert and after the last one of a workgroup, by all
+// of its threads.
+__device__ inline void start_inserts(InsertList* list) {
+  if (threadIdx.x == 0) list->n = 0;
+  __syncthreads();
+}
+__device__ inline void finish_inserts(const MapView& m, InsertList* list) {
+  __syncthreads();
+  const int n = min(list->n, kInsertList);
+  if (n == 0) return;
+  if (threadIdx.x == 0) list->base = atomicAdd(&m.ctr[kCtrAlloc], n);
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += blockDim.x) take_pool_index(m, list->key[i], list->slot[i], list->base + i);
 }
 
 }  // namespace yas

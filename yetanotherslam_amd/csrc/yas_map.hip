@@ -135,22 +135,34 @@ __global__ void __launch_bounds__(256) k_zero_u32(uint32_t* p, size_t n) {
     p[i] = 0u;
 }
 
+// Clears what a map holds: the slots and voxels of its allocated blocks (the
+// rest of the pool has never been written, or was cleared when it last was).
+// Where more blocks were claimed than the pool has, their slots are in no
+// list: then the whole table is cleared.  The counters are cleared by the
+// next launch, since every workgroup reads them here.
+__global__ void __launch_bounds__(256) k_reset_used(MapView m, int words16 /* 16-byte words of a block's voxels */) {
+  const int na = m.ctr[kCtrAlloc];
+  const int n = na < m.num_blocks ? na : m.num_blocks;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+  HashSlot e;
+  e.key = kEmptyKey;
+  e.val = -1;
+  e.flags = 0;
+  if (na > m.num_blocks) {
+    for (int i = t; i < m.num_buckets; i += nt) m.slots[i] = e;
+  } else {
+    for (int i = t; i < n; i += nt) m.slots[m.block_slot[i]] = e;
+  }
+  uint4* v = (uint4*)m.voxels;
+  for (size_t i = t; i < (size_t)n * words16; i += nt) v[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // Writes the float pose pair of a by-value double pose and clears the
 // visible-block counter for the call that follows.
 __global__ void k_pose_prep(Mat44 T, PosePair* out, int* ctr) {
   if (threadIdx.x == 0) {
     PosePair p;
     pose_pair_from(T.m, p);
-    *out = p;
-    if (ctr) ctr[kCtrVisible] = 0;
-  }
-}
-
-// Same from a device-resident double pose (used by the pipeline).
-__global__ void k_pose_prep_dev(const double* T, PosePair* out, int* ctr) {
-  if (threadIdx.x == 0) {
-    PosePair p;
-    pose_pair_from(T, p);
     *out = p;
     if (ctr) ctr[kCtrVisible] = 0;
   }
@@ -165,39 +177,60 @@ __global__ void __launch_bounds__(256) k_depth_u16(const uint16_t* src, size_t s
   ((float*)((char*)dst + y * dp))[x] = (float)d * scale;
 }
 
-// K3 (VoxelMap.cu:517-652), 16x16 pixels per workgroup: a wavefront covers
-// a 16x4 patch whose rays mostly share blocks.
-__global__ void __launch_bounds__(256) k_alloc(MapView m, const float* depth, size_t pitch, int W, int H, Intr K,
-                                               const PosePair* pose, const int* gate) {
+// The pose pair of a call: prepared in device memory (the pipeline's), or by
+// value, formed on the host.  Types of their own, so that either is read by
+// scalar loads (a choice at run time puts it in 12 vector registers).
+struct PoseDev {
+  const PosePair* p;  // written by an earlier launch
+  __device__ static inline PoseF read(const YAS_CONSTANT PoseF& q) {
+    PoseF o;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) o.r[i] = q.r[i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o.t[i] = q.t[i];
+    return o;
+  }
+  __device__ inline PoseF T() const { return read(((const YAS_CONSTANT PosePair*)p)->T); }
+  __device__ inline PoseF Tinv() const { return read(((const YAS_CONSTANT PosePair*)p)->Tinv); }
+};
+struct PoseVal {
+  PosePair p;
+  __device__ inline PoseF T() const { return p.T; }
+  __device__ inline PoseF Tinv() const { return p.Tinv; }
+};
+
+// K3 (VoxelMap.cu:517-652), 32x32 pixels per workgroup.  `clear`: the map's
+// visible counter is cleared for the visibility pass that follows.
+template <class D, class P>
+__global__ void __launch_bounds__(kAllocThreads) k_alloc(MapView m, D depth, int W, int H, Intr K, P pose,
+                                                         const int* gate, int clear) {
   if (gate && *gate == 0) return;
-  __shared__ int walked;
-  if (threadIdx.x == 0) walked = 0;
-  __syncthreads();
-  alloc_walk(m, DepthF32{depth, pitch}, W, H, K, pose->T, blockIdx.x * 16 + (threadIdx.x & 15),
-             blockIdx.y * 16 + (threadIdx.x >> 4), &walked);
-  __syncthreads();
-  if (threadIdx.x == 0 && walked) atomicAdd(&m.ctr[kCtrWalk], walked);
+  __shared__ AllocLds lds;
+  if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) m.ctr[kCtrVisible] = 0;
+  int x, y;
+  alloc_pixel(blockIdx.x, blockIdx.y, x, y);
+  alloc_group(m, depth, W, H, K, pose.T(), x, y, &lds);
 }
 
 // K4 (VoxelMap.cu:654-717).
-__global__ void __launch_bounds__(256) k_visible(MapView m, const PosePair* pose, Intr K, int W, int H,
-                                                 const int* gate) {
+template <class P>
+__global__ void __launch_bounds__(256) k_visible(MapView m, P pose, Intr K, int W, int H, const int* gate) {
   if (gate && *gate == 0) return;
-  visible_scan(m, pose->Tinv, K, W, H, blockIdx.x * blockDim.x, gridDim.x * blockDim.x);
+  visible_scan(m, pose.Tinv(), K, W, H, blockIdx.x * blockDim.x, gridDim.x * blockDim.x);
 }
 
 // K5 (VoxelMap.cu:719-786).  `stats` (optional) receives the map's first
 // four counters (allocated, visible, flags, walk steps), final once
 // allocation and visibility have run.
-template <class VT>
+template <class VT, class D, class P>
 // At least six wavefronts per SIMD.  With the block index made
 // wavefront-uniform and 32-bit depth offsets every storage's kernel fits
 // in 64 registers (eight wavefronts, no spills); asking for eight with
 // 64-bit depth addresses spilled the float storage's kernel and slowed it.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
-k_integrate(MapView m, const PosePair* pose, Intr K, const float* depth, size_t pitch, int W, int H, int* stats) {
+k_integrate(MapView m, P pose, Intr K, D depth, int W, int H, int* stats) {
   if (stats && blockIdx.x == 0 && threadIdx.x < 4) stats[threadIdx.x] = m.ctr[threadIdx.x];
-  integrate_waves<VT>(m, pose->Tinv, K, DepthF32{depth, pitch}, W, H, integrate_wave(m, blockIdx.x, gridDim.x),
+  integrate_waves<VT>(m, pose.Tinv(), K, depth, W, H, integrate_wave(m, blockIdx.x, gridDim.x),
                       gridDim.x * (blockDim.x >> 6));
 }
 
@@ -210,62 +243,75 @@ static int grid_for(long n, int per, int cap) {
   return (int)g;
 }
 
-static int launch_integrate(yas_map* map, const float* depth, size_t pitch, int W, int H,
+static PoseDev pose_on_device(yas_map* map) { return PoseDev{map->pose_dev}; }
+static PoseVal pose_of(const double T[16]) {
+  PoseVal p;
+  pose_pair_from(T, p.p);
+  return p;
+}
+
+template <class D, class P>
+static int launch_alloc(yas_map* map, const D& depth, int W, int H, const P& pose, const int* gate, int clear,
+                        const hipEvent_t* ev = nullptr) {
+  launch_timed(k_alloc<D, P>, dim3((W + 31) / 32, (H + 31) / 32), dim3(kAllocThreads), map->ctx->stream, ev, map->v, depth,
+               W, H, map->K, pose, gate, clear);
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+template <class P>
+static int launch_visible(yas_map* map, int W, int H, const P& pose, const int* gate,
+                          const hipEvent_t* ev = nullptr) {
+  launch_timed(k_visible<P>, dim3(grid_for(map->P.num_blocks, 256, 4096)), dim3(256), map->ctx->stream, ev, map->v, pose,
+               map->K, W, H, gate);
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+template <class D, class P>
+static int launch_integrate(yas_map* map, const D& depth, int W, int H, const P& pose,
                             const hipEvent_t* ev = nullptr, int* stats = nullptr) {
   hipStream_t s = map->ctx->stream;
   // enough wavefronts for one visible block each up to 32768 visible blocks
   // (those past the visible count return at once)
   dim3 grid(grid_for(map->P.num_blocks, 4, 8192));
-  const PosePair* pose = map->pose_dev;
   switch (map->P.voxel_format) {
     case YAS_VOXEL_I16_U8:
-      launch_timed(k_integrate<VoxI16>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, pitch, W, H, stats);
+      launch_timed(k_integrate<VoxI16, D, P>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, W, H, stats);
       break;
     case YAS_VOXEL_F16_U16:
-      launch_timed(k_integrate<VoxF16>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, pitch, W, H, stats);
+      launch_timed(k_integrate<VoxF16, D, P>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, W, H, stats);
       break;
     default:
-      launch_timed(k_integrate<VoxF32>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, pitch, W, H, stats);
+      launch_timed(k_integrate<VoxF32, D, P>, grid, dim3(256), s, ev, map->v, pose, map->K, depth, W, H, stats);
   }
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
-// Allocation + visibility + integration with the pose already in pose_dev.
-// The three fusion stages with the pose already in pose_dev.  A non-null
-// `gate` pointing at 0 turns allocation and visibility into no-ops on the
-// device (integration then sees no visible blocks).
+// The three fusion stages with the pose already in pose_dev and the visible
+// counter cleared (pipeline).  A non-null `gate` pointing at 0 turns
+// allocation and visibility into no-ops on the device (integration then sees
+// no visible blocks).
 int yas_map_alloc_stage(yas_map* map, const float* depth, size_t pitch, int W, int H, const int* gate,
                         const hipEvent_t* ev = nullptr) {
   YAS_REQUIRE(depth_span_fits(pitch, W, H), "depth image spans 4 GiB or more");
-  dim3 g((W + 15) / 16, (H + 15) / 16);
-  launch_timed(k_alloc, g, dim3(256), map->ctx->stream, ev, map->v, depth, pitch, W, H, map->K,
-               (const PosePair*)map->pose_dev, gate);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
+  return launch_alloc(map, DepthF32{depth, pitch}, W, H, pose_on_device(map), gate, 0, ev);
 }
 int yas_map_visible_stage(yas_map* map, int W, int H, const int* gate, const hipEvent_t* ev = nullptr) {
-  launch_timed(k_visible, dim3(grid_for(map->P.num_blocks, 256, 4096)), dim3(256), map->ctx->stream, ev, map->v,
-               (const PosePair*)map->pose_dev, map->K, W, H, gate);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
+  return launch_visible(map, W, H, pose_on_device(map), gate, ev);
 }
 int yas_map_integrate_stage(yas_map* map, const float* depth, size_t pitch, int W, int H,
                             const hipEvent_t* ev = nullptr, int* stats = nullptr) {
   YAS_REQUIRE(depth_span_fits(pitch, W, H), "depth image spans 4 GiB or more");
-  return launch_integrate(map, depth, pitch, W, H, ev, stats);
+  return launch_integrate(map, DepthF32{depth, pitch}, W, H, pose_on_device(map), ev, stats);
 }
-int yas_map_fuse_prepared(yas_map* map, const float* depth, size_t pitch, int W, int H, const int* gate) {
-  int rc = yas_map_alloc_stage(map, depth, pitch, W, H, gate);
-  if (!rc) rc = yas_map_visible_stage(map, W, H, gate);
-  if (!rc) rc = yas_map_integrate_stage(map, depth, pitch, W, H);
+// All three at pose T.
+template <class D>
+static int fuse_at(yas_map* map, const D& depth, int W, int H, const double T[16]) {
+  const PoseVal pose = pose_of(T);
+  int rc = launch_alloc(map, depth, W, H, pose, nullptr, 1);
+  if (!rc) rc = launch_visible(map, W, H, pose, nullptr);
+  if (!rc) rc = launch_integrate(map, depth, W, H, pose);
   return rc;
-}
-
-int yas_map_prepare_pose_dev(yas_map* map, const double* T_dev) {
-  hipLaunchKernelGGL(k_pose_prep_dev, dim3(1), dim3(64), 0, map->ctx->stream, T_dev, map->pose_dev, map->v.ctr);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
 }
 
 static int prepare_pose(yas_map* map, const double T[16], bool reset_visible) {
@@ -286,33 +332,32 @@ yas_ctx* yas_map_ctx(yas_map* map) { return map->ctx; }
 // Visibility only (used by the ray caster): clears and refills the visible list.
 int yas_map_visible_async(yas_map* map, const double T[16], int W, int H) {
   int rc = prepare_pose(map, T, true);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_visible, dim3(grid_for(map->P.num_blocks, 256, 4096)), dim3(256), 0, map->ctx->stream,
-                     map->v, (const PosePair*)map->pose_dev, map->K, W, H, (const int*)nullptr);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
+  return rc ? rc : launch_visible(map, W, H, pose_on_device(map), nullptr);
 }
 // Visibility with the pose pair already in pose_dev and the visible counter
 // already cleared.
 int yas_map_visible_prepared(yas_map* map, int W, int H) {
-  hipLaunchKernelGGL(k_visible, dim3(grid_for(map->P.num_blocks, 256, 4096)), dim3(256), 0, map->ctx->stream,
-                     map->v, (const PosePair*)map->pose_dev, map->K, W, H, (const int*)nullptr);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
-}
-int yas_map_visible_async_dev(yas_map* map, const double* T_dev, int W, int H) {
-  int rc = yas_map_prepare_pose_dev(map, T_dev);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_visible, dim3(grid_for(map->P.num_blocks, 256, 4096)), dim3(256), 0, map->ctx->stream,
-                     map->v, (const PosePair*)map->pose_dev, map->K, W, H, (const int*)nullptr);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
+  return launch_visible(map, W, H, pose_on_device(map), nullptr);
 }
 
 int yas_convert_depth_u16(yas_ctx* ctx, const uint16_t* src, size_t sp, float* dst, size_t dp, int W, int H,
                           float depth_scale) {
   float s = (float)(1.0 / (double)depth_scale);
   hipLaunchKernelGGL(k_depth_u16, dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, ctx->stream, src, sp, dst, dp, W, H, s);
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+
+// New arrays: every slot, voxel and counter.
+static int clear_all(yas_map* m) {
+  hipStream_t s = m->ctx->stream;
+  hipLaunchKernelGGL(k_reset_hash, dim3(grid_for(m->P.num_buckets, 256, 8192)), dim3(256), 0, s, m->v.slots,
+                     m->P.num_buckets);
+  YAS_LAUNCH_CHECK();
+  size_t words = (size_t)voxel_bytes(m->P.voxel_format) * 512 * (size_t)m->P.num_blocks / 4;
+  hipLaunchKernelGGL(k_zero_u32, dim3(grid_for((long)(words / 4), 256, 16384)), dim3(256), 0, s, (uint32_t*)m->v.voxels,
+                     words);
+  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, (uint32_t*)m->v.ctr, (size_t)kCtrCount);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
@@ -360,7 +405,7 @@ int yas_map_create(yas_ctx* ctx, const yas_map_params* P, const float K[4], yas_
     yas_map_destroy(m);
     return YAS_E_HIP;
   }
-  int rc = yas_map_reset(m);
+  int rc = clear_all(m);
   if (rc) {
     yas_map_destroy(m);
     return rc;
@@ -373,12 +418,8 @@ int yas_map_reset(yas_map* m) {
   YAS_REQUIRE(m, "null map");
   YAS_REQUIRE_ACTIVE(m);
   hipStream_t s = m->ctx->stream;
-  hipLaunchKernelGGL(k_reset_hash, dim3(grid_for(m->P.num_buckets, 256, 8192)), dim3(256), 0, s, m->v.slots,
-                     m->P.num_buckets);
-  YAS_LAUNCH_CHECK();
-  size_t words = (size_t)voxel_bytes(m->P.voxel_format) * 512 * (size_t)m->P.num_blocks / 4;
-  hipLaunchKernelGGL(k_zero_u32, dim3(grid_for((long)(words / 4), 256, 16384)), dim3(256), 0, s, (uint32_t*)m->v.voxels,
-                     words);
+  hipLaunchKernelGGL(k_reset_used, dim3(grid_for(m->P.num_blocks, 1, 4096)), dim3(256), 0, s, m->v,
+                     voxel_bytes(m->P.voxel_format) * 512 / 16);
   hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, (uint32_t*)m->v.ctr, (size_t)kCtrCount);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
@@ -424,9 +465,8 @@ int yas_map_fuse(yas_map* m, const float* depth, size_t pitch, int W, int H, con
   YAS_REQUIRE_ACTIVE(m);
   YAS_REQUIRE(W > 0 && H > 0 && pitch >= (size_t)W * sizeof(float), "yas_map_fuse: bad image size");
   YAS_HIP(hipSetDevice(m->ctx->device));
-  int rc = prepare_pose(m, T, true);
-  if (rc) return rc;
-  return yas_map_fuse_prepared(m, depth, pitch, W, H, nullptr);
+  YAS_REQUIRE(depth_span_fits(pitch, W, H), "depth image spans 4 GiB or more");
+  return fuse_at(m, DepthF32{depth, pitch}, W, H, T);
 }
 
 int yas_map_fuse_u16(yas_map* m, const uint16_t* depth, size_t pitch, int W, int H, float depth_scale,
@@ -436,6 +476,9 @@ int yas_map_fuse_u16(yas_map* m, const uint16_t* depth, size_t pitch, int W, int
   YAS_REQUIRE(W > 0 && H > 0 && pitch >= (size_t)W * sizeof(uint16_t), "yas_map_fuse_u16: bad image size");
   YAS_REQUIRE(depth_scale > 0.f, "yas_map_fuse_u16: depth_scale must be > 0");
   YAS_HIP(hipSetDevice(m->ctx->device));
+  // the kernels convert what they read, as (float)raw * (float)(1 / scale)
+  if (depth_span_fits(pitch, W, H, 2u))
+    return fuse_at(m, DepthU16Near{depth, pitch, (float)(1.0 / (double)depth_scale)}, W, H, T);
   size_t need = (size_t)W * H * sizeof(float);
   if (m->depth_f32_bytes < need) {
     YAS_HIP(hipStreamSynchronize(m->ctx->stream));

@@ -80,6 +80,8 @@ __global__ void __launch_bounds__(256) k_merge_alloc(MapView dst, MapView src, P
   const int nwaves = gridDim.x * (blockDim.x >> 6);
   const typename VT::T* sv = (const typename VT::T*)src.voxels;
   const float vs = dst.voxel_size;
+  __shared__ InsertList list;
+  start_inserts(&list);
   for (int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); w < nsrc; w += nwaves) {
     int bx, by, bz;
     unpack_key(src.block_keys[w], bx, by, bz);
@@ -104,9 +106,10 @@ __global__ void __launch_bounds__(256) k_merge_alloc(MapView dst, MapView src, P
           atomicOr(&dst.ctr[kCtrFlags], kFlagKeyRange);
         }
       }
-      wave_insert(dst, key, has, home);
+      wave_insert(dst, key, has, home, &list);
     }
   }
+  finish_inserts(dst, &list);
 }
 
 // Voxel reads of the source map with a one-entry block cache; ReadSDF

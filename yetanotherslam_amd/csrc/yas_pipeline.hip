@@ -15,7 +15,6 @@
 
 using namespace yas;
 
-int yas_map_fuse_prepared(yas_map* map, const float* depth, size_t pitch, int W, int H, const int* gate);
 int yas_map_alloc_stage(yas_map* map, const float* depth, size_t pitch, int W, int H, const int* gate,
                         const hipEvent_t* ev);
 int yas_map_visible_stage(yas_map* map, int W, int H, const int* gate, const hipEvent_t* ev);

@@ -15,7 +15,6 @@ MapView yas_map_view(yas_map* map);
 const PosePair* yas_map_pose_dev(yas_map* map);
 yas_ctx* yas_map_ctx(yas_map* map);
 int yas_map_visible_async(yas_map* map, const double T[16], int W, int H);
-int yas_map_visible_async_dev(yas_map* map, const double* T_dev, int W, int H);
 int yas_map_visible_prepared(yas_map* map, int W, int H);
 
 struct yas_raycaster {
@@ -136,15 +135,6 @@ static int scratch_on_device(int device, unsigned** out) {
   }
   *out = g_scratch_dev[device];
   return YAS_OK;
-}
-
-// Ray cast with the pose held in device memory (pipeline).
-// `before_march` (optional) is recorded between the z-range and march kernels.
-int yas_raycast_dev(yas_raycaster* rc, yas_map* map, const double* T_dev, hipEvent_t before_march,
-                    const hipEvent_t* march_ev) {
-  int r = yas_map_visible_async_dev(map, T_dev, rc->W, rc->H);
-  if (r) return r;
-  return launch_raycast(rc, map, before_march, march_ev);
 }
 
 // Ray cast whose set-up the caller has already enqueued on this stream: the

@@ -315,17 +315,14 @@ __global__ void k_s_post(const StreamDev* streams, const Table* tab) {
   sl.out[16] = (double)tracked;
 }
 
-__global__ void __launch_bounds__(256) k_s_alloc(const StreamDev* streams, const Table* tab) {
+__global__ void __launch_bounds__(kAllocThreads) k_s_alloc(const StreamDev* streams, const Table* tab) {
   SLOT_OR_RETURN;
   if (!sl.first && *S.gate == 0) return;
-  if ((int)blockIdx.x * 16 >= S.W || (int)blockIdx.y * 16 >= S.H) return;
-  __shared__ int walked;
-  if (threadIdx.x == 0) walked = 0;
-  __syncthreads();
-  alloc_walk(S.m, DepthF32{S.depth, (size_t)S.W * 4}, S.W, S.H, S.K, S.pose->T, blockIdx.x * 16 + (threadIdx.x & 15),
-             blockIdx.y * 16 + (threadIdx.x >> 4), &walked);
-  __syncthreads();
-  if (threadIdx.x == 0 && walked) atomicAdd(&S.m.ctr[kCtrWalk], walked);
+  if ((int)blockIdx.x * 32 >= S.W || (int)blockIdx.y * 32 >= S.H) return;
+  __shared__ AllocLds lds;
+  int x, y;
+  alloc_pixel(blockIdx.x, blockIdx.y, x, y);
+  alloc_group(S.m, DepthF32{S.depth, (size_t)S.W * 4}, S.W, S.H, S.K, S.pose->T, x, y, &lds);
 }
 
 // At least six wavefronts per SIMD, as k_integrate.
@@ -501,7 +498,7 @@ static int launch_batch_kernels(yas_server* sv, hipStream_t s, int nz) {
   for (int l = 0; l < L; ++l) hipLaunchKernelGGL(k_s_keep, level_grid(l), dim3(256), 0, s, S, T, l);
   // fusion at the new pose
   hipLaunchKernelGGL(k_s_pose, dim3(1, 1, nz), dim3(64), 0, s, S, T, 0);
-  hipLaunchKernelGGL(k_s_alloc, dim3((W + 15) / 16, (H + 15) / 16, nz), dim3(256), 0, s, S, T);
+  hipLaunchKernelGGL(k_s_alloc, dim3((W + 31) / 32, (H + 31) / 32, nz), dim3(kAllocThreads), 0, s, S, T);
   hipLaunchKernelGGL(k_s_visible, dim3(4096, 1, nz), dim3(256), 0, s, S, T, 1);
   switch (sv->voxel_format) {
     case YAS_VOXEL_I16_U8: hipLaunchKernelGGL(k_s_integrate<VoxI16>, dim3(2048, 1, nz), dim3(256), 0, s, S, T); break;

@@ -209,6 +209,28 @@ __host__ __device__ inline void inv44(const double* T, double* o) {
   for (int i = 0; i < 16; ++i) o[i] = t[i];
 }
 
+// The pose pair of a call: prepared in device memory (the pipeline's), or by
+// value, formed on the host.  Types of their own, so that either is read by
+// scalar loads (a choice at run time puts it in 12 vector registers).
+struct PoseDev {
+  const PosePair* p;  // written by an earlier launch
+  __device__ static inline PoseF read(const YAS_CONSTANT PoseF& q) {
+    PoseF o;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) o.r[i] = q.r[i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o.t[i] = q.t[i];
+    return o;
+  }
+  __device__ inline PoseF T() const { return read(((const YAS_CONSTANT PosePair*)p)->T); }
+  __device__ inline PoseF Tinv() const { return read(((const YAS_CONSTANT PosePair*)p)->Tinv); }
+};
+struct PoseVal {
+  PosePair p;
+  __device__ inline PoseF T() const { return p.T; }
+  __device__ inline PoseF Tinv() const { return p.Tinv; }
+};
+
 struct Intr {
   float fx, fy, cx, cy, invfx, invfy;
 };

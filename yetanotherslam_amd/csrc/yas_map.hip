@@ -177,28 +177,6 @@ __global__ void __launch_bounds__(256) k_depth_u16(const uint16_t* src, size_t s
   ((float*)((char*)dst + y * dp))[x] = (float)d * scale;
 }
 
-// The pose pair of a call: prepared in device memory (the pipeline's), or by
-// value, formed on the host.  Types of their own, so that either is read by
-// scalar loads (a choice at run time puts it in 12 vector registers).
-struct PoseDev {
-  const PosePair* p;  // written by an earlier launch
-  __device__ static inline PoseF read(const YAS_CONSTANT PoseF& q) {
-    PoseF o;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) o.r[i] = q.r[i];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) o.t[i] = q.t[i];
-    return o;
-  }
-  __device__ inline PoseF T() const { return read(((const YAS_CONSTANT PosePair*)p)->T); }
-  __device__ inline PoseF Tinv() const { return read(((const YAS_CONSTANT PosePair*)p)->Tinv); }
-};
-struct PoseVal {
-  PosePair p;
-  __device__ inline PoseF T() const { return p.T; }
-  __device__ inline PoseF Tinv() const { return p.Tinv; }
-};
-
 // K3 (VoxelMap.cu:517-652), 32x32 pixels per workgroup.  `clear`: the map's
 // visible counter is cleared for the visibility pass that follows.
 template <class D, class P>

@@ -29,50 +29,62 @@ struct yas_raycaster {
   float* depth;  // VMapToDepth of the last vertex map (lazily allocated)
 };
 
-__global__ void __launch_bounds__(256) k_zrange_init(unsigned* zmin, unsigned* zmax, int n) {
+// The cells before a ray cast, and the map's visible counter.
+__global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zmax, int n, int* ctr) {
   zrange_init_at(zmin, zmax, n, blockIdx.x, gridDim.x);
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctr[kCtrVisible] = 0;
 }
 
+// Visibility and z-range cells (view_scan).  Workgroup b: slice b / chunks of
+// the block list, chunk b % chunks of the cell rows (rows_per each).
+template <class P>
+__global__ void __launch_bounds__(256) k_view(MapView m, P pose, Intr K, int W, int H, int cols, int rows,
+                                              unsigned* zmin, unsigned* zmax, int slices, int chunks, int rows_per) {
+  extern __shared__ unsigned lz[];
+  const int chunk = blockIdx.x % chunks, r0 = chunk * rows_per;
+  view_scan(m, pose.Tinv(), K, W, H, cols, rows, zmin, zmax, lz, blockIdx.x / chunks, slices, r0,
+            min(rows, r0 + rows_per), chunk == 0);
+}
+
+// The cells of an image too wide for k_view's chunks, straight into memory
+// (after the map's visibility pass).
 __global__ void __launch_bounds__(256) k_zrange(MapView m, const PosePair* pose, Intr K, int cols, int rows,
                                                 unsigned* zmin, unsigned* zmax) {
   zrange_at(m, pose, K, cols, rows, zmin, zmax, blockIdx.x, gridDim.x);
 }
 
-__global__ void __launch_bounds__(256) k_zrange_lds(MapView m, const PosePair* pose, Intr K, int cols, int rows,
-                                                    unsigned* zmin, unsigned* zmax) {
-  extern __shared__ unsigned lz[];
-  zrange_lds_at(m, pose, K, cols, rows, zmin, zmax, lz, blockIdx.x, gridDim.x);
+template <class VT, class P>
+__global__ void __launch_bounds__(256) k_march(MapView m, P pose, Intr K, int W, int H, int cols, const float* zmin,
+                                               const float* zmax, float4* vmap, float vsinv, float step_scale) {
+  march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, vmap, vsinv, step_scale, blockIdx.x);
 }
 
-// Workgroups of the LDS-privatised z-range: one per CU.
-constexpr int kZrangeLdsGroups = 256;
+// Workgroups of k_view: one per CU.
+constexpr int kViewGroups = 256;
 
-template <class VT>
-__global__ void __launch_bounds__(256) k_march(MapView m, const PosePair* pose, Intr K, int W, int H, int cols,
-                                               const float* zmin, const float* zmax, float4* vmap, float vsinv,
-                                               float step_scale) {
-  march_at<VT>(m, pose, K, W, H, cols, zmin, zmax, vmap, vsinv, step_scale, blockIdx.x);
-}
-
-// z-range tiles then the march (RayTraceEngine.cu:412-450) after the map's
-// visibility pass: z-range maps zmin/zmax of (W/8)*(H/8) cells, vertex map
-// `vmap` dense W*H float4.  `cells_reset`: the caller has already reset the
-// z-range cells on this stream.
-static int launch_raycast_to(hipStream_t s, yas_map* map, const Intr& K, int W, int H, unsigned* zmin,
-                             unsigned* zmax, float4* vmap, hipEvent_t before_march,
-                             const hipEvent_t* march_ev = nullptr, bool cells_reset = false) {
+// Visibility and z-range cells, then the march (RayTraceEngine.cu:412-450):
+// cells zmin/zmax of (W/8)*(H/8), vertex map `vmap` dense W*H float4.  The
+// pose is T's, or with T null the map's pose pair on the device; the map's
+// visible counter and the cells have been reset on this stream.
+template <class P>
+static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const double* T, const Intr& K, int W, int H,
+                             unsigned* zmin, unsigned* zmax, float4* vmap, hipEvent_t before_march,
+                             const hipEvent_t* march_ev) {
   MapView v = yas_map_view(map);
-  const PosePair* pose = yas_map_pose_dev(map);
-  const int cols = W / 8, rows = H / 8, ncell = cols * rows;
-  if (!cells_reset)
-    hipLaunchKernelGGL(k_zrange_init, dim3((ncell + 255) / 256), dim3(256), 0, s, zmin, zmax, ncell);
-  if (ncell <= kZrangeLdsCells) {
-    hipLaunchKernelGGL(k_zrange_lds, dim3(kZrangeLdsGroups), dim3(256), 2 * ncell * sizeof(unsigned), s, v, pose, K,
-                       cols, rows, zmin, zmax);
+  const int cols = W / 8, rows = H / 8;
+  if (cols <= kViewCells) {
+    // equal chunks of whole cell rows; the block list in slices, one
+    // workgroup a CU in all
+    const int most = kViewCells / cols, chunks = (rows + most - 1) / most, rows_per = (rows + chunks - 1) / chunks;
+    const int slices = chunks < kViewGroups ? kViewGroups / chunks : 1;
+    hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(256), 2 * sizeof(unsigned) * (size_t)rows_per * cols, s,
+                       v, pose, K, W, H, cols, rows, zmin, zmax, slices, chunks, rows_per);
   } else {
+    int r = T ? yas_map_visible_async(map, T, W, H) : yas_map_visible_prepared(map, W, H);
+    if (r) return r;
     int g = (v.num_blocks + 255) / 256;
     if (g > 2048) g = 2048;
-    hipLaunchKernelGGL(k_zrange, dim3(g), dim3(256), 0, s, v, pose, K, cols, rows, zmin, zmax);
+    hipLaunchKernelGGL(k_zrange, dim3(g), dim3(256), 0, s, v, yas_map_pose_dev(map), K, cols, rows, zmin, zmax);
   }
   YAS_LAUNCH_CHECK();
   if (before_march) YAS_HIP(hipEventRecord(before_march, s));
@@ -83,28 +95,33 @@ static int launch_raycast_to(hipStream_t s, yas_map* map, const Intr& K, int W, 
   const float* zf = (const float*)zmax;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
-      launch_timed(k_march<VoxI16>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxI16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
                    step_scale);
       break;
     case YAS_VOXEL_F16_U16:
-      launch_timed(k_march<VoxF16>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxF16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
                    step_scale);
       break;
     default:
-      launch_timed(k_march<VoxF32>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxF32, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
                    step_scale);
   }
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
-static int launch_raycast(yas_raycaster* rc, yas_map* map, hipEvent_t before_march = nullptr,
-                          const hipEvent_t* march_ev = nullptr, bool cells_reset = false) {
-  int r = launch_raycast_to(rc->ctx->stream, map, rc->K, rc->W, rc->H, rc->zmin, rc->zmax, rc->vmap, before_march,
-                            march_ev, cells_reset);
-  if (r) return r;
-  rc->last_map = map;
-  return YAS_OK;
+// A whole ray cast at pose T: the cells and the visible counter reset, then
+// launch_view_march.
+static int launch_raycast_to(yas_map* map, const double T[16], const Intr& K, int W, int H, unsigned* zmin,
+                             unsigned* zmax, float4* vmap) {
+  hipStream_t s = yas_map_ctx(map)->stream;
+  const int ncell = (W / 8) * (H / 8);
+  hipLaunchKernelGGL(k_cells_init, dim3((ncell + 255) / 256), dim3(256), 0, s, zmin, zmax, ncell,
+                     yas_map_view(map).ctr);
+  YAS_LAUNCH_CHECK();
+  PoseVal pose;
+  pose_pair_from(T, pose.p);
+  return launch_view_march(s, map, pose, T, K, W, H, zmin, zmax, vmap, nullptr, nullptr);
 }
 
 // ------------------------------------------------------------------ ray cast without allocation
@@ -139,11 +156,14 @@ static int scratch_on_device(int device, unsigned** out) {
 
 // Ray cast whose set-up the caller has already enqueued on this stream: the
 // map's pose pair written, its visible counter cleared and this ray caster's
-// z-range cells reset (the pipeline does all three in its first launch).
+// cells reset (the pipeline does all three in its first launch).
+// `before_march` (optional) is recorded between the view and march kernels.
 int yas_raycast_prepared(yas_raycaster* rc, yas_map* map, hipEvent_t before_march, const hipEvent_t* march_ev) {
-  int r = yas_map_visible_prepared(map, rc->W, rc->H);
+  int r = launch_view_march(rc->ctx->stream, map, PoseDev{yas_map_pose_dev(map)}, (const double*)nullptr, rc->K, rc->W,
+                            rc->H, rc->zmin, rc->zmax, rc->vmap, before_march, march_ev);
   if (r) return r;
-  return launch_raycast(rc, map, before_march, march_ev, true);
+  rc->last_map = map;
+  return YAS_OK;
 }
 
 float4* yas_raycaster_vmap_dev(yas_raycaster* rc) { return rc->vmap; }
@@ -215,9 +235,10 @@ int yas_raycast(yas_raycaster* rc, yas_map* map, const double T[16]) {
   YAS_REQUIRE_ACTIVE(map);
   YAS_HIP(hipSetDevice(rc->ctx->device));
   YAS_REQUIRE(yas_map_ctx(map)->stream == rc->ctx->stream, "yas_raycast: map and ray caster must share a stream");
-  int r = yas_map_visible_async(map, T, rc->W, rc->H);
+  int r = launch_raycast_to(map, T, rc->K, rc->W, rc->H, rc->zmin, rc->zmax, rc->vmap);
   if (r) return r;
-  return launch_raycast(rc, map);
+  rc->last_map = map;
+  return YAS_OK;
 }
 
 int yas_raycast_into(yas_map* map, const double T[16], const float K[4], int W, int H, float* vmap, size_t pitch) {
@@ -234,8 +255,7 @@ int yas_raycast_into(yas_map* map, const double T[16], const float K[4], int W, 
   unsigned* zr = nullptr;
   int r = scratch_on_device(ctx->device, &zr);
   if (r) return r;
-  if ((r = yas_map_visible_async(map, T, W, H))) return r;
-  return launch_raycast_to(ctx->stream, map, make_intr(K), W, H, zr, zr + kScratchCells, (float4*)vmap, nullptr);
+  return launch_raycast_to(map, T, make_intr(K), W, H, zr, zr + kScratchCells, (float4*)vmap);
 }
 
 int yas_raycaster_vmap(yas_raycaster* rc, float** vmap, size_t* pitch) {

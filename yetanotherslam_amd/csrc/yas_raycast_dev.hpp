@@ -12,12 +12,15 @@
 //            into 16x16 tiles (RayTraceEngine.cu:146-214) only distributed
 //            work; the per-cell result is the same min/max over all covering
 //            blocks, without its 100000-tile cap.
+//   view     the visibility pass and zrange in one pass over the block list
+//            (single maps; the batched launches run the two).
 //   march    one thread per pixel marches from the cell's zmin to zmax in
 //            voxel units (RayTraceEngine.cu:331-410).  The block looked up last
 //            is cached in registers, so consecutive samples inside one 8^3
 //            block cost no hash probe.
 #pragma once
 
+#include "yas_fusion_dev.hpp"
 #include "yas_internal.hpp"
 
 namespace yas {
@@ -118,6 +121,69 @@ __device__ inline void zrange_lds_at(const MapView& m, const PosePair* pose, con
     const unsigned a = lz[c], b = lz[ncell + c];
     if (a < far) atomicMin(&zmin[c], a);
     if (b != 0u) atomicMax(&zmax[c], b);
+  }
+}
+
+// What a ray cast needs of the block list in one pass: the visible blocks
+// compacted into the visible list (visible_scan's test) and their depth
+// ranges reduced into the cells, as zrange_lds_at does.  Workgroup (slice,
+// chunk) takes a contiguous slice of the block list and the cell rows r0 ..
+// r1 - 1 (nc cells, 2 words of LDS each); the workgroups of the first chunk
+// write the list.  One launch instead of two of about 5 us, and grids above
+// kZrangeLdsCells, whose atomics went to memory (25 us for 19200 cells),
+// reduce in LDS too, in chunks.
+constexpr int kViewCells = 9728;  // cells of a chunk: 76 KB, two workgroups a CU
+
+__device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& K, int W, int H, int cols, int rows,
+                                 unsigned* zmin, unsigned* zmax, unsigned* lds, int slice, int slices, int r0, int r1,
+                                 bool list) {
+  const int c0 = r0 * cols, nc = (r1 - r0) * cols;
+  unsigned* lmin = lds;
+  unsigned* lmax = lds + nc;
+  const unsigned far = __float_as_uint(kZrangeFar);
+  for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+    lmin[c] = far;
+    lmax[c] = 0u;
+  }
+  __syncthreads();
+  const int n0 = m.ctr[kCtrAlloc];
+  const int n = n0 < m.num_blocks ? n0 : m.num_blocks;
+  const int per = (n + slices - 1) / slices;
+  const int i1 = min(n, (slice + 1) * per);
+  for (int base = slice * per; base < i1; base += blockDim.x) {
+    const int i = base + (int)threadIdx.x;
+    bool vis = false;
+    unsigned long long key = 0;
+    if (i < i1) {
+      int bx, by, bz;
+      key = m.block_keys[i];
+      unpack_key(key, bx, by, bz);
+      vis = block_visible(bx, by, bz, Ti, K, W, H, m.voxel_size, m.depth_min, m.depth_max);
+    }
+    if (list) {
+      const unsigned long long mask = __ballot(vis);
+      if (mask) {
+        const int first = __ffsll(mask) - 1;
+        int b = 0;
+        if (lane_id() == first) b = atomicAdd(&m.ctr[kCtrVisible], __popcll(mask));
+        b = __shfl(b, first);
+        const int slot = b + __popcll(mask & lane_mask_lt());
+        if (vis && slot < m.num_blocks) m.visible[slot] = i;
+      }
+    }
+    CellBox cb;
+    if (!vis || !block_cells(m, Ti, K, cols, rows, key, cb)) continue;
+    for (int y = max(cb.y0, r0); y <= min(cb.y1, r1 - 1); ++y)
+      for (int x = cb.x0; x <= cb.x1; ++x) {
+        atomicMin(&lmin[y * cols + x - c0], cb.a);
+        atomicMax(&lmax[y * cols + x - c0], cb.b);
+      }
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+    const unsigned a = lmin[c], b = lmax[c];
+    if (a < far) atomicMin(&zmin[c0 + c], a);
+    if (b != 0u) atomicMax(&zmax[c0 + c], b);
   }
 }
 
@@ -356,7 +422,7 @@ __device__ inline bool march_ray(const MapView& m, float& rx, float& ry, float& 
 // unwritten get w = -1 (x = NaN, as the reference writes first).
 // Tile `tile` (raster order) of the image's (W/16)*(H/16) tiles of 16x16.
 template <class VT>
-__device__ inline void march_tile_at(const MapView& m, const PosePair* pose, const Intr& K, int W, int H, int cols,
+__device__ inline void march_tile_at(const MapView& m, const PoseF& T, const PoseF& Ti, const Intr& K, int W, int H, int cols,
                                      const float* zmin, const float* zmax, float4* vmap, float vsinv,
                                      float step_scale, int tile) {
   // A 16x16 tile per workgroup; each wavefront takes one 8x8 z-range cell,
@@ -371,7 +437,6 @@ __device__ inline void march_tile_at(const MapView& m, const PosePair* pose, con
   const float zf = zmax[(y >> 3) * cols + (x >> 3)];
   const float eps = 1.1920928955078125e-07f;
   if (!(zn < eps || zf < eps || zn != zn || zf != zf)) {
-    const PoseF T = pose->T;
     float pnx = K.invfx * ((float)x - K.cx) * zn, pny = K.invfy * ((float)y - K.cy) * zn;
     float dist_s = sqrtf(pnx * pnx + pny * pny + zn * zn) * vsinv;
     float bsx, bsy, bsz;
@@ -395,7 +460,6 @@ __device__ inline void march_tile_at(const MapView& m, const PosePair* pose, con
     const bool hit = __all(in_range) ? march_ray<VT, true>(m, rx, ry, rz, dx, dy, dz, dist_s, dist_e, step_scale)
                                      : march_ray<VT, false>(m, rx, ry, rz, dx, dy, dz, dist_s, dist_e, step_scale);
     if (hit) {
-      const PoseF Ti = pose->Tinv;
       float cx, cy, cz;
       xform(Ti, rx / vsinv, ry / vsinv, rz / vsinv, cx, cy, cz);
       out = make_float4(cx, cy, cz, 1.0f);
@@ -406,9 +470,9 @@ __device__ inline void march_tile_at(const MapView& m, const PosePair* pose, con
 
 // Workgroup b in launch order: the tiles dealt to the XCDs in bands (xcd_tile).
 template <class VT>
-__device__ inline void march_at(const MapView& m, const PosePair* pose, const Intr& K, int W, int H, int cols,
+__device__ inline void march_at(const MapView& m, const PoseF& T, const PoseF& Ti, const Intr& K, int W, int H, int cols,
                                 const float* zmin, const float* zmax, float4* vmap, float vsinv, float step_scale, int b) {
-  march_tile_at<VT>(m, pose, K, W, H, cols, zmin, zmax, vmap, vsinv, step_scale,
+  march_tile_at<VT>(m, T, Ti, K, W, H, cols, zmin, zmax, vmap, vsinv, step_scale,
                     xcd_tile(b, ((W + 15) >> 4) * ((H + 15) >> 4)));
 }
 

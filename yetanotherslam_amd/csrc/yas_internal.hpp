@@ -254,6 +254,10 @@ struct VoxI16 {  // int16 sdf (x32767, truncation) | uint8 weight << 16
   typedef uint32_t T;
   static constexpr int kFormat = YAS_VOXEL_I16_U8;
   __device__ static inline float sdf(T v) { return (float)(int16_t)(v & 0xFFFFu) / 32767.0f; }
+  // sdf(v) < 0, and sdf(v) by way of one 32-bit word
+  __device__ static inline bool negative(T v) { return (int16_t)(v & 0xFFFFu) < 0; }
+  __device__ static inline uint32_t sdf_word(T v) { return v; }
+  __device__ static inline float word_sdf(uint32_t w) { return sdf(w); }
   __device__ static inline bool observed(T v) { return ((v >> 16) & 0xFFu) != 0; }
   __device__ static inline uint32_t pack(float f) {
     int i = trunc_sat(f * 32767.0f);
@@ -282,6 +286,9 @@ struct VoxF32 {  // float sdf, float weight
   typedef float2 T;
   static constexpr int kFormat = YAS_VOXEL_F32_F32;
   __device__ static inline float sdf(T v) { return v.x; }
+  __device__ static inline bool negative(T v) { return v.x < 0.0f; }
+  __device__ static inline uint32_t sdf_word(T v) { return __builtin_bit_cast(uint32_t, v.x); }
+  __device__ static inline float word_sdf(uint32_t w) { return __builtin_bit_cast(float, w); }
   __device__ static inline bool observed(T v) { return v.y != 0.0f; }
   __device__ static inline T update(T v, float s, int maxw) {
     float w = v.y;
@@ -305,6 +312,9 @@ struct VoxF16 {  // half sdf | uint16 weight << 16
   }
   __device__ static inline uint32_t f2h(float f) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f); }
   __device__ static inline float sdf(T v) { return h2f(v); }
+  __device__ static inline bool negative(T v) { return h2f(v) < 0.0f; }
+  __device__ static inline uint32_t sdf_word(T v) { return v; }
+  __device__ static inline float word_sdf(uint32_t w) { return h2f(w); }
   __device__ static inline bool observed(T v) { return (v >> 16) != 0; }
   __device__ static inline T update(T v, float s, int maxw) {
     int w = (int)(v >> 16);

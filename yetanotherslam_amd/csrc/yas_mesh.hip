@@ -1,16 +1,13 @@
 // Marching-cubes mesh extraction: the reference's MeshEngine
 // (RGBDFusion/src/MeshEngine.cu:7-339, tables RGBDFusion/utils/TriangleTable.h).
 //
-// MI355X design: one wavefront (64 threads) per allocated block, eight
-// voxels per thread.  The +1 corners of a block's voxels live in up to seven
-// neighbour blocks; their pool indices are resolved once per workgroup
-// (seven hash probes) instead of eight probes per voxel, and the block with
-// its +1 halo is staged in LDS, so each voxel's eight corners are LDS reads.
-// Extraction is a count
-// pass, a three-phase device scan of the per-block counts and an emit pass,
-// so every block's output is contiguous and ordered by voxel index, then
-// table order: the output is deterministic, unlike the reference's atomic
-// triangle counter (MeshEngine.cu:246).
+// MI355X design: one wavefront per allocated block.  The +1 corners of a
+// block's voxels live in up to seven neighbour blocks, whose pool indices are
+// resolved once per block (seven hash probes) and recorded.  Extraction is a
+// count pass over two bits per voxel, a scan of the per-block counts and an
+// emission pass through lists, so every block's output is contiguous and
+// ordered by voxel index, then table order: the output is deterministic,
+// unlike the reference's atomic triangle counter (MeshEngine.cu:246).
 //
 // Two output forms share the count pass:
 //   * the reference's triangle soup (9 positions + 9 face-normal floats per
@@ -23,6 +20,7 @@
 //     lower end.  Triangles of a cube reference the owners' vertices, so a
 //     vertex is shared by every triangle that touches its edge.
 
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -41,189 +39,135 @@ __constant__ uint64_t kTriTable[256] = {
 #include "mc_tables.inc"
 };
 
-// MeshEngine.cu:76-112 corner order and MeshEngine.cu:150-224 edge geometry.
-__constant__ int kCorner[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0}, {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
-__constant__ int kEdgeA[12] = {0, 1, 2, 3, 4, 5, 6, 7, 0, 1, 2, 3};
-__constant__ int kEdgeB[12] = {1, 2, 3, 0, 5, 6, 7, 4, 4, 5, 6, 7};
+// MeshEngine.cu:76-112 corner order: corner c lies at x + (0x66 >> c & 1),
+// y + (0xCC >> c & 1), z + (c >> 2).
+__device__ inline int corner_step(int c, int sx, int sy, int sz) {
+  return ((0x66 >> c) & 1) * sx + ((0xCC >> c) & 1) * sy + (c >> 2) * sz;
+}
+// MeshEngine.cu:150-224: cube edge e runs from corner edge_a(e) to edge_b(e).
+__device__ inline int edge_a(int e) { return (int)((0x321076543210ull >> (4 * e)) & 7); }
+__device__ inline int edge_b(int e) { return (int)((0x765447650321ull >> (4 * e)) & 7); }
 
-// MeshEngine.cu:114-123 (thresholds compared in double: the literal is a double).
+// MeshEngine.cu:114-123.  The reference compares with the double 1e-6; the
+// largest float below it is 1e-6f, so |v| < 1e-6 is |v| <= 1e-6f.
 __device__ inline float edge_t(float v1, float v2) {
-  if (fabs((double)(0.0f - v1)) < 1e-6) return 0.0f;
-  if (fabs((double)(0.0f - v2)) < 1e-6) return 1.0f;
-  if (fabs((double)(v1 - v2)) < 1e-6) return 0.0f;
+  if (fabsf(0.0f - v1) <= 1e-6f) return 0.0f;
+  if (fabsf(0.0f - v2) <= 1e-6f) return 1.0f;
+  if (fabsf(v1 - v2) <= 1e-6f) return 0.0f;
   return (0.0f - v1) / (v2 - v1);
 }
 
+// Edge e's point at parameter t in the unit cube: along x for edges 0, 2, 4,
+// 6 (2 and 6 backwards), along y for 1, 3, 5, 7 (3 and 7 backwards), along z
+// for 8 to 11.
 __device__ inline void edge_offset(int e, float t, float& ox, float& oy, float& oz) {
-  switch (e) {
-    case 0: ox = t; oy = 0.f; oz = 0.f; break;
-    case 1: ox = 1.f; oy = t; oz = 0.f; break;
-    case 2: ox = 1.f - t; oy = 1.f; oz = 0.f; break;
-    case 3: ox = 0.f; oy = 1.f - t; oz = 0.f; break;
-    case 4: ox = t; oy = 0.f; oz = 1.f; break;
-    case 5: ox = 1.f; oy = t; oz = 1.f; break;
-    case 6: ox = 1.f - t; oy = 1.f; oz = 1.f; break;
-    case 7: ox = 0.f; oy = 1.f - t; oz = 1.f; break;
-    case 8: ox = 0.f; oy = 0.f; oz = t; break;
-    case 9: ox = 1.f; oy = 0.f; oz = t; break;
-    case 10: ox = 1.f; oy = 1.f; oz = t; break;
-    default: ox = 0.f; oy = 1.f; oz = t; break;
-  }
+  const float u = ((0x0CC >> e) & 1) ? 1.f - t : t;
+  ox = ((0x055 >> e) & 1) ? u : ((0x622 >> e) & 1) ? 1.f : 0.f;
+  oy = ((0x0AA >> e) & 1) ? u : ((0xC44 >> e) & 1) ? 1.f : 0.f;
+  oz = e >= 8 ? t : ((0x0F0 >> e) & 1) ? 1.f : 0.f;
+}
+// Owner of cube edge e: the voxel at the edge's lower end, an offset from
+// the cube's corner 0, and the edge's axis (0 = x, 1 = y, 2 = z).
+__device__ inline int owner_x(int e) { return (0x622 >> e) & 1; }
+__device__ inline int owner_y(int e) { return (0xC44 >> e) & 1; }
+__device__ inline int owner_z(int e) { return (0x0F0 >> e) & 1; }
+__device__ inline int owner_axis(int e) { return (0xAA4444 >> (2 * e)) & 3; }
+
+// One wavefront takes one block at a time, four a workgroup: they share a copy
+// of the triangulation table in LDS and meet at one barrier, after which the
+// wavefronts go on by themselves.
+constexpr int kMcWaves = 4;
+constexpr int kMcThreads = 64 * kMcWaves;
+constexpr int kMcCube = 9 * 9 * 9;  // a block and its +1 halo, index (z*9 + y)*9 + x
+
+// The block of this thread's wavefront.
+__device__ inline int mc_block() {
+  return __builtin_amdgcn_readfirstlane((int)blockIdx.x * kMcWaves + (int)(threadIdx.x >> 6));
 }
 
-// Owner of each cube edge: the voxel offset (from the cube's corner 0) of
-// the edge's lower end and the edge's axis (0 = x, 1 = y, 2 = z).
-__constant__ int kOwner[12][4] = {{0, 0, 0, 0}, {1, 0, 0, 1}, {0, 1, 0, 0}, {0, 0, 0, 1}, {0, 0, 1, 0}, {1, 0, 1, 1},
-                                  {0, 1, 1, 0}, {0, 0, 1, 1}, {0, 0, 0, 2}, {1, 0, 0, 2}, {1, 1, 0, 2}, {0, 1, 0, 2}};
+__device__ inline int mc_cube_at(int x, int y, int z) { return (z * 9 + y) * 9 + x; }
 
-// A workgroup of kMcThreads threads takes one block; thread t owns voxels
-// l = r * kMcThreads + t (r < kMcRounds), l = z*64 + y*8 + x, so the owned
-// voxels of a round are consecutive and the rounds in order are the voxel
-// order.  The block's 512 voxels and its +1 halo (217 voxels of up to seven
-// neighbour blocks) are staged in LDS as a 9x9x9 cube of (sdf, observed),
-// index (z*9 + y)*9 + x, once per block: the corner reads of the cubes then
-// come from LDS (eight per voxel), and a workgroup of one wavefront lets
-// eight times as many blocks wait on memory at once as one thread per voxel
-// did (measured against 128 threads: 5 % faster, against 512: 1.7 times).
-constexpr int kMcThreads = 64;
-constexpr int kMcRounds = 512 / kMcThreads;
-constexpr int kMcCube = 9 * 9 * 9;
-constexpr int kMcHalo = kMcCube - 512;
-
-// One word per voxel: the sdf, or kMcAbsent's bits where the voxel is not
-// observed (absent block or weight 0).  An observed NaN sdf is staged as the
-// canonical quiet NaN, so no observed value has those bits.
-constexpr unsigned kMcAbsent = 0xFFFFFFFFu;
-struct McCube {
-  float v[kMcCube];
-};
-__device__ inline float mc_staged(bool observed, float sdf) {
-  return !observed ? __uint_as_float(kMcAbsent) : sdf != sdf ? __uint_as_float(0x7FC00000u) : sdf;
-}
-
-// Pool indices of the block and its neighbours at offset (k&1, k>>1&1,
-// k>>2&1) in nb[k] (-1 if absent), and the staged cube.  The block's own
-// voxels are loaded while threads 0-7 probe the neighbours.  With `vinfo`,
-// the count pass's per-voxel vertex info of the same 9x9x9 voxels is staged
-// in `cvi` too (0 in absent blocks).
-// The neighbours come from `nbr_in` (the count pass's record, 8 per block)
-// when given, else from the hash, and are recorded in `nbr_out` when given.
+// A staged word's sdf; every NaN as the quiet one.
 template <class VT>
-__device__ inline void stage_cube(const MapView& m, int blk, int* nb, McCube& c, int& bx, int& by, int& bz,
-                                  const int* nbr_in, int* nbr_out, const uint16_t* vinfo = nullptr,
-                                  uint16_t* cvi = nullptr) {
-  const typename VT::T* vox = (const typename VT::T*)m.voxels;
-  const int t = threadIdx.x;
-  typename VT::T own[kMcRounds];
-#pragma unroll
-  for (int r = 0; r < kMcRounds; ++r) own[r] = vox[(size_t)blk * 512 + r * kMcThreads + t];
-  if (vinfo) {
-#pragma unroll
-    for (int r = 0; r < kMcRounds; ++r) {
-      const int l = r * kMcThreads + t;
-      cvi[((l >> 6) * 9 + ((l >> 3) & 7)) * 9 + (l & 7)] = vinfo[(size_t)blk * 512 + l];
-    }
-  }
-  unpack_key(m.block_keys[blk], bx, by, bz);
-  if (t < 8) {
-    const int b = nbr_in ? nbr_in[(size_t)blk * 8 + t]
-                         : t == 0 ? blk : find_block_xyz(m, bx + (t & 1), by + ((t >> 1) & 1), bz + ((t >> 2) & 1));
-    nb[t] = b;
-    if (nbr_out) nbr_out[(size_t)blk * 8 + t] = b;
-  }
-#pragma unroll
-  for (int r = 0; r < kMcRounds; ++r) {
-    const int l = r * kMcThreads + t, x = l & 7, y = (l >> 3) & 7, z = l >> 6;
-    const int i = (z * 9 + y) * 9 + x;
-    c.v[i] = mc_staged(VT::observed(own[r]), VT::sdf(own[r]));
-  }
-  __syncthreads();
-  for (int h = t; h < kMcHalo; h += kMcThreads) {
-    // the x = 8 face (81), then y = 8 with x < 8 (72), then z = 8 with x, y < 8 (64)
-    int x, y, z;
-    if (h < 81) {
-      x = 8; y = h % 9; z = h / 9;
-    } else if (h < 153) {
-      x = (h - 81) & 7; y = 8; z = (h - 81) >> 3;
-    } else {
-      x = (h - 153) & 7; y = (h - 153) >> 3; z = 8;
-    }
-    const int b = nb[(x >> 3) | ((y >> 3) << 1) | ((z >> 3) << 2)];
-    const size_t at = (size_t)b * 512 + ((z & 7) * 8 + (y & 7)) * 8 + (x & 7);
-    float v = __uint_as_float(kMcAbsent);
-    uint16_t vi = 0;
-    if (b >= 0) {
-      const typename VT::T w = vox[at];
-      if (vinfo) vi = vinfo[at];
-      v = mc_staged(VT::observed(w), VT::sdf(w));
-    }
-    const int i = (z * 9 + y) * 9 + x;
-    c.v[i] = v;
-    if (vinfo) cvi[i] = vi;
-  }
-  __syncthreads();
+__device__ inline float mc_sdf(uint32_t w) {
+  const float f = VT::word_sdf(w);
+  return f != f ? __uint_as_float(0x7FC00000u) : f;
 }
 
-// The 8 corner values of voxel (lx, ly, lz) and a bit mask of the corners
-// that are observed (in an allocated block with weight > 0), from the cube.
-__device__ inline int read_corners(const McCube& c, int lx, int ly, int lz, float* s) {
-  int valid = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int i = ((lz + kCorner[k][2]) * 9 + (ly + kCorner[k][1])) * 9 + (lx + kCorner[k][0]);
-    s[k] = c.v[i];
-    valid |= (int)(__float_as_uint(s[k]) != kMcAbsent) << k;
-  }
-  return valid;
+// Lanes of one wavefront exchanging values through LDS.
+__device__ inline void mc_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Cube index (MeshEngine.cu:76-112): -1 unless all 8 corners are observed.
-__device__ inline int cube_index(int valid, const float* s) {
-  if (valid != 0xFF) return -1;
-  int cube = 0;
-#pragma unroll
-  for (int c = 0; c < 8; ++c)
-    if (s[c] < 0.0f) cube |= 1 << c;
-  return cube;
+// A value per voxel of a block's +1 halo as a wavefront holds it: of the up
+// to seven neighbour blocks (pool index nb of lane k for the
+// offset (k&1, k>>1&1, k>>2&1), -1 absent: zeros) the faces x = 8 (lane (z,
+// y)), y = 8 (lane (z, x)), z = 8 (lane (y, x)), and in `e` the edges: lanes
+// 0-7 x = y = 8 (z = lane), 8-15 x = z = 8 (y = lane - 8), 16-23 y = z = 8
+// (x = lane - 16), 24 the corner.
+template <class T>
+struct McHalo {
+  T fx, fy, fz, e;
+};
+__device__ inline bool mc_bit(unsigned m, int i) { return (m >> i) & 1u; }
+template <class T>
+__device__ inline T mc_load(const T* src, bool wanted, int blk, int at) {
+  T v = {};
+  if (wanted && blk >= 0) v = src[(size_t)blk * 512 + at];
+  return v;
+}
+// The layers z = 0..8 whose bit of `layers` is set; zeros for the others.
+template <class T>
+__device__ inline void mc_load_halo(const T* src, int nb, unsigned layers, McHalo<T>& v) {
+  const int lane = threadIdx.x & 63, a = lane & 7, b = lane >> 3;
+  const bool mine = mc_bit(layers, b), top = mc_bit(layers, 8);
+  v.fx = mc_load(src, mine, __builtin_amdgcn_readlane(nb, 1), lane * 8);
+  v.fy = mc_load(src, mine, __builtin_amdgcn_readlane(nb, 2), b * 64 + a);
+  v.fz = mc_load(src, top, __builtin_amdgcn_readlane(nb, 4), lane);
+  v.e = mc_load(src, lane < 8 ? mc_bit(layers, a) : lane < 25 && top, __shfl(nb, b == 0 ? 3 : b == 1 ? 5 : b == 2 ? 6 : 7),
+                b == 0 ? a * 64 : b == 1 ? a * 8 : a);
+}
+// The halo's values written to LDS as f(value), index mc_cube_at.
+template <class T, class S, class F>
+__device__ inline void mc_stage_halo(const McHalo<T>& v, S* cube, F f) {
+  const int lane = threadIdx.x & 63, a = lane & 7, b = lane >> 3;
+  cube[mc_cube_at(8, a, b)] = f(v.fx);
+  cube[mc_cube_at(a, 8, b)] = f(v.fy);
+  cube[mc_cube_at(a, b, 8)] = f(v.fz);
+  if (lane < 25) cube[mc_cube_at(b == 2 ? a : 8, b == 1 ? a : 8, b == 0 ? a : 8)] = f(v.e);
 }
 
-// Owned edges of the voxel (bit a = edge along axis a from corner 0 to
-// corner 1, 3 or 4) that carry a vertex.
-__device__ inline int owned_edges(int valid, const float* s) {
-  const int far[3] = {1, 3, 4};
-  int m = 0;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const int c = far[a];
-    if ((valid & 1) && (valid & (1 << c)) && ((s[0] < 0.0f) != (s[c] < 0.0f))) m |= 1 << a;
-  }
-  return m;
+// Inclusive scan of v over the wavefront.
+__device__ inline unsigned mc_scan(unsigned v) {
+  int x = (int)v;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31
+  return (unsigned)x;
 }
-
-// Exclusive prefix of v over the threads of a workgroup (thread order), and
-// the workgroup total.  `wsum` holds one int per wavefront.
-// Exclusive prefix of v over a one-wavefront workgroup (the marching-cubes
-// passes run kMcThreads = 64 threads); `total` receives the sum.  No LDS
-// word and no barrier.
-static_assert(kMcThreads == 64, "the marching-cubes passes run one wavefront per block");
-__device__ inline int wave_excl_scan(int v, int& total) {
-  const int lane = threadIdx.x & 63;
-  int inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += t;
-  }
-  total = __builtin_amdgcn_readlane(inc, 63);
-  return inc - v;
+// The value of the next lane of 16 (the last: 0).
+__device__ inline unsigned mc_next_lane(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xF, 0xF, false);  // row_shl:1
 }
-// Triangle counts of the 256 cases (kTriTable's low nibbles) into LDS, for
-// the count pass to read per voxel instead of the table in memory (the
-// emission passes need the whole table word); published by stage_cube's
-// first barrier.
-__device__ inline void stage_tri_counts(unsigned char* nt) {
-  for (int i = threadIdx.x; i < 256; i += kMcThreads) nt[i] = (unsigned char)(kTriTable[i] & 0xF);
+// Bits i, 8 + i, .., 56 + i of m to bits 0..7.
+__device__ inline unsigned mc_gather(unsigned long long m, int i) {
+  const unsigned lo = ((unsigned)m >> i) & 0x01010101u, hi = ((unsigned)(m >> 32) >> i) & 0x01010101u;
+  return ((lo * 0x01020408u) >> 24) | (((hi * 0x01020408u) >> 24) << 4);
 }
+// Bits 0..7 of v to bits 0, 4, .., 28.
+__device__ inline unsigned mc_spread4(unsigned v) {
+  v &= 0xFFu;
+  v = (v | (v << 12)) & 0x000F000Fu;
+  v = (v | (v << 6)) & 0x03030303u;
+  return (v | (v << 3)) & 0x11111111u;
+}
+// Bits 0..3 of v to bits 0, 8, 16, 24.
+__device__ inline unsigned mc_spread8(unsigned v) { return ((v & 0xFu) * 0x00204081u) & 0x01010101u; }
 
 __device__ inline int block_excl_scan(int v, int* wsum, int& total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -247,64 +191,136 @@ __device__ inline int block_excl_scan(int v, int* wsum, int& total) {
 }
 
 // Count pass: per block, triangles and owned vertices; per voxel, the cube
-// index and (local vertex prefix << 3 | owned edge mask).  One scan a round
-// of the packed counts (triangles << 16 | vertices: a block has at most 2560
-// and 1536).
+// index (MeshEngine.cu:76-112; -1 unless all 8 corners are observed) and
+// (local vertex prefix << 3 | owned edge mask).  It needs two bits of a
+// voxel, its sign and whether it is observed.  A lane packs those of its
+// column of voxels z = 0..8 into one word, signs in bits 0-8 and observed in
+// bits 16-24; with the columns at x + 1, y + 1 and both, fetched from the next
+// lanes, the tests of a column's 8 cubes are bit operations on 4 words, and
+// the 8 slices' vertex prefixes are two scans of bytes (a slice owns at most
+// 192 vertices).  Bound by memory: 58k float32 blocks, some 380 MB with the
+// neighbours' faces, in 85 us.  (121 us with the block in LDS, each voxel
+// reading its 8 corners there; 107 us with a slice's planes as 64-bit scalar
+// masks, some 850 scalar instructions a block for a CU's one scalar unit.)
 template <class VT>
 __global__ void __launch_bounds__(kMcThreads) k_mc_count(MapView m, int nblocks, int2* counts, int16_t* cases,
                                                          uint16_t* vinfo, int* nbr) {
-  __shared__ int nb[8];
   __shared__ unsigned char tri_n[256];
-  __shared__ McCube c;
-  const int blk = blockIdx.x;
+  if (threadIdx.x < 256) tri_n[threadIdx.x] = (unsigned char)(kTriTable[threadIdx.x] & 0xF);
+  __syncthreads();
+  const int blk = mc_block();
   if (blk >= nblocks) return;
-  int bx, by, bz;
-  stage_tri_counts(tri_n);
-  stage_cube<VT>(m, blk, nb, c, bx, by, bz, nullptr, nbr);
-  int tri = 0, vert = 0;  // totals of the rounds so far
-#pragma unroll 1
-  for (int r = 0; r < kMcRounds; ++r) {
-    const int l = r * kMcThreads + threadIdx.x, lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-    float s[8];
-    const int valid = read_corners(c, lx, ly, lz, s);
-    const int cube = cube_index(valid, s);
-    const int om = owned_edges(valid, s);
-    cases[(size_t)blk * 512 + l] = (int16_t)cube;
-    const int nt = cube > 0 ? (int)tri_n[cube] : 0;
-    int total;
-    const int pre = wave_excl_scan((nt << 16) | __popc(om), total);
-    vinfo[(size_t)blk * 512 + l] = (uint16_t)(((vert + (pre & 0xFFFF)) << 3) | om);
-    tri += total >> 16;
-    vert += total & 0xFFFF;
+  const int lane = threadIdx.x & 63, a = lane & 7, b = lane >> 3;
+  const typename VT::T* vox = (const typename VT::T*)m.voxels;
+  typename VT::T own[8];
+  McHalo<typename VT::T> v;
+#pragma unroll
+  for (int z = 0; z < 8; ++z) own[z] = vox[(size_t)blk * 512 + z * 64 + lane];
+  int nb = -1;
+  if (lane < 8) {
+    int bx, by, bz;
+    unpack_key(m.block_keys[blk], bx, by, bz);
+    nb = lane == 0 ? blk : find_block_xyz(m, bx + (lane & 1), by + ((lane >> 1) & 1), bz + ((lane >> 2) & 1));
+    nbr[(size_t)blk * 8 + lane] = nb;
   }
-  if (threadIdx.x == 0) counts[blk] = make_int2(tri, vert);
+  mc_load_halo(vox, nb, 0x1FFu, v);
+  unsigned c0 = 0;  // this lane's column
+#pragma unroll
+  for (int z = 0; z < 9; ++z) {
+    typename VT::T w = v.fz;
+    if (z < 8) w = own[z];
+    c0 |= (VT::negative(w) ? 1u << z : 0u) | (VT::observed(w) ? 0x10000u << z : 0u);
+  }
+  // the columns (8, y = b), (x = a, 8) and (8, 8)
+  const unsigned en = (unsigned)__ballot(VT::negative(v.e)), eo = (unsigned)__ballot(VT::observed(v.e));
+  const unsigned hx = mc_gather(__ballot(VT::negative(v.fx)), b) | (((en >> (8 + b)) & 1u) << 8) |
+                      (mc_gather(__ballot(VT::observed(v.fx)), b) | (((eo >> (8 + b)) & 1u) << 8)) << 16;
+  const unsigned hy = mc_gather(__ballot(VT::negative(v.fy)), a) | (((en >> (16 + a)) & 1u) << 8) |
+                      (mc_gather(__ballot(VT::observed(v.fy)), a) | (((eo >> (16 + a)) & 1u) << 8)) << 16;
+  const unsigned hxy = ((en & 0xFFu) | ((en >> 16) & 0x100u)) | ((eo & 0xFFu) | ((eo >> 16) & 0x100u)) << 16;
+  // the columns at the cube's corners 1 (x + 1), 2 (x + 1, y + 1), 3 (y + 1)
+  const unsigned n0 = mc_next_lane(c0), nhy = mc_next_lane(hy);
+  const unsigned c1 = a == 7 ? hx : n0;
+  const unsigned u0 = (unsigned)__shfl_down((int)c0, 8, 64), u1 = (unsigned)__shfl_down((int)c1, 8, 64);
+  const unsigned c3 = b == 7 ? hy : u0;
+  const unsigned c2 = b < 7 ? u1 : a == 7 ? hxy : nhy;
+  unsigned all = c0 & c1 & c2 & c3, any = c0 | c1 | c2 | c3;
+  all &= all >> 1;
+  any |= any >> 1;
+  const unsigned valid = (all >> 16) & 0xFFu;
+  const unsigned mixed = valid & any & ~all;  // cubes with both signs: the others have no triangles
+  const unsigned lo = mc_spread4(c0) | mc_spread4(c1) << 1 | mc_spread4(c2) << 2 | mc_spread4(c3) << 3;
+  const unsigned hi = ((c0 >> 8) & 1u) | ((c1 >> 7) & 2u) | ((c2 >> 6) & 4u) | ((c3 >> 5) & 8u);
+  const unsigned long long corners = (unsigned long long)hi << 32 | lo;
+  const size_t at = (size_t)blk * 512 + lane;
+  int tri = 0;
+#pragma unroll
+  for (int z = 0; z < 8; ++z) {
+    const int cube = (int)(corners >> (4 * z)) & 0xFF;
+    cases[at + z * 64] = (int16_t)((valid >> z) & 1u ? cube : -1);
+    if ((mixed >> z) & 1u) tri += (int)tri_n[cube];
+  }
+  // owned edges: both ends observed, with a sign change
+  const unsigned ex = (c0 ^ c1) & (c0 >> 16) & (c1 >> 16) & 0xFFu;
+  const unsigned ey = (c0 ^ c3) & (c0 >> 16) & (c3 >> 16) & 0xFFu;
+  const unsigned ez = (c0 ^ (c0 >> 1)) & (c0 >> 16) & (c0 >> 17) & 0xFFu;
+  const unsigned edges = mc_spread4(ex) | mc_spread4(ey) << 1 | mc_spread4(ez) << 2;
+  int vert = 0;  // vertices of the slices below
+  if (__ballot(edges != 0u) != 0ull) {
+    const unsigned nlo = mc_spread8(ex) + mc_spread8(ey) + mc_spread8(ez);
+    const unsigned nhi = mc_spread8(ex >> 4) + mc_spread8(ey >> 4) + mc_spread8(ez >> 4);
+    const unsigned slo = mc_scan(nlo), shi = mc_scan(nhi);
+    const unsigned tlo = (unsigned)__builtin_amdgcn_readlane((int)slo, 63);
+    const unsigned thi = (unsigned)__builtin_amdgcn_readlane((int)shi, 63);
+#pragma unroll
+    for (int z = 0; z < 8; ++z) {
+      const int sh = 8 * (z & 3);
+      const int pre = vert + (int)(((z < 4 ? slo - nlo : shi - nhi) >> sh) & 0xFFu);
+      vinfo[at + z * 64] = (uint16_t)((pre << 3) | ((edges >> (4 * z)) & 7u));
+      vert += (int)(((z < 4 ? tlo : thi) >> sh) & 0xFFu);
+    }
+  } else {
+#pragma unroll
+    for (int z = 0; z < 8; ++z) vinfo[at + z * 64] = 0;
+  }
+  tri = (int)mc_scan((unsigned)tri);
+  if (lane == 63) counts[blk] = make_int2(tri, vert);
 }
 
-// Three-phase exclusive scan of int2 counts: 1024-element chunks scanned in
-// parallel, the chunk totals scanned by one workgroup, then added back.
-__global__ void __launch_bounds__(1024) k_scan_local(const int2* in, int2* out, int n, int2* chunk) {
+// Exclusive scan of the blocks' counts: 1024-block chunks scanned in parallel
+// into `out`, and the chunks' totals, by the workgroup that ends last, into
+// `chunk`; block i's prefix is out[i] + chunk[i >> kMcChunkShift], which its
+// readers add.  (As three launches, local scan, chunk scan and addition, it
+// cost 14 us of a 284 us extraction.)  `done` is 0 before and after.
+constexpr int kMcChunkShift = 10, kMcChunk = 1 << kMcChunkShift;
+__device__ inline unsigned long long mc_pack2(int x, int y) {
+  return (unsigned long long)(unsigned)x | (unsigned long long)(unsigned)y << 32;
+}
+__global__ void __launch_bounds__(kMcChunk) k_mc_scan(const int2* in, int2* out, int n, unsigned long long* chunk,
+                                                      int2* total, unsigned* done) {
   __shared__ int wsum[16];
-  const int i = blockIdx.x * 1024 + threadIdx.x;
+  __shared__ int carry[2];
+  __shared__ int last;
+  const int i = blockIdx.x * kMcChunk + threadIdx.x, nchunks = gridDim.x;
   const int2 v = i < n ? in[i] : make_int2(0, 0);
   int tx, ty;
   const int ex = block_excl_scan(v.x, wsum, tx);
   const int ey = block_excl_scan(v.y, wsum, ty);
   if (i < n) out[i] = make_int2(ex, ey);
-  if (threadIdx.x == 0) chunk[blockIdx.x] = make_int2(tx, ty);
-}
-
-__global__ void __launch_bounds__(1024) k_scan_chunks(int2* chunk, int nchunks, int2* total) {
-  __shared__ int wsum[16];
-  __shared__ int carry[2];
-  if (threadIdx.x == 0) carry[0] = carry[1] = 0;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(&chunk[blockIdx.x], mc_pack2(tx, ty), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nchunks - 1u;
+    carry[0] = carry[1] = 0;
+  }
   __syncthreads();
-  for (int base = 0; base < nchunks; base += 1024) {
-    const int i = base + threadIdx.x;
-    const int2 v = i < nchunks ? chunk[i] : make_int2(0, 0);
-    int tx, ty;
-    const int ex = block_excl_scan(v.x, wsum, tx);
-    const int ey = block_excl_scan(v.y, wsum, ty);
-    if (i < nchunks) chunk[i] = make_int2(carry[0] + ex, carry[1] + ey);
+  if (!last) return;
+  for (int base = 0; base < nchunks; base += kMcChunk) {
+    const int c = base + threadIdx.x;
+    unsigned long long w = 0;
+    if (c < nchunks) w = __hip_atomic_load(&chunk[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int cx = block_excl_scan((int)(unsigned)w, wsum, tx);
+    const int cy = block_excl_scan((int)(unsigned)(w >> 32), wsum, ty);
+    if (c < nchunks) chunk[c] = mc_pack2(carry[0] + cx, carry[1] + cy);
     __syncthreads();
     if (threadIdx.x == 0) {
       carry[0] += tx;
@@ -312,135 +328,359 @@ __global__ void __launch_bounds__(1024) k_scan_chunks(int2* chunk, int nchunks, 
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) *total = make_int2(carry[0], carry[1]);
+  if (threadIdx.x == 0) {
+    *total = make_int2(carry[0], carry[1]);
+    *done = 0;
+  }
 }
+// The scan's result for block `blk`.
+struct McOffsets {
+  const int2* local;
+  const unsigned long long* chunk;
+  __device__ inline int tri(int blk) const { return local[blk].x + (int)(unsigned)chunk[blk >> kMcChunkShift]; }
+  __device__ inline int vert(int blk) const { return local[blk].y + (int)(unsigned)(chunk[blk >> kMcChunkShift] >> 32); }
+};
 
-__global__ void __launch_bounds__(1024) k_scan_add(int2* out, const int2* chunk, int n) {
-  const int i = blockIdx.x * 1024 + threadIdx.x;
-  if (i >= n) return;
-  const int2 c = chunk[blockIdx.x], v = out[i];
-  out[i] = make_int2(v.x + c.x, v.y + c.y);
+// The emission passes.  A wavefront takes blocks in turn; lane l holds row
+// (y, z) = (l & 7, l >> 3) of the count pass's records, voxels 8 l + x, so one
+// 16-byte load brings each, a lane's entries are consecutive in voxel order
+// and one scan places them.  The records of its next block are loaded while
+// it works on the present one; of the sdf, the slices that this block's
+// triangles or vertices need.
+// The triangles and vertices are first listed in LDS and then taken from the
+// list one per lane: only one voxel in five of a surface block has triangles,
+// and those up to five, so emitting them voxel by voxel left most lanes idle,
+// and the lanes of a list write consecutive entries.  A list holds entries
+// done .. done + its size of the block; a block with more is listed again.
+// 58k float32 blocks, 6.0 M indexed triangles: 110 us (246 us voxel by voxel,
+// with the cubes formed again from a staged block); 2.1k int16 blocks, 232k
+// triangles of the soup: 18 us (86 us).  About as much instruction issue as
+// memory; 5 waves a SIMD instead of 4 (96 registers, some spilled) 115 us.
+//   triangle entry: voxel (9 bits) | which of its triangles << 9
+//   vertex entry:   voxel (9 bits) | axis << 9
+constexpr int kTriList = 512, kVertList = 320;
+
+struct McTables {
+  uint64_t word[256];       // kTriTable
+  unsigned char count[256]; // triangles
+};
+__device__ inline void mc_fill_tables(McTables& T) {
+  T.word[threadIdx.x] = kTriTable[threadIdx.x];
+  T.count[threadIdx.x] = (unsigned char)(kTriTable[threadIdx.x] & 0xF);
 }
+static_assert(kMcThreads == 256, "mc_fill_tables: a thread per case");
 
-// Vertex on cube edge e of the voxel at integer position p (voxel units),
-// MeshEngine.cu:114-224: corner A + t * (edge direction), scaled by vs.
-__device__ inline void edge_vertex(int e, const float* s, float px, float py, float pz, float vs, float* out) {
-  float t = edge_t(s[kEdgeA[e]], s[kEdgeB[e]]);
-  float ox, oy, oz;
-  edge_offset(e, t, ox, oy, oz);
-  out[0] = (px + ox) * vs;
-  out[1] = (py + oy) * vs;
-  out[2] = (pz + oz) * vs;
+// A lane's row of a per-voxel 16-bit record.
+struct McRow {
+  unsigned w[4];
+  __device__ inline unsigned at(int x) const { return (w[x >> 1] >> (16 * (x & 1))) & 0xFFFFu; }
+};
+__device__ inline McRow mc_load_row(const void* records, int blk) {
+  const uint4 v = ((const uint4*)records)[(size_t)blk * 64 + (threadIdx.x & 63)];
+  return McRow{{v.x, v.y, v.z, v.w}};
+}
+// Triangles of the row's voxels, 4 bits each.
+__device__ inline unsigned mc_row_triangles(const McTables& T, const McRow& cases) {
+  unsigned nt = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const unsigned c = cases.at(x);  // 0xFFFF: not all corners observed
+    nt |= (c - 1u < 254u ? (unsigned)T.count[c] : 0u) << (4 * x);
+  }
+  return nt;
+}
+__device__ inline int mc_nibble_sum(unsigned v) {  // of eight values, 40 at most
+  v = (v & 0x0F0F0F0Fu) + ((v >> 4) & 0x0F0F0F0Fu);
+  return (int)((v * 0x01010101u) >> 24);
+}
+// Slices with a lane for which `has` holds.
+__device__ inline unsigned mc_slices(bool has) {
+  unsigned long long m = __ballot(has);
+  m |= m >> 4;
+  m |= m >> 2;
+  m |= m >> 1;
+  return mc_gather(m, 0);
+}
+// The lane's triangles, at block positions first .. first + their number, put
+// where the list's window [done, done + kTriList) holds them; last first.
+__device__ inline void mc_list_triangles(uint16_t* list, unsigned nt, int end, int done) {
+  const unsigned row = (threadIdx.x & 63) * 8;
+  while (nt) {
+    const int x4 = (31 - __clz((int)nt)) & ~3;
+    const unsigned i = (nt >> x4) - 1u;
+    nt -= 1u << x4;
+    const unsigned at = (unsigned)(--end - done);
+    if (at < (unsigned)kTriList) list[at] = (uint16_t)(row | (unsigned)(x4 >> 2) | (i << 9));
+  }
+}
+__device__ inline void mc_list_vertices(uint16_t* list, unsigned edges, int first, int done) {
+  const unsigned row = (threadIdx.x & 63) * 8;
+  while (edges) {
+    const int bit = __ffs((int)edges) - 1;
+    edges &= edges - 1u;
+    const unsigned at = (unsigned)(first++ - done);
+    if (at < (unsigned)kVertList) list[at] = (uint16_t)(row | (unsigned)(bit >> 2) | (unsigned)(bit & 3) << 9);
+  }
+}
+// A block's sdf and its halo's, layers z of the set bits, as 32-bit words.
+template <class VT>
+struct McSdf {
+  static constexpr int kPer = 16 / (int)sizeof(typename VT::T);  // voxels of one load
+  static constexpr int kLoads = 8 / kPer;
+  uint4 own[kLoads];
+  McHalo<typename VT::T> halo;
+  __device__ inline void load(const typename VT::T* vox, int blk, int nb, unsigned layers) {
+    const int lane = threadIdx.x & 63;
+    const uint4* src = (const uint4*)(vox + (size_t)blk * 512);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      own[i] = make_uint4(0, 0, 0, 0);
+      if (mc_bit(layers, (i * 64 + lane) * kPer >> 6)) own[i] = src[i * 64 + lane];
+    }
+    mc_load_halo(vox, nb, layers, halo);
+  }
+  __device__ inline void stage(uint32_t* cube) const {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int l = (i * 64 + lane) * kPer, at = mc_cube_at(l & 7, (l >> 3) & 7, l >> 6);
+      if constexpr (kPer == 2) {
+        cube[at] = own[i].x;  // {sdf, weight} twice
+        cube[at + 1] = own[i].z;
+      } else {
+        cube[at] = own[i].x;
+        cube[at + 1] = own[i].y;
+        cube[at + 2] = own[i].z;
+        cube[at + 3] = own[i].w;
+      }
+    }
+    mc_stage_halo(halo, cube, [](const typename VT::T& w) { return VT::sdf_word(w); });
+  }
+};
+
+__device__ inline void mc_voxel_xyz(int l, int& x, int& y, int& z) {
+  x = l & 7;
+  y = (l >> 3) & 7;
+  z = l >> 6;
 }
 
 // Emit, reference form: triangle slot = block offset + exclusive prefix (in
 // voxel index order) of the per-voxel counts.
+struct McSoupLds {
+  uint32_t sdf[kMcCube];
+  alignas(16) uint16_t cases[512];
+  uint16_t tri[kTriList];
+};
 template <class VT>
-__global__ void __launch_bounds__(kMcThreads) k_mc_emit(MapView m, int nblocks, const int2* offsets, float* tris,
-                                                        float* normals, int cap, const int* nbr) {
-  __shared__ int nb[8];
-  __shared__ McCube c;
-  const int blk = blockIdx.x;
-  if (blk >= nblocks) return;
-  int bx, by, bz;
-  stage_cube<VT>(m, blk, nb, c, bx, by, bz, nbr, nullptr);
-  const float vs = m.voxel_size;
-  int base = offsets[blk].x;
-#pragma unroll 1
-  for (int r = 0; r < kMcRounds; ++r) {
-    const int l = r * kMcThreads + threadIdx.x, lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-    float s[8];
-    const int cube = cube_index(read_corners(c, lx, ly, lz, s), s);
-    const uint64_t word = cube > 0 ? kTriTable[cube] : 0ull;
-    const int nt = (int)(word & 0xF);
-    int total;
-    int slot = base + wave_excl_scan(nt, total);
-    base += total;
-    const float px = (float)(bx * 8 + lx), py = (float)(by * 8 + ly), pz = (float)(bz * 8 + lz);
-    for (int i = 0; i < nt && slot < cap; ++i, ++slot) {
-      float a[3], b[3], cc[3];
-      edge_vertex((int)((word >> (4 + 12 * i)) & 0xF), s, px, py, pz, vs, a);
-      edge_vertex((int)((word >> (8 + 12 * i)) & 0xF), s, px, py, pz, vs, b);
-      edge_vertex((int)((word >> (12 + 12 * i)) & 0xF), s, px, py, pz, vs, cc);
-      float u0 = b[0] - a[0], u1 = b[1] - a[1], u2 = b[2] - a[2];
-      float w0 = cc[0] - a[0], w1 = cc[1] - a[1], w2 = cc[2] - a[2];
-      float n0 = u1 * w2 - u2 * w1, n1 = u2 * w0 - u0 * w2, n2 = u0 * w1 - u1 * w0;
-      float q = n0 * n0 + n1 * n1 + n2 * n2;
-      if (q > 0.0f) {
-        float nn = sqrtf(q);
-        n0 = n0 / nn; n1 = n1 / nn; n2 = n2 / nn;
-      }
-      float* T = tris + (size_t)slot * 9;
-      T[0] = a[0]; T[1] = a[1]; T[2] = a[2];
-      T[3] = b[0]; T[4] = b[1]; T[5] = b[2];
-      T[6] = cc[0]; T[7] = cc[1]; T[8] = cc[2];
-      if (normals) {
-        float* N = normals + (size_t)slot * 9;
-        N[0] = N[3] = N[6] = n0;
-        N[1] = N[4] = N[7] = n1;
-        N[2] = N[5] = N[8] = n2;
+__device__ inline void mc_soup_flush(const McSoupLds& S, const McTables& T, int bx, int by, int bz, float vs,
+                                     int first, int n, float* tris, float* normals, int cap) {
+  for (int t = threadIdx.x & 63; t < n && first + t < cap; t += 64) {
+    const unsigned ent = S.tri[t];
+    int x, y, z;
+    mc_voxel_xyz((int)(ent & 511u), x, y, z);
+    const unsigned edges = (unsigned)(T.word[S.cases[ent & 511u]] >> (4 + 12 * (ent >> 9)));
+    const int at = mc_cube_at(x, y, z);
+    const float px = (float)(bx * 8 + x), py = (float)(by * 8 + y), pz = (float)(bz * 8 + z);
+    float p[3][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      // MeshEngine.cu:114-224: corner A + t * (edge direction), scaled by vs
+      const int e = (int)((edges >> (4 * k)) & 0xF);
+      const float sa = mc_sdf<VT>(S.sdf[at + corner_step(edge_a(e), 1, 9, 81)]);
+      const float sb = mc_sdf<VT>(S.sdf[at + corner_step(edge_b(e), 1, 9, 81)]);
+      float ox, oy, oz;
+      edge_offset(e, edge_t(sa, sb), ox, oy, oz);
+      p[k][0] = (px + ox) * vs;
+      p[k][1] = (py + oy) * vs;
+      p[k][2] = (pz + oz) * vs;
+    }
+    const float u0 = p[1][0] - p[0][0], u1 = p[1][1] - p[0][1], u2 = p[1][2] - p[0][2];
+    const float w0 = p[2][0] - p[0][0], w1 = p[2][1] - p[0][1], w2 = p[2][2] - p[0][2];
+    float n0 = u1 * w2 - u2 * w1, n1 = u2 * w0 - u0 * w2, n2 = u0 * w1 - u1 * w0;
+    const float q = n0 * n0 + n1 * n1 + n2 * n2;
+    if (q > 0.0f) {
+      const float nn = sqrtf(q);
+      n0 = n0 / nn; n1 = n1 / nn; n2 = n2 / nn;
+    }
+    float* P = tris + (size_t)(first + t) * 9;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      P[3 * k] = p[k][0]; P[3 * k + 1] = p[k][1]; P[3 * k + 2] = p[k][2];
+    }
+    if (normals) {
+      float* N = normals + (size_t)(first + t) * 9;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        N[3 * k] = n0; N[3 * k + 1] = n1; N[3 * k + 2] = n2;
       }
     }
   }
 }
-
-// Emit, indexed form: the voxel's owned vertices, then its triangles as
-// indices of the owners' vertices.
 template <class VT>
-__global__ void __launch_bounds__(kMcThreads) k_mc_emit_indexed(MapView m, int nblocks, const int2* offsets,
-                                                                const uint16_t* vinfo, float* verts, int vcap,
-                                                                int* tris, int tcap, const int* nbr) {
-  __shared__ int nb[8];
-  __shared__ int vbase[8];
-  __shared__ McCube c;
-  __shared__ uint16_t cvi[kMcCube];
-  const int blk = blockIdx.x;
-  if (blk >= nblocks) return;
-  int bx, by, bz;
-  stage_cube<VT>(m, blk, nb, c, bx, by, bz, nbr, nullptr, vinfo, cvi);
-  if (threadIdx.x < 8) vbase[threadIdx.x] = nb[threadIdx.x] >= 0 ? offsets[nb[threadIdx.x]].y : 0;
+__global__ void __launch_bounds__(kMcThreads) k_mc_emit(MapView m, int nblocks, McOffsets offsets,
+                                                        const int16_t* cases, float* tris, float* normals, int cap,
+                                                        const int* nbr) {
+  __shared__ McTables T;
+  __shared__ McSoupLds lds[kMcWaves];
+  mc_fill_tables(T);
   __syncthreads();
-  const float vs = m.voxel_size;
-  int base = offsets[blk].x;
-  const int far[3] = {1, 3, 4};
-#pragma unroll 1
-  for (int r = 0; r < kMcRounds; ++r) {
-    const int l = r * kMcThreads + threadIdx.x, lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-    float s[8];
-    const int valid = read_corners(c, lx, ly, lz, s);
-    const int cube = cube_index(valid, s);
-    const uint64_t word = cube > 0 ? kTriTable[cube] : 0ull;
-    const int nt = (int)(word & 0xF);
-    int total;
-    int slot = base + wave_excl_scan(nt, total);
-    base += total;
-    const float px = (float)(bx * 8 + lx), py = (float)(by * 8 + ly), pz = (float)(bz * 8 + lz);
-    // owned vertices, interpolated from this voxel towards +x, +y, +z
-    const int own = cvi[(lz * 9 + ly) * 9 + lx];
-    int vid = vbase[0] + (own >> 3);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      if (!(own & (1 << a))) continue;
-      const float t = edge_t(s[0], s[far[a]]);
-      if (vid < vcap) {
-        float* V = verts + (size_t)vid * 3;
-        V[0] = (px + (a == 0 ? t : 0.0f)) * vs;
-        V[1] = (py + (a == 1 ? t : 0.0f)) * vs;
-        V[2] = (pz + (a == 2 ? t : 0.0f)) * vs;
-      }
-      ++vid;
+  const int lane = threadIdx.x & 63, stride = gridDim.x * kMcWaves;
+  McSoupLds& S = lds[threadIdx.x >> 6];
+  int blk = mc_block(), nb = -1;
+  McRow row = {};
+  if (blk < nblocks) {
+    row = mc_load_row(cases, blk);
+    if (lane < 8) nb = nbr[(size_t)blk * 8 + lane];
+  }
+  while (blk < nblocks) {
+    const int next = blk + stride;
+    const McRow cur = row;
+    const int cur_nb = nb;
+    const unsigned nt = mc_row_triangles(T, cur), slices = mc_slices(nt != 0u), layers = slices | slices << 1;
+    McSdf<VT> v;
+    if (slices) v.load((const typename VT::T*)m.voxels, blk, cur_nb, layers);
+    if (next < nblocks) {
+      row = mc_load_row(cases, next);
+      if (lane < 8) nb = nbr[(size_t)next * 8 + lane];
     }
-    for (int i = 0; i < nt && slot < tcap; ++i, ++slot) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int e = (int)((word >> (4 + 12 * i + 4 * k)) & 0xF);
-        const int x = lx + kOwner[e][0], y = ly + kOwner[e][1], z = lz + kOwner[e][2];
-        const int nbk = (x >> 3) | ((y >> 3) << 1) | ((z >> 3) << 2);
-        // the owner's block is present: every corner of an emitting cube is observed
-        const int oi = cvi[(z * 9 + y) * 9 + x];
-        tris[(size_t)slot * 3 + k] = vbase[nbk] + (oi >> 3) + __popc((oi & 7) & ((1 << kOwner[e][3]) - 1));
+    if (slices) {
+      const int sum = mc_nibble_sum(nt), end = (int)mc_scan((unsigned)sum);
+      const int total = __builtin_amdgcn_readlane(end, 63), first = offsets.tri(blk);
+      int bx, by, bz;
+      unpack_key(m.block_keys[blk], bx, by, bz);
+      __builtin_memcpy(&S.cases[lane * 8], cur.w, 16);
+      mc_list_triangles(S.tri, nt, end, 0);
+      v.stage(S.sdf);
+      for (int done = 0; done < total; done += kTriList) {
+        if (done > 0) mc_list_triangles(S.tri, nt, end, done);
+        mc_wave_sync();
+        mc_soup_flush<VT>(S, T, bx, by, bz, m.voxel_size, first + done, min(kTriList, total - done), tris, normals, cap);
+        mc_wave_sync();
       }
     }
+    blk = next;
+  }
+}
+
+// Emit, indexed form: the voxels' owned vertices, and their triangles as
+// indices of the owners' vertices.
+struct McIndexedLds {
+  uint32_t sdf[kMcCube];
+  uint16_t vi[kMcCube];    // the count pass's vertex info
+  uint16_t vert[kVertList];
+  uint16_t tri[kTriList];
+  alignas(16) uint16_t cases[512];
+  int vbase[8];            // first vertex of the block and its neighbours
+};
+// Owned vertices, interpolated from the voxel towards +x, +y, +z.
+template <class VT>
+__device__ inline void mc_vertex_flush(const McIndexedLds& S, int bx, int by, int bz, float vs, int first, int n,
+                                       float* verts, int vcap) {
+  for (int t = threadIdx.x & 63; t < n && first + t < vcap; t += 64) {
+    const int ent = S.vert[t], a = ent >> 9;
+    int x, y, z;
+    mc_voxel_xyz(ent & 511, x, y, z);
+    const int at = mc_cube_at(x, y, z);
+    const float f = edge_t(mc_sdf<VT>(S.sdf[at]), mc_sdf<VT>(S.sdf[at + (a == 0 ? 1 : a == 1 ? 9 : 81)]));
+    const float px = (float)(bx * 8 + x), py = (float)(by * 8 + y), pz = (float)(bz * 8 + z);
+    float* V = verts + (size_t)(first + t) * 3;
+    V[0] = (px + (a == 0 ? f : 0.0f)) * vs;
+    V[1] = (py + (a == 1 ? f : 0.0f)) * vs;
+    V[2] = (pz + (a == 2 ? f : 0.0f)) * vs;
+  }
+}
+__device__ inline void mc_index_flush(const McIndexedLds& S, const McTables& T, int first, int n, int* tris,
+                                      int tcap) {
+  for (int t = threadIdx.x & 63; t < n && first + t < tcap; t += 64) {
+    const unsigned ent = S.tri[t];
+    int x, y, z;
+    mc_voxel_xyz((int)(ent & 511u), x, y, z);
+    const unsigned edges = (unsigned)(T.word[S.cases[ent & 511u]] >> (4 + 12 * (ent >> 9)));
+    const int at = mc_cube_at(x, y, z);
+    const unsigned xyz = (unsigned)(x | (y << 4) | (z << 8));  // 4 bits a coordinate: 8 is the neighbour's 0
+    int id[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int e = (int)((edges >> (4 * k)) & 0xF);
+      const int ox = owner_x(e), oy = owner_y(e), oz = owner_z(e);
+      // the owner's block is present: every corner of an emitting cube is observed
+      const unsigned oi = S.vi[at + mc_cube_at(ox, oy, oz)];
+      const unsigned over = (xyz + (unsigned)(ox | (oy << 4) | (oz << 8))) & 0x888u;
+      id[k] = S.vbase[((over * 0x49u) >> 9) & 7u] + (int)(oi >> 3) + __popc(oi & ((1u << owner_axis(e)) - 1u));
+    }
+    int* P = tris + (size_t)(first + t) * 3;
+    P[0] = id[0]; P[1] = id[1]; P[2] = id[2];
+  }
+}
+template <class VT>
+__global__ void __launch_bounds__(kMcThreads) k_mc_emit_indexed(MapView m, int nblocks, McOffsets offsets,
+                                                                const int16_t* cases, const uint16_t* vinfo,
+                                                                float* verts, int vcap, int* tris, int tcap,
+                                                                const int* nbr) {
+  __shared__ McTables T;
+  __shared__ McIndexedLds lds[kMcWaves];
+  mc_fill_tables(T);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, stride = gridDim.x * kMcWaves;
+  McIndexedLds& S = lds[threadIdx.x >> 6];
+  int blk = mc_block(), nb = -1;
+  McRow row = {}, irow = {};
+  if (blk < nblocks) {
+    row = mc_load_row(cases, blk);
+    irow = mc_load_row(vinfo, blk);
+    if (lane < 8) nb = nbr[(size_t)blk * 8 + lane];
+  }
+  while (blk < nblocks) {
+    const int next = blk + stride;
+    const McRow cur = row, info = irow;
+    const int cur_nb = nb;
+    const unsigned nt = mc_row_triangles(T, cur);
+    unsigned edges = 0;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) edges |= (info.at(x) & 7u) << (4 * x);
+    const unsigned slices = mc_slices((nt | edges) != 0u), layers = slices | slices << 1;
+    McSdf<VT> v;
+    McHalo<uint16_t> ih;
+    int vb = 0;
+    if (slices) {
+      v.load((const typename VT::T*)m.voxels, blk, cur_nb, layers);
+      mc_load_halo(vinfo, cur_nb, layers, ih);
+      if (lane < 8 && cur_nb >= 0) vb = offsets.vert(cur_nb);
+    }
+    if (next < nblocks) {
+      row = mc_load_row(cases, next);
+      irow = mc_load_row(vinfo, next);
+      if (lane < 8) nb = nbr[(size_t)next * 8 + lane];
+    }
+    if (slices) {
+      const int sum = mc_nibble_sum(nt), end = (int)mc_scan((unsigned)sum), vfirst = (int)(info.at(0) >> 3);
+      const int ntri = __builtin_amdgcn_readlane(end, 63);
+      const int nvert = __builtin_amdgcn_readlane(vfirst + __popc(edges), 63);
+      const int tfirst = offsets.tri(blk), vbase = __builtin_amdgcn_readlane(vb, 0);
+      int bx, by, bz;
+      unpack_key(m.block_keys[blk], bx, by, bz);
+      __builtin_memcpy(&S.cases[lane * 8], cur.w, 16);
+      mc_list_triangles(S.tri, nt, end, 0);
+      mc_list_vertices(S.vert, edges, vfirst, 0);
+      if (lane < 8) S.vbase[lane] = vb;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) S.vi[mc_cube_at(x, lane & 7, lane >> 3)] = (uint16_t)info.at(x);
+      mc_stage_halo(ih, S.vi, [](uint16_t w) { return w; });
+      v.stage(S.sdf);
+      for (int done = 0; done < nvert; done += kVertList) {
+        if (done > 0) mc_list_vertices(S.vert, edges, vfirst, done);
+        mc_wave_sync();
+        mc_vertex_flush<VT>(S, bx, by, bz, m.voxel_size, vbase + done, min(kVertList, nvert - done), verts, vcap);
+        mc_wave_sync();
+      }
+      for (int done = 0; done < ntri; done += kTriList) {
+        if (done > 0) mc_list_triangles(S.tri, nt, end, done);
+        mc_wave_sync();
+        mc_index_flush(S, T, tfirst + done, min(kTriList, ntri - done), tris, tcap);
+        mc_wave_sync();
+      }
+    }
+    blk = next;
   }
 }
 
@@ -452,13 +692,15 @@ struct yas_mesher {
   float* tris;      // soup: 9 floats per triangle; indexed: 3 ints per triangle
   float* normals;   // soup: 9 floats per triangle; indexed: 3 floats per vertex
   int2* counts;     // per block {triangles, vertices}
-  int2* offsets;    // exclusive prefix of counts
-  int2* chunk;      // scan chunk totals
-  int2* total;      // {triangles, vertices}
+  int2* offsets;    // exclusive prefix of counts within a chunk
+  unsigned long long* chunk;  // exclusive prefix of 1024-block chunks, {triangles, vertices}
+  unsigned* done;   // the scan's finished workgroups
+  int2* total;      // {triangles, vertices}, host memory
   int16_t* cases;   // per voxel cube index
   uint16_t* vinfo;  // per voxel (local vertex prefix << 3 | owned edges)
   int* nbr;         // per block, pool indices of it and its 7 +x/+y/+z neighbours (-1 absent)
   int block_cap;
+  int cus;
   int num_blocks;
   int num_tri;
   int num_vert;
@@ -475,13 +717,14 @@ static int ensure_block_cap(yas_mesher* me, int n) {
   hipFree(me->vinfo);
   hipFree(me->nbr);
   me->nbr = nullptr;
-  me->counts = me->offsets = me->chunk = nullptr;
+  me->counts = me->offsets = nullptr;
+  me->chunk = nullptr;
   me->cases = nullptr;
   me->vinfo = nullptr;
   me->block_cap = 0;
   YAS_HIP(hipMalloc((void**)&me->counts, sizeof(int2) * n));
   YAS_HIP(hipMalloc((void**)&me->offsets, sizeof(int2) * n));
-  YAS_HIP(hipMalloc((void**)&me->chunk, sizeof(int2) * ((n + 1023) / 1024)));
+  YAS_HIP(hipMalloc((void**)&me->chunk, sizeof(*me->chunk) * ((n + kMcChunk - 1) / kMcChunk)));
   YAS_HIP(hipMalloc((void**)&me->cases, sizeof(int16_t) * 512 * (size_t)n));
   YAS_HIP(hipMalloc((void**)&me->vinfo, sizeof(uint16_t) * 512 * (size_t)n));
   YAS_HIP(hipMalloc((void**)&me->nbr, sizeof(int) * 8 * (size_t)n));
@@ -507,36 +750,41 @@ static int count_and_scan(yas_mesher* me, yas_map* map, MapView& v) {
   if ((rc = ensure_block_cap(me, n))) return rc;
   v = yas_map_view(map);
   hipStream_t s = me->ctx->stream;
+  const int groups = (n + kMcWaves - 1) / kMcWaves;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
-      hipLaunchKernelGGL(k_mc_count<VoxI16>, dim3(n), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
+      hipLaunchKernelGGL(k_mc_count<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
                          me->nbr);
       break;
     case YAS_VOXEL_F16_U16:
-      hipLaunchKernelGGL(k_mc_count<VoxF16>, dim3(n), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
+      hipLaunchKernelGGL(k_mc_count<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
                          me->nbr);
       break;
     default:
-      hipLaunchKernelGGL(k_mc_count<VoxF32>, dim3(n), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
+      hipLaunchKernelGGL(k_mc_count<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
                          me->nbr);
   }
   YAS_LAUNCH_CHECK();
-  const int nchunks = (n + 1023) / 1024;
-  hipLaunchKernelGGL(k_scan_local, dim3(nchunks), dim3(1024), 0, s, (const int2*)me->counts, me->offsets, n, me->chunk);
-  YAS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, s, me->chunk, nchunks, me->total);
-  YAS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_scan_add, dim3(nchunks), dim3(1024), 0, s, me->offsets, (const int2*)me->chunk, n);
+  hipLaunchKernelGGL(k_mc_scan, dim3((n + kMcChunk - 1) / kMcChunk), dim3(kMcChunk), 0, s, (const int2*)me->counts,
+                     me->offsets, n, me->chunk, me->total, me->done);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
 static int read_totals(yas_mesher* me) {
-  int2 t;
-  YAS_HIP(hipMemcpyAsync(&t, me->total, sizeof(int2), hipMemcpyDeviceToHost, me->ctx->stream));
   YAS_HIP(hipStreamSynchronize(me->ctx->stream));
-  me->num_tri = t.x;
-  me->num_vert = t.y;
+  me->num_tri = me->total->x;
+  me->num_vert = me->total->y;
+  return YAS_OK;
+}
+
+// Workgroups of an emission pass: as many as the device holds at once, each
+// wavefront taking blocks in turn.
+static int emit_groups(yas_mesher* me, const void* kernel, int* groups) {
+  int per = 0;
+  YAS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, kMcThreads, 0));
+  const int all = (me->num_blocks + kMcWaves - 1) / kMcWaves, fit = std::max(1, per) * me->cus;
+  *groups = std::min(all, fit);
   return YAS_OK;
 }
 
@@ -563,7 +811,10 @@ int yas_mesher_create(yas_ctx* ctx, int max_triangles, yas_mesher** out) {
   me->max_tri = max_triangles;
   hipError_t e = hipMalloc((void**)&me->tris, sizeof(float) * 9 * (size_t)max_triangles);
   if (e == hipSuccess) e = hipMalloc((void**)&me->normals, sizeof(float) * 9 * (size_t)max_triangles);
-  if (e == hipSuccess) e = hipMalloc((void**)&me->total, sizeof(int2));
+  if (e == hipSuccess) e = hipHostMalloc((void**)&me->total, sizeof(int2), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipMalloc((void**)&me->done, sizeof(unsigned));
+  if (e == hipSuccess) e = hipMemset(me->done, 0, sizeof(unsigned));
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&me->cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
   if (e != hipSuccess) {
     yas_set_error("yas_mesher_create: %s", hipGetErrorString(e));
     yas_mesher_destroy(me);
@@ -582,7 +833,8 @@ int yas_mesher_destroy(yas_mesher* me) {
   hipFree(me->counts);
   hipFree(me->offsets);
   hipFree(me->chunk);
-  hipFree(me->total);
+  hipHostFree(me->total);
+  hipFree(me->done);
   hipFree(me->cases);
   hipFree(me->vinfo);
   hipFree(me->nbr);
@@ -600,18 +852,23 @@ int yas_mesh_extract(yas_mesher* me, yas_map* map, int* num_triangles) {
   const int n = me->num_blocks;
   if (n == 0) return YAS_OK;
   hipStream_t s = me->ctx->stream;
+  const McOffsets off = {me->offsets, me->chunk};
+  int groups = 0;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
-      hipLaunchKernelGGL(k_mc_emit<VoxI16>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets, me->tris,
-                         me->normals, me->max_tri, (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxI16>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
       break;
     case YAS_VOXEL_F16_U16:
-      hipLaunchKernelGGL(k_mc_emit<VoxF16>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets, me->tris,
-                         me->normals, me->max_tri, (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxF16>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
       break;
     default:
-      hipLaunchKernelGGL(k_mc_emit<VoxF32>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets, me->tris,
-                         me->normals, me->max_tri, (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxF32>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
   }
   YAS_LAUNCH_CHECK();
   if ((rc = read_totals(me))) return rc;
@@ -637,21 +894,23 @@ int yas_mesh_extract_indexed(yas_mesher* me, yas_map* map, int* num_vertices, in
   // vertices in the normal buffer (capacity max_tri * 3 vertices)
   int* tri_idx = (int*)me->tris;
   const int vcap = me->max_tri * 3;
+  const McOffsets off = {me->offsets, me->chunk};
+  int groups = 0;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxI16>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri,
-                         (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxI16>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit_indexed<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
       break;
     case YAS_VOXEL_F16_U16:
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF16>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri,
-                         (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxF16>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
       break;
     default:
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF32>, dim3(n), dim3(kMcThreads), 0, s, v, n, (const int2*)me->offsets,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri,
-                         (const int*)me->nbr);
+      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxF32>, &groups))) return rc;
+      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
+                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
   }
   YAS_LAUNCH_CHECK();
   if ((rc = read_totals(me))) return rc;
@@ -711,10 +970,12 @@ int yas_mesher_blocks(yas_mesher* me, int32_t* keys, int32_t* first, int32_t* co
   }
   if (first || count) {
     std::vector<int2> o(n), c(n);
+    std::vector<unsigned long long> chunk((n + kMcChunk - 1) / kMcChunk);
+    YAS_HIP(hipMemcpy(chunk.data(), me->chunk, sizeof(chunk[0]) * chunk.size(), hipMemcpyDeviceToHost));
     YAS_HIP(hipMemcpy(o.data(), me->offsets, sizeof(int2) * n, hipMemcpyDeviceToHost));
     YAS_HIP(hipMemcpy(c.data(), me->counts, sizeof(int2) * n, hipMemcpyDeviceToHost));
     for (int i = 0; i < n; ++i) {
-      if (first) first[i] = o[i].x;
+      if (first) first[i] = o[i].x + (int)(unsigned)chunk[i >> kMcChunkShift];
       if (count) count[i] = c[i].x;
     }
   }

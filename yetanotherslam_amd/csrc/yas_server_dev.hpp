@@ -40,7 +40,7 @@ struct StreamDev {
   float* part_res;
   float* part_rgb;
   TrackState* st;
-  float angle_th, dist_th;
+  float sin2_max, dist2_max;
   // pose chain
   double* T_last;
   int* gate;

@@ -60,7 +60,7 @@ struct SolveArgs {
   int iters[kMaxLevels];
   int groups[kMaxLevels];  // workgroups of the level's passes
   int levels, mode;
-  float angle_th, dist_th;
+  float sin2_max, dist2_max;
   float wrh, wrb, wih, wib;
   TrackState* st;
   SolveXchg* x;
@@ -123,14 +123,15 @@ __device__ inline int wave_sum8_index(int lane) {
 }
 
 // wave_stats with the lanes' values exchanged by data-parallel moves instead
-// of LDS permutes: the same merges, the lower lane's values first.
+// of LDS permutes, the lower lane's values first: lane 0 gets the wavefront's
+// (the others' are of no use, which spares telling which lane is the lower).
 template <int M>
-__device__ inline void merge_xor(float& n, float& mean, float& m2) {
-  const float nb = lane_xor<M>(n), mb = lane_xor<M>(mean), qb = lane_xor<M>(m2);
-  const bool hi = (threadIdx.x & M) != 0;
-  float a = hi ? nb : n, b = hi ? mb : mean, c = hi ? qb : m2;
-  chan_merge(a, b, c, hi ? n : nb, hi ? mean : mb, hi ? m2 : qb);
-  n = a; mean = b; m2 = c;
+__device__ inline float lane_above(float v) {  // lane l + M's of the same 16; 0 past them
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + M, 0xF, 0xF, true));
+}
+template <int M>
+__device__ inline void merge_above(float& n, float& mean, float& m2) {
+  chan_merge(n, mean, m2, lane_above<M>(n), lane_above<M>(mean), lane_above<M>(m2));
 }
 // {v of the lower, v of the upper lane} of partners at 16 and 32.
 __device__ inline float2 both16(float v) {
@@ -144,10 +145,10 @@ __device__ inline float2 both32(float v) {
   return make_float2(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
 }
 __device__ inline void wave_stats_moves(float& n, float& mean, float& m2) {
-  merge_xor<1>(n, mean, m2);
-  merge_xor<2>(n, mean, m2);
-  merge_xor<4>(n, mean, m2);
-  merge_xor<8>(n, mean, m2);
+  merge_above<1>(n, mean, m2);
+  merge_above<2>(n, mean, m2);
+  merge_above<4>(n, mean, m2);
+  merge_above<8>(n, mean, m2);
   float2 a = both16(n), b = both16(mean), c = both16(m2);
   n = a.x; mean = b.x; m2 = c.x;
   chan_merge(n, mean, m2, a.y, b.y, c.y);
@@ -341,7 +342,7 @@ struct PixelTerms {
 };
 template <bool ICP, bool RGB>
 __device__ inline PixelTerms pixel_terms(const Level& L, const TrackBufs& B, const PoseF& T, const float* wp,
-                                         float angle_th, float dist_th, float winv, int k, bool in,
+                                         float sin2_max, float dist2_max, float winv, int k, bool in,
                                          const RefPixel& ref) {
   PixelTerms o;
   float vx = 0.f, vy = 0.f, vz = 1.f;
@@ -384,10 +385,10 @@ __device__ inline PixelTerms pixel_terms(const Level& L, const TrackBufs& B, con
     float nx, ny, nz;
     rot3(T, ref.p.nx, ref.p.ny, ref.p.nz, nx, ny, nz);
     const float dx = vx - c.vx, dy = vy - c.vy, dz = vz - c.vz;
-    const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+    const float dist2 = dx * dx + dy * dy + dz * dz;
     const float c0 = c.ny * nz - c.nz * ny, c1 = c.nz * nx - c.nx * nz, c2 = c.nx * ny - c.ny * nx;
-    const float ang = sqrtf(c0 * c0 + c1 * c1 + c2 * c2);
-    o.icp = hit && ang < angle_th && dist <= dist_th;
+    const float sin2 = c0 * c0 + c1 * c1 + c2 * c2;
+    o.icp = hit && sin2 <= sin2_max && dist2 <= dist2_max;
     const float row[7] = {nx, ny, nz, vy * nz - vz * ny, vz * nx - vx * nz, vx * ny - vy * nx,
                           nx * (c.vx - vx) + ny * (c.vy - vy) + nz * (c.vz - vz)};
 #pragma unroll
@@ -415,7 +416,7 @@ __device__ inline int solve_rounds(int N, int nb) { return (N + nb * 1024 - 1) /
 // workgroup waits for those.
 template <bool ICP, bool RGB>
 __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs& B, const PoseF& T, const float* wp,
-                                   float angle_th, float dist_th, int bx, int nb, RefPixel nxt, float (&acc)[8],
+                                   float sin2_max, float dist2_max, int bx, int nb, RefPixel nxt, float (&acc)[8],
                                    int& count) {
   const int tid = fresh_tid();
   const int t = tid & 255;
@@ -438,7 +439,7 @@ __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs&
       PixelTerms o = {};
       o.r = __builtin_nanf("");
       // a wavefront past the image (most of a last round) has no pixel to do
-      if (__any(in)) o = pixel_terms<ICP, RGB>(L, B, T, wp, angle_th, dist_th, winv, k, in, cur);
+      if (__any(in)) o = pixel_terms<ICP, RGB>(L, B, T, wp, sin2_max, dist2_max, winv, k, in, cur);
       const int slot = r * kSolveSlots + q;
       if (ICP) {
 #pragma unroll
@@ -715,7 +716,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
       int count = 0;
-      solve_pass1<ICP, RGB>(S, L, B, T, wu, a.angle_th, a.dist_th, bx, nb, ref, acc, count);
+      solve_pass1<ICP, RGB>(S, L, B, T, wu, a.sin2_max, a.dist2_max, bx, nb, ref, acc, count);
       if (RGB) {
         __syncthreads();
         if (threadIdx.x == 64) {
@@ -799,7 +800,7 @@ __device__ inline void solve_rescue(const SolveArgs& a) {
     for (int it = 0; it < a.iters[l]; ++it, ++used) {
       const int G = a.groups[l];
       for (int b = 0; b < G; ++b) {
-        pass1_at<ICP, RGB>(a.lv[l], a.tb[l], a.st, a.part_icp, a.part_res, a.angle_th, a.dist_th, b, G);
+        pass1_at<ICP, RGB>(a.lv[l], a.tb[l], a.st, a.part_icp, a.part_res, a.sin2_max, a.dist2_max, b, G);
         __syncthreads();
       }
       if (RGB)

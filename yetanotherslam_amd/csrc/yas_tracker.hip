@@ -87,8 +87,8 @@ __global__ void __launch_bounds__(256) k_vmap_to_depth(const float4* v, size_t s
 
 template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_pass1(Level L, TrackBufs B, const TrackState* st, float* part_icp,
-                                               float* part_res, float angle_th, float dist_th) {
-  pass1_at<ICP, RGB, true>(L, B, st, part_icp, part_res, angle_th, dist_th, blockIdx.x, gridDim.x);
+                                               float* part_res, float sin2_max, float dist2_max) {
+  pass1_at<ICP, RGB, true>(L, B, st, part_icp, part_res, sin2_max, dist2_max, blockIdx.x, gridDim.x);
 }
 __global__ void __launch_bounds__(256) k_pass2(Level L, TrackBufs B, TrackState* st, const float* part_res, int g1,
                                                float* part_rgb) {
@@ -107,8 +107,8 @@ __global__ void __launch_bounds__(256) k_update_into(const TrackState* st_in, Tr
 // Step of the previous linearisation, then pass 1 at the new pose.
 template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_step_pass1(Level L, TrackBufs B, StepArgs a, float* part_icp,
-                                                    float* part_res, float angle_th, float dist_th) {
-  pass1_at<ICP, RGB, true, true>(L, B, nullptr, part_icp, part_res, angle_th, dist_th, blockIdx.x, gridDim.x, &a);
+                                                    float* part_res, float sin2_max, float dist2_max) {
+  pass1_at<ICP, RGB, true, true>(L, B, nullptr, part_icp, part_res, sin2_max, dist2_max, blockIdx.x, gridDim.x, &a);
 }
 // The whole solve in one launch (yas_solve_dev.hpp).  1024 threads a
 // workgroup, so 128 registers a lane; one workgroup per CU.  Bound by the
@@ -160,7 +160,7 @@ struct yas_tracker {
   TrackState* host_st;
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
-  float angle_th, dist_th;
+  float sin2_max, dist2_max;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
   float* raw_image;  // intensity uploaded by the host-image setters
 };
@@ -224,13 +224,13 @@ static int launch_iteration(yas_tracker* t, int l, bool icp, bool rgb, bool do_s
   TrackBufs B = bufs(t, l);
   if (icp && rgb)
     hipLaunchKernelGGL((k_pass1<true, true>), dim3(G), dim3(256), 0, s, a, B, (const TrackState*)t->st, t->part_icp,
-                       t->part_res, t->angle_th, t->dist_th);
+                       t->part_res, t->sin2_max, t->dist2_max);
   else if (icp)
     hipLaunchKernelGGL((k_pass1<true, false>), dim3(G), dim3(256), 0, s, a, B, (const TrackState*)t->st, t->part_icp,
-                       t->part_res, t->angle_th, t->dist_th);
+                       t->part_res, t->sin2_max, t->dist2_max);
   else
     hipLaunchKernelGGL((k_pass1<false, true>), dim3(G), dim3(256), 0, s, a, B, (const TrackState*)t->st, t->part_icp,
-                       t->part_res, t->angle_th, t->dist_th);
+                       t->part_res, t->sin2_max, t->dist2_max);
   if (rgb)
     hipLaunchKernelGGL(k_pass2, dim3(G), dim3(256), 0, s, a, B, t->st, (const float*)t->part_res, G, t->part_rgb);
   hipLaunchKernelGGL(k_update, dim3(1), dim3(256), 0, s, t->st, (const float*)t->part_icp, icp ? G : 0,
@@ -263,25 +263,25 @@ static int solve_by_passes(yas_tracker* t) {
       if (i == 0) {
         if (icp && rgb)
           hipLaunchKernelGGL((k_pass1<true, true>), dim3(G), dim3(256), 0, s, lv, B, (const TrackState*)cur, pic,
-                             t->part_res, t->angle_th, t->dist_th);
+                             t->part_res, t->sin2_max, t->dist2_max);
         else if (icp)
           hipLaunchKernelGGL((k_pass1<true, false>), dim3(G), dim3(256), 0, s, lv, B, (const TrackState*)cur, pic,
-                             t->part_res, t->angle_th, t->dist_th);
+                             t->part_res, t->sin2_max, t->dist2_max);
         else
           hipLaunchKernelGGL((k_pass1<false, true>), dim3(G), dim3(256), 0, s, lv, B, (const TrackState*)cur, pic,
-                             t->part_res, t->angle_th, t->dist_th);
+                             t->part_res, t->sin2_max, t->dist2_max);
       } else {
         a.st_in = S[(i - 1) & 1];
         a.st_out = cur;
         if (icp && rgb)
           hipLaunchKernelGGL((k_step_pass1<true, true>), dim3(G), dim3(256), 0, s, lv, B, a, pic, t->part_res,
-                             t->angle_th, t->dist_th);
+                             t->sin2_max, t->dist2_max);
         else if (icp)
           hipLaunchKernelGGL((k_step_pass1<true, false>), dim3(G), dim3(256), 0, s, lv, B, a, pic, t->part_res,
-                             t->angle_th, t->dist_th);
+                             t->sin2_max, t->dist2_max);
         else
           hipLaunchKernelGGL((k_step_pass1<false, true>), dim3(G), dim3(256), 0, s, lv, B, a, pic, t->part_res,
-                             t->angle_th, t->dist_th);
+                             t->sin2_max, t->dist2_max);
       }
       if (rgb)
         hipLaunchKernelGGL(k_pass2, dim3(G), dim3(256), 0, s, lv, B, cur, (const float*)t->part_res, G, t->part_rgb);
@@ -374,8 +374,8 @@ int yas_tracker_solve_async(yas_tracker* t) {
     a.groups[l] = groups_for(t->lv[l]);
   }
   a.mode = t->P.mode;
-  a.angle_th = t->angle_th;
-  a.dist_th = t->dist_th;
+  a.sin2_max = t->sin2_max;
+  a.dist2_max = t->dist2_max;
   a.wrh = t->P.w_rgb_h; a.wrb = t->P.w_rgb_b; a.wih = t->P.w_icp_h; a.wib = t->P.w_icp_b;
   a.st = t->st;
   a.x = t->xchg;
@@ -426,8 +426,8 @@ int yas_tracker_fill(yas_tracker* t, StreamDev& d) {
   d.part_res = t->part_res;
   d.part_rgb = t->part_rgb;
   d.st = t->st;
-  d.angle_th = t->angle_th;
-  d.dist_th = t->dist_th;
+  d.sin2_max = t->sin2_max;
+  d.dist2_max = t->dist2_max;
   return YAS_OK;
 }
 const yas_tracker_params& yas_tracker_params_of(yas_tracker* t) { return t->P; }
@@ -465,6 +465,17 @@ int yas_rgb_to_gray_async(yas_ctx* ctx, const uint8_t* rgb, size_t sp, float* ds
   return YAS_OK;
 }
 
+// The largest float whose square root, rounded, is below `limit` (or equal to
+// it, `inclusive`): the passes compare squares with it instead of taking two
+// roots a pixel, with the same outcome.
+static float largest_square(float limit, bool inclusive) {
+  auto within = [&](float v) { return inclusive ? std::sqrt(v) <= limit : std::sqrt(v) < limit; };
+  float v = limit * limit;
+  while (within(std::nextafter(v, FLT_MAX))) v = std::nextafter(v, FLT_MAX);
+  while (!within(v)) v = std::nextafter(v, 0.0f);
+  return v;
+}
+
 extern "C" {
 
 int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_tracker_params* P, yas_tracker** out) {
@@ -483,8 +494,8 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   t->H = H;
   t->P = *P;
   // RGBDTracking.cu:432-433: sin(20 deg) computed in float, 1 cm.
-  t->angle_th = (float)std::sin(20.f * 3.14159254f / 180.f);
-  t->dist_th = 0.01f;
+  t->sin2_max = largest_square((float)std::sin(20.f * 3.14159254f / 180.f), false);
+  t->dist2_max = largest_square(0.01f, true);
   t->wait_ticks = kSolveWaitTicks;
   hipError_t e = hipSuccess;
   auto alloc = [&](void** p, size_t bytes) {

@@ -78,17 +78,31 @@ __device__ inline float block_sum32(float (&v)[32], float* lds /* [nwaves * 32] 
   return t;
 }
 
-// Chan et al.'s pairwise update of (count, mean, M2) statistics.
+// a / d and b / d, correctly rounded, by one reciprocal: the refinement that
+// the division expands to, without the scaling that it does first, which these
+// positive counts (and their products) are far from needing.
+__device__ inline float2 count_quotients(float a, float b, float d) {
+  const float r0 = __builtin_amdgcn_rcpf(d);
+  const float r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+  auto quotient = [&](float x) {
+    float q = x * r;
+    q = fmaf(fmaf(-d, q, x), r, q);
+    return fmaf(fmaf(-d, q, x), r, q);
+  };
+  return make_float2(quotient(a), quotient(b));
+}
+// Chan et al.'s pairwise update of (count, mean, M2) statistics.  By selects:
+// a merge is a link of the solve's serial chain, some 18 to an iteration, and
+// costs what it issues (with branches and two full divisions 40 instructions,
+// now 27).
 __device__ inline void chan_merge(float& n, float& mean, float& m2, float nb, float meanb, float m2b) {
   const float nn = n + nb;
-  if (nb == 0.0f) return;
-  if (n == 0.0f) {
-    n = nb; mean = meanb; m2 = m2b;
-    return;
-  }
+  const float2 w = count_quotients(nb, n * nb, nn);
   const float d = meanb - mean;
-  mean = mean + d * (nb / nn);
-  m2 = m2 + m2b + d * d * (n * nb / nn);
+  const float mm = mean + d * w.x, qq = m2 + m2b + d * d * w.y;
+  const bool none = n == 0.0f, keep = nb == 0.0f;
+  mean = keep ? mean : none ? meanb : mm;
+  m2 = keep ? m2 : none ? m2b : qq;
   n = nn;
 }
 
@@ -395,7 +409,7 @@ struct TrackBufs {
 // the current frame, gated at sin(20 deg) normal angle and 1 cm; on a match
 // the point-to-plane row [n, v x n, n.(v_c - v)] is accumulated.  Only
 // pixels with a vertex and a normal on both sides can match (IcpPoint).
-__device__ inline void icp_pixel(const Level& L, const TrackBufs& B, const PoseF& T, float angle_th, float dist_th,
+__device__ inline void icp_pixel(const Level& L, const TrackBufs& B, const PoseF& T, float sin2_max, float dist2_max,
                                  const IcpPoint& r, float (&acc)[32]) {
   if (!(r.vx == r.vx)) return;
   float vx, vy, vz;
@@ -408,10 +422,10 @@ __device__ inline void icp_pixel(const Level& L, const TrackBufs& B, const PoseF
   float nx, ny, nz;
   rot3(T, r.nx, r.ny, r.nz, nx, ny, nz);
   const float dx = vx - q.vx, dy = vy - q.vy, dz = vz - q.vz;
-  const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+  const float dist2 = dx * dx + dy * dy + dz * dz;
   const float c0 = q.ny * nz - q.nz * ny, c1 = q.nz * nx - q.nx * nz, c2 = q.nx * ny - q.ny * nx;
-  const float ang = sqrtf(c0 * c0 + c1 * c1 + c2 * c2);
-  if (!(ang < angle_th && dist <= dist_th)) return;  // a NaN distance (no current point) fails here
+  const float sin2 = c0 * c0 + c1 * c1 + c2 * c2;
+  if (!(sin2 <= sin2_max && dist2 <= dist2_max)) return;  // a NaN distance (no current point) fails here
   float row[7];
   row[0] = nx; row[1] = ny; row[2] = nz;
   row[3] = vy * nz - vz * ny;
@@ -539,7 +553,7 @@ __device__ __attribute__((always_inline)) inline void gn_update(const TrackState
 
 template <bool ICP, bool RGB, bool PREFETCH = false, bool STEP = false>
 __device__ inline void pass1_at(const Level& L, const TrackBufs& B, const TrackState* st, float* part_icp,
-                                float* part_res, float angle_th, float dist_th, int bx, int nb,
+                                float* part_res, float sin2_max, float dist2_max, int bx, int nb,
                                 const StepArgs* sa = nullptr) {
   __shared__ float pose[12];
   __shared__ float wp[12];
@@ -581,7 +595,7 @@ __device__ inline void pass1_at(const Level& L, const TrackBufs& B, const TrackS
     } else {
       cur = load_ref_pixel<ICP, RGB>(B, N, k);
     }
-    if (ICP) icp_pixel(L, B, T, angle_th, dist_th, cur.p, acc);
+    if (ICP) icp_pixel(L, B, T, sin2_max, dist2_max, cur.p, acc);
     if (RGB) rgb_pixel(L, B, wu, k, cur.iz, cur.inten, n, mean, m2);
   }
   if (ICP && RGB) {
@@ -945,7 +959,8 @@ __device__ inline void se3_exp_wave(const double* xi, double* w9, double* E) {
   } else {
     // A = sin / th, B = (1 - cos) / th2, C = (th - sin) / (th2 th): one
     // division, each quotient in a lane of its own
-    const double sn = sin(th), cs = cos(th);
+    double sn, cs;
+    sincos(th, &sn, &cs);
     const double num = lane == 0 ? sn : lane == 1 ? 1.0 - cs : th - sn;
     const double den = lane == 0 ? th : lane == 1 ? th2 : th2 * th;
     const double quo = num / den;

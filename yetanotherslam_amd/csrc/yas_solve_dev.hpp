@@ -189,9 +189,10 @@ __device__ inline bool wait_words(const void* base, P at, W want, unsigned epoch
     }
     const bool all = miss == 0;
     if (all) return true;
-    if ((looks & 15) == 0) {  // the clock is read at every 16th look
+    const unsigned every = ticks ? 31u : 0u;
+    if ((looks & every) == every) {  // the clock is read at every 32nd look
       const unsigned long long now = wall_clock64();
-      if (looks == 0) t0 = now;
+      if (looks == every) t0 = now;
       if (now - t0 >= ticks) return false;
     }
   }
@@ -220,10 +221,10 @@ struct SolveLds {
 // The products of the upper triangle of a 7-element row that quarter q sums
 // over slots first .. first + 3, in that order; 7 products each:
 //   q 0: row 0; q 1: row 1 and (6,6); q 2: rows 2 and 5; q 3: rows 3 and 4
-template <bool WEIGHTED>
-__device__ inline void add_products(const SolveLds& S, int first, int q, int t, float (&acc)[8]) {
+template <bool WEIGHTED, int N>
+__device__ inline void add_slots(const SolveLds& S, int first, int q, int t, float (&acc)[8]) {
 #pragma unroll
-  for (int s = first; s < first + kSolveSlots; ++s) {
+  for (int s = first; s < first + N; ++s) {
     const float w = WEIGHTED ? S.row[s][7][t] : 1.0f;
     // wt * row[i] * row[j] is summed as (wt * row[i]) * row[j]
     auto lead = [&](float x) { return WEIGHTED ? w * x : x; };
@@ -260,6 +261,15 @@ __device__ inline void add_products(const SolveLds& S, int first, int q, int t, 
       acc[6] += c * x6;
     }
   }
+}
+// Slots 0 .. n - 1 of a batch.
+template <bool WEIGHTED>
+__device__ inline void add_products(const SolveLds& S, int n, int q, int t, float (&acc)[8]) {
+  int s = 0;
+#pragma unroll 1
+  for (; s + kSolveSlots <= n; s += kSolveSlots) add_slots<WEIGHTED, kSolveSlots>(S, s, q, t, acc);
+#pragma unroll 1
+  for (; s < n; ++s) add_slots<WEIGHTED, 1>(S, s, q, t, acc);
 }
 // Where quarter q's v-th product lies in the packed 28.
 __device__ inline int product_index(int q, int v) {
@@ -407,7 +417,15 @@ __device__ inline PixelTerms pixel_terms(const Level& L, const TrackBufs& B, con
   return o;
 }
 
-__device__ inline int solve_rounds(int N, int nb) { return (N + nb * 1024 - 1) / (nb * 1024); }
+// Pixel slots of a workgroup's thread t < 256 (a last one may be past the
+// image), worked on in rounds of kSolveSlots, and of those the batch's from
+// round r0.  Slots past the count are left out: their zero rows add +0.
+__device__ inline int solve_slots(int N, int nb) { return (N + nb * 256 - 1) / (nb * 256); }
+__device__ inline int solve_rounds(int slots) { return (slots + kSolveSlots - 1) / kSolveSlots; }
+__device__ inline int batch_slots(int slots, int r0) {
+  const int n = slots - r0 * kSolveSlots;
+  return n < kSolveBatch * kSolveSlots ? n : kSolveBatch * kSolveSlots;
+}
 
 // Pass 1 of workgroup bx of nb: the rows of the last batch of slots in LDS
 // (the ICP products of the batches before it are in `acc`), the residuals'
@@ -422,19 +440,19 @@ __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs&
   const int t = tid & 255;
   const int q = __builtin_amdgcn_readfirstlane(tid >> 8);
   const int N = L.w * L.h, stride = nb * 256;
-  const int rounds = solve_rounds(N, nb);
+  const int slots = solve_slots(N, nb), rounds = solve_rounds(slots);
   const float winv = 1.0f / (float)L.w;
   float n = 0.0f, mean = 0.0f, m2 = 0.0f;
   int k = bx * 256 + t + q * stride;
 #pragma unroll 1
   for (int r0 = 0; r0 < rounds; r0 += kSolveBatch) {
     if (r0 > 0) __syncthreads();  // the last batch's rows have been read
-    const int nr = rounds - r0 < kSolveBatch ? rounds - r0 : kSolveBatch;
+    const int ns = batch_slots(slots, r0);
 #pragma unroll 1
-    for (int r = 0; r < nr; ++r, k += kSolveSlots * stride) {
+    for (int r = 0; r * kSolveSlots + q < ns; ++r, k += kSolveSlots * stride) {
       const RefPixel cur = nxt;
       const int kn = k + kSolveSlots * stride;
-      if (r0 + r + 1 < rounds) nxt = solve_ref_pixel<ICP, RGB>(B, N, kn < N ? kn : N - 1);
+      if ((r0 + r + 1) * kSolveSlots + q < slots) nxt = solve_ref_pixel<ICP, RGB>(B, N, kn < N ? kn : N - 1);
       const bool in = k < N;
       PixelTerms o = {};
       o.r = __builtin_nanf("");
@@ -459,7 +477,7 @@ __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs&
     __syncthreads();
     if (RGB && q == 3) {
 #pragma unroll 4
-      for (int s = 0; s < nr * kSolveSlots; ++s) {
+      for (int s = 0; s < ns; ++s) {
         const float e = S.r[s][t];
         if (e == e) {
           n += 1.0f;
@@ -469,9 +487,7 @@ __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs&
         }
       }
     }
-    if (ICP && r0 + kSolveBatch < rounds)
-#pragma unroll 1
-      for (int r = 0; r < nr; ++r) add_products<false>(S, r * kSolveSlots, q, t, acc);
+    if (ICP && r0 + kSolveBatch < rounds) add_products<false>(S, ns, q, t, acc);
   }
   if (RGB && q == 3) {
     wave_stats_moves(n, mean, m2);
@@ -482,12 +498,11 @@ __device__ inline void solve_pass1(SolveLds& S, const Level& L, const TrackBufs&
   }
 }
 // The ICP products of pass 1's last batch, then S.part / S.count.
-__device__ inline void solve_pass1_end(SolveLds& S, int rounds, float (&acc)[8], int count) {
+__device__ inline void solve_pass1_end(SolveLds& S, int slots, float (&acc)[8], int count) {
   const int tid = fresh_tid();
   const int q = __builtin_amdgcn_readfirstlane(tid >> 8);
-  const int nr = rounds - (rounds - 1) / kSolveBatch * kSolveBatch;
-#pragma unroll 1
-  for (int r = 0; r < nr; ++r) add_products<false>(S, r * kSolveSlots, q, tid & 255, acc);
+  const int last = (solve_rounds(slots) - 1) / kSolveBatch * kSolveBatch;  // the last batch's first round
+  add_products<false>(S, batch_slots(slots, last), q, tid & 255, acc);
   put_sums(S, q, acc, count);
 }
 
@@ -498,7 +513,7 @@ __device__ inline void solve_pass2(SolveLds& S, const Level& L, const TrackBufs&
   const int t = tid & 255;
   const int q = __builtin_amdgcn_readfirstlane(tid >> 8);
   const int N = L.w * L.h, stride = nb * 256;
-  const int rounds = solve_rounds(N, nb);
+  const int slots = solve_slots(N, nb), rounds = solve_rounds(slots);
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
@@ -507,9 +522,9 @@ __device__ inline void solve_pass2(SolveLds& S, const Level& L, const TrackBufs&
 #pragma unroll 1
   for (int r0 = 0; r0 < rounds; r0 += kSolveBatch) {
     if (r0 > 0) __syncthreads();  // the last batch's rows have been read
-    const int nr = rounds - r0 < kSolveBatch ? rounds - r0 : kSolveBatch;
+    const int ns = batch_slots(slots, r0);
 #pragma unroll 1
-    for (int r = 0; r < nr; ++r, k += kSolveSlots * stride) {
+    for (int r = 0; r * kSolveSlots + q < ns; ++r, k += kSolveSlots * stride) {
       float e, gx, gy, px, py, pz;
       if (r0 == 0) {
         const float(&kp)[6][kSolveThreads] = S.kept[r];
@@ -543,8 +558,7 @@ __device__ inline void solve_pass2(SolveLds& S, const Level& L, const TrackBufs&
       count += __popcll(__ballot(has));
     }
     __syncthreads();
-#pragma unroll 1
-    for (int r = 0; r < nr; ++r) add_products<true>(S, r * kSolveSlots, q, t, acc);
+    add_products<true>(S, ns, q, t, acc);
   }
   put_sums(S, q, acc, count);
 }
@@ -729,7 +743,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         }
       }
       if (ICP) {
-        solve_pass1_end(S, solve_rounds(L.w * L.h, nb), acc, count);
+        solve_pass1_end(S, solve_slots(L.w * L.h, nb), acc, count);
         __syncthreads();
         if (threadIdx.x < 29) put_word(&a.x->icp[bx][threadIdx.x], row_total(S, threadIdx.x), epoch);
       }

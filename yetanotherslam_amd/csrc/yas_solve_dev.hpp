@@ -652,14 +652,16 @@ __device__ inline SolveLds& solve_lds() {
   return S;
 }
 
-// Workgroup 0's step (wavefront 0), a function of its own: the pixel loops'
-// registers and the double-precision solve's do not fit together, and inlined
-// the solve spilled (13000 against 8300 cycles).
-__device__ __attribute__((noinline)) void solve_step(int gi, int gr, int mode, int first_of_level, int record,
-                                                     float wrh, float wrb, float wih, float wib) {
+// Workgroup 0's step (wavefront 0) into S.est, a function of its own: the
+// pixel loops' registers and the double-precision solve's do not fit together,
+// and inlined the solve spilled (13000 against 8300 cycles).
+__device__ __attribute__((noinline)) GnStep solve_step(int mode, float wrh, float wrb, float wih, float wib) {
   SolveLds& S = solve_lds();
-  gn_step_wave0(S.sums, S.est, S.s.good, S.s.last_err, &S.s, S.est, gi, gr, mode, first_of_level, 1, record, wrh, wrb,
-                wih, wib, S.H, S.b, S.xs, S.W, S.E);
+  GnStep g = {false, false, 0.0f};
+  double t = 0.0;
+  if (S.s.good) g = gn_step_pose(S.sums, S.est, mode, wrh, wrb, wih, wib, S.H, S.b, S.xs, S.W, S.E, t);
+  if (g.moved && (threadIdx.x & 63) < 16) S.est[threadIdx.x & 63] = t;
+  return g;
 }
 
 template <bool ICP, bool RGB>
@@ -678,6 +680,8 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
     const int iters = a.iters[l];
     if (iters <= 0) continue;
     const int nb = a.groups[l];
+    int below = l - 1;  // the next level with iterations
+    while (below >= 0 && a.iters[below] <= 0) --below;
     if (bx >= nb) {  // no work at this level: its poses are not read here
       epoch += iters;
       fresh = false;
@@ -770,15 +774,10 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         }
         wave_lds_sync();
       }
-      int nl = it + 1 < iters ? l : l - 1;
-      while (nl >= 0 && a.iters[nl] <= 0) --nl;
-      if (threadIdx.x < 29) {
-        if (ICP) S.s.sums_icp[threadIdx.x] = S.sums[0][threadIdx.x];
-        if (RGB) S.s.sums_rgb[threadIdx.x] = S.sums[1][threadIdx.x];
-      }
       if (threadIdx.x < 64) {
-        solve_step(ICP ? nb : 0, RGB ? nb : 0, a.mode, it == 0 ? 1 : 0, l == 0 ? 1 : 0, a.wrh, a.wrb, a.wih, a.wib);
+        const GnStep g = solve_step(a.mode, a.wrh, a.wrb, a.wih, a.wib);
         wave_lds_sync();
+        const int nl = it + 1 < iters ? l : below;
         if (nl >= 0) {
           load_pose_f(S.est, S.pose);
           if (RGB) load_warp(S.est, a.lv[nl].Kinv, S.warp);
@@ -787,6 +786,13 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
           if (w < 12) put_word(&a.x->pose[w], S.pose[w], epoch);
           else if (RGB && w < 24) put_word(&a.x->pose[w], S.warp[w - 12], epoch);
         }
+        // the state, while the pose is on its way
+        if (threadIdx.x < 29) {
+          if (ICP) S.s.sums_icp[threadIdx.x] = S.sums[0][threadIdx.x];
+          if (RGB) S.s.sums_rgb[threadIdx.x] = S.sums[1][threadIdx.x];
+        }
+        gn_step_record(&S.s, S.sums, S.s.last_err, ICP ? nb : 0, RGB ? nb : 0, it == 0, l == 0, g,
+                       S.est[threadIdx.x & 15]);
       }
       __syncthreads();
     }

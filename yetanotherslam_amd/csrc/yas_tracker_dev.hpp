@@ -836,29 +836,12 @@ __device__ inline double lane_value(double v, int src) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// ldlt_solve6_presorted run by a whole wavefront (all 64 lanes active,
-// every lane gets x): lane r < 6 holds row r of the permuted matrix, and at
-// factorisation step k the rows r >= k update their column k at once, each
-// by the same operations in the same order as the serial loops (the
-// products temp[j] = D_j L_kj from lane j's diagonal and lane k's row, the
-// sums from j = 0 up, the division by D_k), so x has the same bits.  The
-// pivots and the back substitution stay serial (the latter's sums run over
-// j ascending, which needs the finished y_j in that order); lanes 6..63
-// mirror row 5.  H and b are read from LDS; `scratch` (6 doubles, LDS)
-// undoes the permutation.
-__device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* scratch, double (&x)[6]) {
+// The pivot order p of the diagonal magnitudes d (changed), by exchanges as
+// the factorisation makes them; `stop` where there is no pivot at all.
+__device__ inline void ldlt_pivots(float (&d)[6], int (&p)[6], bool& stop) {
   constexpr int n = 6;
-  const int lane = threadIdx.x & 63;
-  const int r = lane < n ? lane : n - 1;
-  // the pivots, from the diagonal as floats (the same order as the doubles')
-  float d[n];
-  int p[n];
 #pragma unroll
-  for (int i = 0; i < n; ++i) {
-    d[i] = fabsf(H[i * n + i]);
-    p[i] = i;
-  }
-  bool stop = false;
+  for (int i = 0; i < n; ++i) p[i] = i;
 #pragma unroll
   for (int k = 0; k < n - 1; ++k) {
     int big = k;
@@ -869,7 +852,7 @@ __device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* 
       bv = gt ? d[i] : bv;
       big = gt ? i : big;
     }
-    if (k == 0) stop = !(bv > 0.0f);  // no pivot at all
+    if (k == 0) stop = !(bv > 0.0f);
     const float dk = d[k];
     const int pk = p[k];
 #pragma unroll
@@ -884,9 +867,47 @@ __device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* 
 #pragma unroll
     for (int i = 0; i < n; ++i) p[i] = i;
   }
-  int pr = p[0];
+}
+
+// ldlt_solve6_presorted run by a whole wavefront (all 64 lanes active,
+// every lane gets x): lane r < 6 holds row r of the permuted matrix, and at
+// factorisation step k the rows r >= k update their column k at once, each
+// by the same operations in the same order as the serial loops (the
+// products temp[j] = D_j L_kj from lane j's diagonal and lane k's row, the
+// sums from j = 0 up, the division by D_k), so x has the same bits.  The
+// pivots and the back substitution stay serial (the latter's sums run over
+// j ascending, which needs the finished y_j in that order); lanes 6..63
+// mirror row 5.  H and b are read from LDS; `scratch` (6 doubles, LDS)
+// undoes the permutation.
+__device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* scratch, double (&x)[6]) {
+  constexpr int n = 6;
+  const int lane = threadIdx.x & 63;
+  const int r = lane < n ? lane : n - 1;
+  // the pivots, from the diagonal as floats (the same order as the doubles'):
+  // where the magnitudes differ, row r's place is the number of larger ones
+  float d[n];
+  int p[n];
+  const float mine = fabsf(H[r * n + r]);
+  int place = 0, equal = 0;
 #pragma unroll
-  for (int j = 1; j < n; ++j) pr = r == j ? p[j] : pr;
+  for (int i = 0; i < n; ++i) {
+    d[i] = fabsf(H[i * n + i]);
+    place += d[i] > mine ? 1 : 0;
+    equal += d[i] == mine ? 1 : 0;
+  }
+  bool stop = false;
+  int pr;
+  if (__ballot(equal != 1) == 0ull) {
+    pr = __builtin_amdgcn_ds_permute(place << 2, r);  // lane `place` gets r
+#pragma unroll
+    for (int i = 0; i < n; ++i) p[i] = __builtin_amdgcn_readlane(pr, i);
+    pr = lane < n ? pr : p[n - 1];
+  } else {  // ties or NaN: the order depends on the exchanges
+    ldlt_pivots(d, p, stop);
+    pr = p[0];
+#pragma unroll
+    for (int j = 1; j < n; ++j) pr = r == j ? p[j] : pr;
+  }
   double a[n];  // row r: a[j] = A(r, j) for j <= r
 #pragma unroll
   for (int j = 0; j < n; ++j) a[j] = (double)H[pr * n + p[j]];
@@ -933,6 +954,28 @@ __device__ inline void ldlt_solve6_wave(const float* H, const float* b, double* 
   for (int i = 0; i < n; ++i) x[i] = scratch[i];
 }
 
+// A = sin th / th, B = (1 - cos th) / th2 and C = (th - sin th) / (th2 th) of
+// a rotation by th, th2 = th th below kExpSeriesMax (half a radian, far above
+// a tracker's step), by their power series: the first term left out is below
+// 1e-19 of the sum.  Some 70 instructions of the solve's serial chain where
+// root, sine, cosine and division are 250, and nearer to the true values,
+// which the differences 1 - cos and th - sin lose at small angles.
+constexpr double kExpSeriesMax = 0.25;
+__host__ __device__ inline void exp_series(double th2, double& A, double& B, double& C) {
+  const double t = -th2;
+  A = B = C = 0.0;
+  // 1 / (2 k + 1)!, 1 / (2 k + 2)!, 1 / (2 k + 3)! for k = 7 .. 0
+  constexpr double f[18] = {1.0, 1.0, 2.0, 6.0, 24.0, 120.0, 720.0, 5040.0, 40320.0, 362880.0, 3628800.0, 39916800.0,
+                            479001600.0, 6227020800.0, 87178291200.0, 1307674368000.0, 20922789888000.0,
+                            355687428096000.0};
+#pragma unroll
+  for (int k = 7; k >= 0; --k) {
+    A = fma(A, t, 1.0 / f[2 * k + 1]);
+    B = fma(B, t, 1.0 / f[2 * k + 2]);
+    C = fma(C, t, 1.0 / f[2 * k + 3]);
+  }
+}
+
 // SE(3) exponential, twist (rho, omega), Rodrigues' formula, by a whole
 // wavefront: lane 4 i + j < 16 writes element (i, j) of the 4x4 result to E
 // (LDS).  Lanes 0..8 first leave W = [omega]x in `w9` (LDS) and the result's
@@ -949,16 +992,14 @@ __device__ inline void se3_exp_wave(const double* xi, double* w9, double* E) {
     const bool neg = (i == 0 && j == 1) || (i == 1 && j == 2) || (i == 2 && j == 0);
     w9[lane] = i == j ? 0.0 : neg ? -v : v;
   }
-  double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
-  double th = sqrt(th2);
+  const double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
   double A, B, C;
-  if (th < 1e-8) {
-    A = 1.0 - th2 / 6.0;
-    B = 0.5 - th2 / 24.0;
-    C = 1.0 / 6.0 - th2 / 120.0;
+  if (th2 < kExpSeriesMax) {
+    exp_series(th2, A, B, C);
   } else {
     // A = sin / th, B = (1 - cos) / th2, C = (th - sin) / (th2 th): one
     // division, each quotient in a lane of its own
+    const double th = sqrt(th2);
     double sn, cs;
     sincos(th, &sn, &cs);
     const double num = lane == 0 ? sn : lane == 1 ? 1.0 - cs : th - sn;
@@ -1003,32 +1044,24 @@ __device__ inline void unpack29(const float* s, float* H, float* b) {
     }
 }
 
-// Wavefront 0's part of gn_update (all 64 lanes, which leave together):
-// inlier counts and, when do_step and the state is good, the step from the
-// pose s_est.  Writes the state's fields to st and the stepped pose to
-// est_out (each when not null).  Each value is formed by the operations of
-// the serial form, in its order: H and b one element per lane
-// (RankUpdateHessian's packing, the RGB term weighted first), the solve by
-// ldlt_solve6_wave, the exponential by se3_exp_wave, and E * est one element
-// per lane for lanes 0..15.  lds_H (36), lds_b (6), lds_x (6), lds_W (9) and
+// What a Gauss-Newton step did.
+struct GnStep {
+  bool moved, bad;  // the pose was changed; the system had no solution
+  float err;
+};
+// One step of a wavefront (all 64 lanes) from the pose s_est: element `lane`
+// of the new pose for lanes 0..15 when it moved (in `t`).  Each value is
+// formed by the operations of the serial form, in its order: H and b one
+// element per lane (RankUpdateHessian's packing, the RGB term weighted first),
+// the solve by ldlt_solve6_wave, the exponential by se3_exp_wave, and E * est
+// one element per lane.  lds_H (36), lds_b (6), lds_x (6), lds_W (9) and
 // lds_E (16) are LDS.
-__device__ __attribute__((always_inline)) inline void gn_step_wave0(const float (*sums)[32], const double* s_est,
-                                                                    int s_good, float s_last_err, TrackState* st,
-                                                                    double* est_out, int gi, int gr, int mode,
-                                                                    int first_of_level, int do_step, int record,
-                                                                    float wrh, float wrb, float wih, float wib,
-                                                                    float* lds_H, float* lds_b, double* lds_x,
-                                                                    double* lds_W, double* lds_E) {
+__device__ __attribute__((always_inline)) inline GnStep gn_step_pose(const float (*sums)[32], const double* s_est,
+                                                                     int mode, float wrh, float wrb, float wih,
+                                                                     float wib, float* lds_H, float* lds_b,
+                                                                     double* lds_x, double* lds_W, double* lds_E,
+                                                                     double& t) {
   const int lane = threadIdx.x & 63;
-  if (st && lane == 0 && record && gi) st->icp_inliers = (int)sums[0][28];
-  if (st && lane == 0 && record && gr) st->rgb_inliers = (int)sums[1][28];
-  if (!do_step) return;
-  float last_err = s_last_err;
-  if (first_of_level) {
-    last_err = FLT_MAX;
-    if (st && lane == 0) st->last_err = FLT_MAX;
-  }
-  if (!s_good) return;
   if (lane < 42) {
     // element (i, j), i <= j, of the packed upper rows [H | b] (7 - i entries in row i)
     const bool isb = lane >= 36;
@@ -1054,26 +1087,59 @@ __device__ __attribute__((always_inline)) inline void gn_step_wave0(const float 
     nres = sums[1][28];
   }
   if (mode != YAS_TRACK_RGB) rsum = sums[0][27];
-  const float err = sqrtf(rsum) / (nres + 6.0f);
+  GnStep g = {false, false, sqrtf(rsum) / (nres + 6.0f)};
   wave_lds_sync();
   double xi[6];
   ldlt_solve6_wave(lds_H, lds_b, lds_x, xi);
   if (isnan(xi[0])) {
-    if (st && lane == 0) st->good = 0;
-    return;
+    g.bad = true;
+    return g;
   }
   se3_exp_wave(xi, lds_W, lds_E);
   if (lane < 16) {
     const int i = lane >> 2, j = lane & 3;
-    const double t = lds_E[4 * i] * s_est[j] + lds_E[4 * i + 1] * s_est[4 + j] + lds_E[4 * i + 2] * s_est[8 + j] +
-                     lds_E[4 * i + 3] * s_est[12 + j];
-    if (est_out) est_out[lane] = t;
-    if (st) {
-      st->est[lane] = t;
-      if (err < last_err) st->last_ok[lane] = t;
-    }
+    t = lds_E[4 * i] * s_est[j] + lds_E[4 * i + 1] * s_est[4 + j] + lds_E[4 * i + 2] * s_est[8 + j] +
+        lds_E[4 * i + 3] * s_est[12 + j];
   }
-  if (st && lane == 0 && err < last_err) st->last_err = err;
+  g.moved = true;
+  return g;
+}
+// The state after a linearisation and step g (t as gn_step_pose left it):
+// inlier counts, pose, and where the error fell, the pose to keep.
+__device__ inline void gn_step_record(TrackState* st, const float (*sums)[32], float last_err, int gi, int gr,
+                                      int first_of_level, int record, const GnStep& g, double t) {
+  const int lane = threadIdx.x & 63;
+  if (first_of_level) last_err = FLT_MAX;
+  if (g.moved && lane < 16) {
+    st->est[lane] = t;
+    if (g.err < last_err) st->last_ok[lane] = t;
+  }
+  if (lane == 0) {
+    if (record && gi) st->icp_inliers = (int)sums[0][28];
+    if (record && gr) st->rgb_inliers = (int)sums[1][28];
+    if (first_of_level) st->last_err = FLT_MAX;
+    if (g.bad) st->good = 0;
+    if (g.moved && g.err < last_err) st->last_err = g.err;
+  }
+}
+
+// Wavefront 0's part of gn_update (all 64 lanes, which leave together):
+// inlier counts and, when do_step and the state is good, the step from the
+// pose s_est.  Writes the state's fields to st and the stepped pose to
+// est_out (each when not null).
+__device__ __attribute__((always_inline)) inline void gn_step_wave0(const float (*sums)[32], const double* s_est,
+                                                                    int s_good, float s_last_err, TrackState* st,
+                                                                    double* est_out, int gi, int gr, int mode,
+                                                                    int first_of_level, int do_step, int record,
+                                                                    float wrh, float wrb, float wih, float wib,
+                                                                    float* lds_H, float* lds_b, double* lds_x,
+                                                                    double* lds_W, double* lds_E) {
+  GnStep g = {false, false, 0.0f};
+  double t = 0.0;
+  if (do_step && s_good)
+    g = gn_step_pose(sums, s_est, mode, wrh, wrb, wih, wib, lds_H, lds_b, lds_x, lds_W, lds_E, t);
+  if (est_out && g.moved && (threadIdx.x & 63) < 16) est_out[threadIdx.x & 63] = t;
+  if (st) gn_step_record(st, sums, s_last_err, gi, gr, do_step && first_of_level, record, g, t);
 }
 
 // Fold the partial rows of one linearisation and, when `do_step`, take one

@@ -200,11 +200,11 @@ __device__ inline bool wait_words(const void* base, P at, W want, unsigned epoch
 
 // ------------------------------------------------------------------ LDS
 // Rows of a batch of slots, [slot][element][thread]; element 7 is the weight
-// (pass 2), `r` the residual of each slot (pass 1).
+// (pass 2), `r` the residual of each slot (pass 1).  The small arrays lie
+// first: an LDS instruction's offset reaches 64 KB, and an array beyond that
+// takes a register for each of its addresses, which the compiler then keeps,
+// and spills, over the whole solve.
 struct SolveLds {
-  float row[kSolveBatch * kSolveSlots][8][256];
-  float r[kSolveBatch * kSolveSlots][256];
-  float kept[kSolveBatch][6][kSolveThreads];  // residual, gradients and warped point, for pass 2
   float part[29][4];                         // a row's wavefront sums
   int count[16];                             // matches by wavefront
   float stats[4][3];
@@ -214,8 +214,12 @@ struct SolveLds {
   double est[16];
   float H[36], b[6];
   double xs[6], W[9], E[16];
+  double Kinv[2][9];  // inverse intrinsics of this level and of the next one with iterations
   TrackState s;  // workgroup 0's running state
   int lost;      // a wait ran out
+  float r[kSolveBatch * kSolveSlots][256];
+  float kept[kSolveBatch][6][kSolveThreads];  // residual, gradients and warped point, for pass 2
+  float row[kSolveBatch * kSolveSlots][8][256];
 };
 
 // The products of the upper triangle of a 7-element row that quarter q sums
@@ -654,7 +658,7 @@ __device__ inline SolveLds& solve_lds() {
 
 // Workgroup 0's step (wavefront 0) into S.est, a function of its own: the
 // pixel loops' registers and the double-precision solve's do not fit together,
-// and inlined the solve spilled (13000 against 8300 cycles).
+// and inlined the solve spilled (RGB-D, 640x480, with its inputs: 347 us against 320 us).
 __device__ __attribute__((noinline)) GnStep solve_step(int mode, float wrh, float wrb, float wih, float wib) {
   SolveLds& S = solve_lds();
   GnStep g = {false, false, 0.0f};
@@ -662,6 +666,15 @@ __device__ __attribute__((noinline)) GnStep solve_step(int mode, float wrh, floa
   if (S.s.good) g = gn_step_pose(S.sums, S.est, mode, wrh, wrb, wih, wib, S.H, S.b, S.xs, S.W, S.E, t);
   if (g.moved && (threadIdx.x & 63) < 16) S.est[threadIdx.x & 63] = t;
   return g;
+}
+
+// load_warp with the inverse intrinsics' matrix in LDS.
+__device__ inline void solve_load_warp(const double* T, const double* Ki, float* out) {
+  if (threadIdx.x >= 16 && threadIdx.x < 28) {
+    const int q = threadIdx.x - 16, i = q / 4, j = q % 4;
+    if (j < 3) out[3 * i + j] = (float)(T[4 * i] * Ki[j] + T[4 * i + 1] * Ki[3 + j] + T[4 * i + 2] * Ki[6 + j]);
+    else out[9 + i] = (float)T[4 * i + 3];
+  }
 }
 
 template <bool ICP, bool RGB>
@@ -682,6 +695,11 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
     const int nb = a.groups[l];
     int below = l - 1;  // the next level with iterations
     while (below >= 0 && a.iters[below] <= 0) --below;
+    if (RGB && bx == 0 && threadIdx.x < 18) {  // read after the barriers of an iteration
+      const int m = threadIdx.x < 9 ? 0 : 1, e = threadIdx.x - 9 * m;
+      const double* K = a.lv[m == 0 || below < 0 ? l : below].Kinv;
+      S.Kinv[m][e] = e == 0 ? K[0] : e == 2 ? K[2] : e == 4 ? K[1] : e == 5 ? K[3] : e == 8 ? 1.0 : 0.0;
+    }
     if (bx >= nb) {  // no work at this level: its poses are not read here
       epoch += iters;
       fresh = false;
@@ -780,7 +798,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         const int nl = it + 1 < iters ? l : below;
         if (nl >= 0) {
           load_pose_f(S.est, S.pose);
-          if (RGB) load_warp(S.est, a.lv[nl].Kinv, S.warp);
+          if (RGB) solve_load_warp(S.est, S.Kinv[it + 1 < iters ? 0 : 1], S.warp);
           wave_lds_sync();
           const int w = threadIdx.x;
           if (w < 12) put_word(&a.x->pose[w], S.pose[w], epoch);

@@ -727,8 +727,8 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         if (RGB) load_warp(S.est, L.Kinv, S.warp);
         fresh = false;
       } else if (bx != 0) {
-        if (threadIdx.x < 64) {
-          const int w = threadIdx.x;
+        const int w = fresh_tid();
+        if (w < 64) {
           float v[1];
           const bool ok = wait_words<1>(a.x->pose, [&](int) { return (w & 31) * 8; }, [&](int) { return w < (RGB ? 24 : 12); },
                                         epoch, a.wait_ticks, v);
@@ -738,8 +738,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         }
       }
       __syncthreads();
-      if (S.lost) return;
-      ++epoch;
+      const int lost = S.lost;  // looked at once the pose is on its way too
       PoseF T;
 #pragma unroll
       for (int i = 0; i < 9; ++i) T.r[i] = wave_uniform(S.pose[i]);
@@ -748,6 +747,8 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
       float wu[12];
 #pragma unroll
       for (int i = 0; i < 12; ++i) wu[i] = RGB ? wave_uniform(S.warp[i]) : 0.0f;
+      if (lost) return;
+      ++epoch;
       float acc[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
@@ -755,7 +756,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
       solve_pass1<ICP, RGB>(S, L, B, T, wu, a.sin2_max, a.dist2_max, bx, nb, ref, acc, count);
       if (RGB) {
         __syncthreads();
-        if (threadIdx.x == 64) {
+        if (fresh_tid() == 64) {
           float n = S.stats[0][0], mean = S.stats[0][1], m2 = S.stats[0][2];
 #pragma unroll
           for (int w = 1; w < 4; ++w) chan_merge(n, mean, m2, S.stats[w][0], S.stats[w][1], S.stats[w][2]);
@@ -767,7 +768,8 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
       if (ICP) {
         solve_pass1_end(S, solve_slots(L.w * L.h, nb), acc, count);
         __syncthreads();
-        if (threadIdx.x < 29) put_word(&a.x->icp[bx][threadIdx.x], row_total(S, threadIdx.x), epoch);
+        const int tid = fresh_tid();
+        if (tid < 29) put_word(&a.x->icp[bx][tid], row_total(S, tid), epoch);
       }
       if (RGB) {
         __syncthreads();  // S.stats and S.part are written again below
@@ -775,24 +777,27 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         if (S.lost) return;  // set before the barrier in solve_threshold
         solve_pass2(S, L, B, wu, th, bx, nb);
         __syncthreads();
-        if (threadIdx.x < 29) put_word(&a.x->rgb[bx][threadIdx.x], row_total(S, threadIdx.x), epoch);
+        const int tid = fresh_tid();
+        if (tid < 29) put_word(&a.x->rgb[bx][tid], row_total(S, tid), epoch);
       }
       if (bx != 0) continue;
       // workgroup 0: the step, and the next iteration's pose
-      if (RGB) solve_fold<16>(S, a.x->rgb, S.fold[1], threadIdx.x >> 6, nb, epoch, a.wait_ticks);
-      else solve_fold<16>(S, a.x->icp, S.fold[0], threadIdx.x >> 6, nb, epoch, a.wait_ticks);
+      const int wave = fresh_tid() >> 6;
+      if (RGB) solve_fold<16>(S, a.x->rgb, S.fold[1], wave, nb, epoch, a.wait_ticks);
+      else solve_fold<16>(S, a.x->icp, S.fold[0], wave, nb, epoch, a.wait_ticks);
       __syncthreads();
       if (S.lost) return;
-      if (threadIdx.x < 64) {
-        const int i = threadIdx.x & 31;
-        if (threadIdx.x < 32) {
+      const int lane = fresh_tid();
+      if (lane < 64) {
+        const int i = lane & 31;
+        if (lane < 32) {
           if (ICP) S.sums[0][i] = RGB ? solve_fold_total<8>(S.fold[0], i) : solve_fold_total<16>(S.fold[0], i);
         } else if (RGB) {
           S.sums[1][i] = solve_fold_total<16>(S.fold[1], i);
         }
         wave_lds_sync();
       }
-      if (threadIdx.x < 64) {
+      if (lane < 64) {
         const GnStep g = solve_step(a.mode, a.wrh, a.wrb, a.wih, a.wib);
         wave_lds_sync();
         const int nl = it + 1 < iters ? l : below;
@@ -800,17 +805,18 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
           load_pose_f(S.est, S.pose);
           if (RGB) solve_load_warp(S.est, S.Kinv[it + 1 < iters ? 0 : 1], S.warp);
           wave_lds_sync();
-          const int w = threadIdx.x;
+          const int w = fresh_tid();
           if (w < 12) put_word(&a.x->pose[w], S.pose[w], epoch);
           else if (RGB && w < 24) put_word(&a.x->pose[w], S.warp[w - 12], epoch);
         }
         // the state, while the pose is on its way
-        if (threadIdx.x < 29) {
-          if (ICP) S.s.sums_icp[threadIdx.x] = S.sums[0][threadIdx.x];
-          if (RGB) S.s.sums_rgb[threadIdx.x] = S.sums[1][threadIdx.x];
+        const int e = fresh_tid();
+        if (e < 29) {
+          if (ICP) S.s.sums_icp[e] = S.sums[0][e];
+          if (RGB) S.s.sums_rgb[e] = S.sums[1][e];
         }
         gn_step_record(&S.s, S.sums, S.s.last_err, ICP ? nb : 0, RGB ? nb : 0, it == 0, l == 0, g,
-                       S.est[threadIdx.x & 15]);
+                       S.est[e & 15]);
       }
       __syncthreads();
     }

@@ -29,8 +29,10 @@
 // when the device holds the grid, and for one stream at a time.  Every wait
 // is bounded by the clock all the same: a workgroup whose wait runs out
 // leaves, the tracker's state stays as it was before the solve, and
-// k_solve_rescue, which follows on the stream, takes the whole solve in one
-// workgroup with the launch-per-pass code (the same sums, so the same bits).
+// k_solve_rescue takes the whole solve in one workgroup with the
+// launch-per-pass code (the same sums, so the same bits).  It follows each
+// solve on the stream, except where the caller waits for the solve: that one
+// sees in host memory whether it completed and launches the rescue only then.
 #pragma once
 
 #include <type_traits>
@@ -54,6 +56,12 @@ struct SolveXchg {
   unsigned long long rgb[kRedGroups][32];
 };
 
+// A solve's result in host memory, for the caller that waits for it.
+struct HostState {
+  TrackState s;
+  int ok;  // the solve completed
+};
+
 struct SolveArgs {
   Level lv[kMaxLevels];
   TrackBufs tb[kMaxLevels];
@@ -68,6 +76,9 @@ struct SolveArgs {
   float* part_res;
   float* part_rgb;
   unsigned long long wait_ticks;  // bound of a wait, 100 MHz clock ticks
+  Mat44 init;      // the pose to start from when `has_init`, else the state's
+  int has_init;
+  HostState* host;  // when set, a completed solve's state goes there too (and `ok` is its)
 };
 
 // The thread index, as a value the compiler takes as new at each call: what
@@ -681,11 +692,16 @@ template <bool ICP, bool RGB>
 __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
   const int bx = blockIdx.x;
   unsigned epoch = a.x->epoch;
-  if (threadIdx.x < 16) S.est[threadIdx.x] = a.st->est[threadIdx.x];
+  if (threadIdx.x < 16) S.est[threadIdx.x] = a.has_init ? a.init.m[threadIdx.x] : a.st->est[threadIdx.x];
   if (threadIdx.x == 0) S.lost = 0;
-  if (bx == 0)
+  if (bx == 0) {
     for (int w = threadIdx.x; w < (int)(sizeof(TrackState) / 4); w += kSolveThreads)
       ((int*)&S.s)[w] = ((const int*)a.st)[w];
+    if (a.has_init) {
+      __syncthreads();
+      track_init_at(&S.s, a.init.m);
+    }
+  }
   __syncthreads();
   bool fresh = true;  // the pose in LDS is for this level's first iteration
 #pragma unroll 1
@@ -824,9 +840,12 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
   if (bx != 0) return;
   for (int w = threadIdx.x; w < (int)(sizeof(TrackState) / 4); w += kSolveThreads)
     ((int*)a.st)[w] = ((const int*)&S.s)[w];
+  if (a.host)
+    for (int w = threadIdx.x; w < (int)(sizeof(TrackState) / 4); w += kSolveThreads)
+      ((int*)&a.host->s)[w] = ((const int*)&S.s)[w];
   if (threadIdx.x == 0) {
     a.x->epoch = epoch;
-    a.x->ok = 1;
+    *(a.host ? &a.host->ok : &a.x->ok) = 1;
   }
 }
 

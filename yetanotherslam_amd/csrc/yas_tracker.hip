@@ -157,7 +157,7 @@ struct yas_tracker {
   float* part_rgb;  // [kRedGroups][32]
   TrackState* st;
   TrackState* st2;  // a solve's steps alternate between st and st2
-  TrackState* host_st;
+  HostState* host_st;
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
   float sin2_max, dist2_max;
@@ -344,26 +344,7 @@ static bool is_capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
-int yas_tracker_solve_async(yas_tracker* t) {
-  const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
-  hipStream_t s = t->ctx->stream;
-  const int device = t->ctx->device;
-  int grid = 0;
-  for (int l = t->P.levels - 1; l >= 0; --l)
-    if (t->P.iters[l] > 0) grid = groups_for(t->lv[l]);
-  if (grid == 0) return YAS_OK;  // no iteration at any level
-  const void* kernel = icp && rgb ? (const void*)k_solve<true, true>
-                                  : icp ? (const void*)k_solve<true, false> : (const void*)k_solve<false, true>;
-  if (device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels || is_capturing(s) ||
-      !solve_fits(device, kernel, grid)) return solve_by_passes(t);
-  std::lock_guard<std::mutex> lk(g_solve_mu);
-  auto& last = g_solve_last[device];
-  if (last.used && last.stream != s && (is_capturing(last.stream) || hipStreamQuery(last.stream) != hipSuccess)) {
-    (void)hipGetLastError();  // hipErrorNotReady is no failure
-    return solve_by_passes(t);
-  }
-  last.used = true;
-  last.stream = s;
+static SolveArgs solve_args(yas_tracker* t) {
   SolveArgs a;
   std::memset(&a, 0, sizeof(a));
   a.levels = t->P.levels;
@@ -381,17 +362,85 @@ int yas_tracker_solve_async(yas_tracker* t) {
   a.x = t->xchg;
   a.part_icp = t->part_icp; a.part_res = t->part_res; a.part_rgb = t->part_rgb;
   a.wait_ticks = t->wait_ticks;
-  if (icp && rgb) {
-    hipLaunchKernelGGL((k_solve<true, true>), dim3(grid), dim3(kSolveThreads), 0, s, a);
-    hipLaunchKernelGGL((k_solve_rescue<true, true>), dim3(1), dim3(256), 0, s, a);
-  } else if (icp) {
-    hipLaunchKernelGGL((k_solve<true, false>), dim3(grid), dim3(kSolveThreads), 0, s, a);
-    hipLaunchKernelGGL((k_solve_rescue<true, false>), dim3(1), dim3(256), 0, s, a);
-  } else {
-    hipLaunchKernelGGL((k_solve<false, true>), dim3(grid), dim3(kSolveThreads), 0, s, a);
-    hipLaunchKernelGGL((k_solve_rescue<false, true>), dim3(1), dim3(256), 0, s, a);
+  return a;
+}
+static void launch_rescue(const SolveArgs& a, hipStream_t s) {
+  const dim3 one(1), threads(256);
+  if (a.mode == YAS_TRACK_RGBD) hipLaunchKernelGGL((k_solve_rescue<true, true>), one, threads, 0, s, a);
+  else if (a.mode == YAS_TRACK_DEPTH) hipLaunchKernelGGL((k_solve_rescue<true, false>), one, threads, 0, s, a);
+  else hipLaunchKernelGGL((k_solve_rescue<false, true>), one, threads, 0, s, a);
+}
+
+// The solve in one launch from `init` (null: the state's pose), its result to
+// `host` too when not null; `done` tells whether this solve may run so (else
+// nothing is launched).
+static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool& done) {
+  hipStream_t s = t->ctx->stream;
+  const int device = t->ctx->device, mode = t->P.mode;
+  int grid = 0;
+  for (int l = t->P.levels - 1; l >= 0; --l)
+    if (t->P.iters[l] > 0) grid = groups_for(t->lv[l]);
+  done = false;
+  const void* kernel = mode == YAS_TRACK_RGBD ? (const void*)k_solve<true, true>
+                                              : mode == YAS_TRACK_DEPTH ? (const void*)k_solve<true, false>
+                                                                        : (const void*)k_solve<false, true>;
+  if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels || is_capturing(s) ||
+      !solve_fits(device, kernel, grid)) return YAS_OK;
+  std::lock_guard<std::mutex> lk(g_solve_mu);
+  auto& last = g_solve_last[device];
+  if (last.used && last.stream != s && (is_capturing(last.stream) || hipStreamQuery(last.stream) != hipSuccess)) {
+    (void)hipGetLastError();  // hipErrorNotReady is no failure
+    return YAS_OK;
   }
+  last.used = true;
+  last.stream = s;
+  SolveArgs a = solve_args(t);
+  if (init) a.init = *init;
+  a.has_init = init != nullptr;
+  a.host = host;
+  const dim3 threads(kSolveThreads);
+  if (mode == YAS_TRACK_RGBD) hipLaunchKernelGGL((k_solve<true, true>), dim3(grid), threads, 0, s, a);
+  else if (mode == YAS_TRACK_DEPTH) hipLaunchKernelGGL((k_solve<true, false>), dim3(grid), threads, 0, s, a);
+  else hipLaunchKernelGGL((k_solve<false, true>), dim3(grid), threads, 0, s, a);
   YAS_LAUNCH_CHECK();
+  done = true;
+  return YAS_OK;
+}
+
+int yas_tracker_solve_async(yas_tracker* t) {
+  bool done;
+  int rc = solve_in_one(t, nullptr, nullptr, done);
+  if (rc) return rc;
+  if (!done) return solve_by_passes(t);
+  launch_rescue(solve_args(t), t->ctx->stream);
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+
+// A solve from `init`, waited for; its state is left in host_st->s.  The one
+// launch takes the pose as an argument and leaves its result in host memory,
+// so the state's initialisation, the rescue and the result's copy, 4 to 5 us
+// each, are launched only where it did not run or did not complete.
+static int solve_and_wait(yas_tracker* t, const Mat44& init) {
+  hipStream_t s = t->ctx->stream;
+  t->host_st->ok = 0;
+  bool done;
+  int rc = solve_in_one(t, &init, t->host_st, done);
+  if (rc) return rc;
+  if (done) {
+    YAS_HIP(hipStreamSynchronize(s));
+    if (t->host_st->ok) return YAS_OK;
+  }
+  hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, s, t->st, init);
+  YAS_LAUNCH_CHECK();
+  if (done) {
+    launch_rescue(solve_args(t), s);
+    YAS_LAUNCH_CHECK();
+  } else if ((rc = solve_by_passes(t))) {
+    return rc;
+  }
+  YAS_HIP(hipMemcpyAsync(&t->host_st->s, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, s));
+  YAS_HIP(hipStreamSynchronize(s));
   return YAS_OK;
 }
 
@@ -528,7 +577,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   alloc((void**)&t->st, sizeof(TrackState));
   alloc((void**)&t->st2, sizeof(TrackState));
   alloc((void**)&t->xchg, sizeof(SolveXchg));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_st, sizeof(TrackState), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_st, sizeof(HostState), hipHostMallocDefault);
   if (e != hipSuccess) {
     yas_set_error("yas_tracker_create: %s", hipGetErrorString(e));
     yas_tracker_destroy(t);
@@ -732,13 +781,9 @@ int yas_tracker_get_transform(yas_tracker* t, const double init[16], int swap, d
   if (init) std::memcpy(M.m, init, sizeof(M.m));
   else
     for (int i = 0; i < 16; ++i) M.m[i] = (i % 5 == 0) ? 1.0 : 0.0;
-  hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, t->ctx->stream, t->st, M);
-  YAS_LAUNCH_CHECK();
-  int rc = yas_tracker_solve_async(t);
+  int rc = solve_and_wait(t, M);
   if (rc) return rc;
-  YAS_HIP(hipMemcpyAsync(t->host_st, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, t->ctx->stream));
-  YAS_HIP(hipStreamSynchronize(t->ctx->stream));
-  const TrackState& h = *t->host_st;
+  const TrackState& h = t->host_st->s;
   // RGBDTracking.cu:187-191: a NaN update returns before the buffer swap
   if (swap && h.good) yas_tracker_swap_frame_buffer(t);
   if (h.good) std::memcpy(out, h.last_ok, sizeof(h.last_ok));
@@ -755,9 +800,9 @@ int yas_tracker_get_transform(yas_tracker* t, const double init[16], int swap, d
 
 int yas_tracker_is_tracking_good(yas_tracker* t, int* good) {
   YAS_REQUIRE(t && good, "null argument");
-  YAS_HIP(hipMemcpyAsync(t->host_st, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, t->ctx->stream));
+  YAS_HIP(hipMemcpyAsync(&t->host_st->s, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, t->ctx->stream));
   YAS_HIP(hipStreamSynchronize(t->ctx->stream));
-  *good = t->host_st->good;
+  *good = t->host_st->s.good;
   return YAS_OK;
 }
 
@@ -770,11 +815,11 @@ int yas_tracker_step_sums(yas_tracker* t, int level, const double T[16], int kin
   hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, t->ctx->stream, t->st, M);
   int rc = launch_iteration(t, level, kind == 0, kind != 0, false, false);
   if (rc) return rc;
-  YAS_HIP(hipMemcpyAsync(t->host_st, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, t->ctx->stream));
+  YAS_HIP(hipMemcpyAsync(&t->host_st->s, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, t->ctx->stream));
   YAS_HIP(hipStreamSynchronize(t->ctx->stream));
-  const float* s = kind == 0 ? t->host_st->sums_icp : t->host_st->sums_rgb;
+  const float* s = kind == 0 ? t->host_st->s.sums_icp : t->host_st->s.sums_rgb;
   std::memcpy(out, s, sizeof(float) * 29);
-  if (stats) std::memcpy(stats, t->host_st->rgb_stats, sizeof(float) * 4);
+  if (stats) std::memcpy(stats, t->host_st->s.rgb_stats, sizeof(float) * 4);
   return YAS_OK;
 }
 

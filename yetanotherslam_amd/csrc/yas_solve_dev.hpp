@@ -92,31 +92,6 @@ __device__ inline int fresh_tid() {
 }
 
 // ------------------------------------------------------------------ lanes
-// Lane l's value from lane l ^ M.
-template <int M>
-__device__ inline float lane_xor(float v) {
-  int x = __builtin_bit_cast(int, v);
-  if (M == 1) x = __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
-  if (M == 2) x = __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, true);  // quad_perm [2,3,0,1]
-  if (M == 4) {
-    x = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, true);  // row_half_mirror: l ^ 7
-    x = __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xF, 0xF, true);   // quad_perm [3,2,1,0]: l ^ 3
-  }
-  if (M == 8) x = __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);  // row_ror:8
-  return __builtin_bit_cast(float, x);
-}
-// a of lanes with bit 32 clear plus a of their partners (l ^ 32), and b's
-// for the lanes with it set: one step of a transpose butterfly.
-__device__ inline float pair32(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
-                                                  false, false);
-  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-__device__ inline float pair16(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
-                                                  false, false);
-  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
 // Wavefront sums of 8 values in wave_sum32's order (partners at 32, 16, 8,
 // 4, 2, 1): lane l returns the total of value wave_sum8_index(l).
 __device__ inline float wave_sum8(const float (&v)[8]) {
@@ -136,6 +111,7 @@ __device__ inline int wave_sum8_index(int lane) {
 // wave_stats with the lanes' values exchanged by data-parallel moves instead
 // of LDS permutes, the lower lane's values first: lane 0 gets the wavefront's
 // (the others' are of no use, which spares telling which lane is the lower).
+// (Not for the passes: there it made the pixel loop spill.)
 template <int M>
 __device__ inline float lane_above(float v) {  // lane l + M's of the same 16; 0 past them
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + M, 0xF, 0xF, true));
@@ -313,9 +289,11 @@ __device__ inline float row_total(const SolveLds& S, int c) {
 }
 
 // ------------------------------------------------------------------ passes
-// Pixel k's row and column: the quotient by a float product, which is off
-// by less than 1 for any image (relative error 2^-22), then set right; the
-// integer division was 25 instructions of each pixel.
+// Pixel k's row and column: the quotient by a float product, set right where
+// it is off by one; the integer division was 25 instructions of each pixel.
+// The product's relative error is below 2^-22, so it is off by no more than
+// one in images of up to 2^22 rows (kFastRows).
+constexpr int kFastRows = 1 << 22;
 __device__ inline void pixel_xy(int k, int w, float winv, int& x, int& y) {
   y = (int)((float)k * winv);
   x = k - y * w;

@@ -384,7 +384,8 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
   const void* kernel = mode == YAS_TRACK_RGBD ? (const void*)k_solve<true, true>
                                               : mode == YAS_TRACK_DEPTH ? (const void*)k_solve<true, false>
                                                                         : (const void*)k_solve<false, true>;
-  if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels || is_capturing(s) ||
+  if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels ||
+      t->H > kFastRows || is_capturing(s) ||
       !solve_fits(device, kernel, grid)) return YAS_OK;
   std::lock_guard<std::mutex> lk(g_solve_mu);
   auto& last = g_solve_last[device];

@@ -36,30 +36,58 @@ struct TrackState {
   int rgb_inliers;
 };
 
+// ------------------------------------------------------------------ lanes
+// Lane l's value from lane l ^ M.
+template <int M>
+__device__ inline float lane_xor(float v) {
+  int x = __builtin_bit_cast(int, v);
+  if (M == 1) x = __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
+  if (M == 2) x = __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, true);  // quad_perm [2,3,0,1]
+  if (M == 4) {
+    x = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, true);  // row_half_mirror: l ^ 7
+    x = __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xF, 0xF, true);   // quad_perm [3,2,1,0]: l ^ 3
+  }
+  if (M == 8) x = __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);  // row_ror:8
+  return __builtin_bit_cast(float, x);
+}
+// a of lanes with bit 32 clear plus a of their partners (l ^ 32), and b's
+// for the lanes with it set: one step of a transpose butterfly.
+__device__ inline float pair32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                  false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ inline float pair16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                  false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
 // ------------------------------------------------------------------ reductions
 // Wave-wide sums of 32 values by a transpose butterfly: at each step a lane
-// keeps half of its values and trades the other half with its partner, so
-// 32 values need 16+8+4+2+1+1 shuffles.  On return, lanes 2i and 2i+1 hold
-// the total of value i.  The step size is a template constant so every
-// register index is static.
-template <int S>
-__device__ inline void butterfly_step(float (&v)[32], int lane) {
-  const bool hi = (lane & (2 * S)) != 0;
+// keeps half of its values and trades the other half with its partner (at
+// 32, 16, 8, 4, 2, 1), by register swaps and data-parallel moves, 74
+// instructions (63 LDS permutes with their selects were 250).  On return,
+// lanes 2i and 2i+1 hold the total of value i.
+template <int M, int S>
+__device__ inline void butterfly_step(float (&v)[32]) {
+  const bool hi = (threadIdx.x & M) != 0;
 #pragma unroll
   for (int i = 0; i < S; ++i) {
     const float send = hi ? v[i] : v[i + S];
     const float keep = hi ? v[i + S] : v[i];
-    v[i] = keep + __shfl_xor(send, 2 * S, 64);
+    v[i] = keep + lane_xor<M>(send);
   }
 }
 __device__ inline float wave_sum32(float (&v)[32]) {
-  const int lane = threadIdx.x & 63;
-  butterfly_step<16>(v, lane);
-  butterfly_step<8>(v, lane);
-  butterfly_step<4>(v, lane);
-  butterfly_step<2>(v, lane);
-  butterfly_step<1>(v, lane);
-  return v[0] + __shfl_xor(v[0], 1, 64);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = pair32(v[i], v[i + 16]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = pair16(v[i], v[i + 8]);
+  butterfly_step<8, 4>(v);
+  butterfly_step<4, 2>(v);
+  butterfly_step<2, 1>(v);
+  return v[0] + lane_xor<1>(v[0]);
 }
 
 // Workgroup sums of 32 values; thread t < 32 returns the total of value t.
@@ -135,28 +163,6 @@ __device__ inline void block_stats(float& n, float& mean, float& m2, float* st /
   float a = st[0], b = st[1], c = st[2];
   for (int k = 1; k < nw; ++k) chan_merge(a, b, c, st[3 * k], st[3 * k + 1], st[3 * k + 2]);
   n = a; mean = b; m2 = c;
-}
-
-// block_sum32 of two arrays in one LDS round: their wavefront sums overlap
-// and one pair of barriers serves both.  Thread t < 32 returns value t's
-// total of `a`, thread 32 + t that of `b`, each summed as block_sum32 does.
-__device__ inline float block_sum32x2(float (&a)[32], float (&b)[32], float* lds /* [2 * nwaves * 32] */) {
-  const float wa = wave_sum32(a);
-  const float wb = wave_sum32(b);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((lane & 1) == 0) {
-    lds[wid * 32 + (lane >> 1)] = wa;
-    lds[(nw + wid) * 32 + (lane >> 1)] = wb;
-  }
-  __syncthreads();
-  float t = 0.0f;
-  if (threadIdx.x < 64) {
-    const int base = threadIdx.x < 32 ? 0 : nw * 32, i = threadIdx.x & 31;
-    t = lds[base + i];
-    for (int k = 1; k < nw; ++k) t += lds[base + k * 32 + i];
-  }
-  __syncthreads();
-  return t;
 }
 
 // The end of a pass 1 with both terms: block_sum32 of the ICP values and
@@ -1142,6 +1148,32 @@ __device__ __attribute__((always_inline)) inline void gn_step_wave0(const float 
   if (st) gn_step_record(st, sums, s_last_err, gi, gr, do_step && first_of_level, record, g, t);
 }
 
+// The fold of up to 256 partial rows by 256 threads in block_sum32's order
+// (rows as threads of four wavefronts: partners at 32, 16, 8, 4, 2, 1, then the
+// wavefronts in turn).  Thread (value i, bit 0 of the row, wavefront) takes the
+// rows that differ in bits 5 to 1, so 32 lanes read a row's 128 bytes and the
+// fold is 31 additions in registers and one swap (a row a thread, folded by
+// wave_sum32, read 64 rows at once and exchanged 63 values).
+static_assert(kRedGroups == 256, "gn_update's fold");
+__device__ inline void load_rows(const float* part, int g, float (&v)[32]) {
+  const int i = threadIdx.x & 31, row0 = (threadIdx.x >> 6) * 64 + ((threadIdx.x >> 5) & 1);
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    const int r = row0 + 2 * j;
+    v[j] = part[(r < g ? r : g - 1) * 32 + i];
+  }
+#pragma unroll
+  for (int j = 0; j < 32; ++j) v[j] = row0 + 2 * j < g ? 0.0f + v[j] : 0.0f;
+}
+__device__ inline void fold_rows(float (&v)[32], float (&out)[4][32]) {
+#pragma unroll
+  for (int h = 16; h > 0; h >>= 1)
+#pragma unroll
+    for (int j = 0; j < h; ++j) v[j] = v[j] + v[j + h];
+  const float w = pair32(v[0], v[0]);
+  if ((threadIdx.x & 32) == 0) out[threadIdx.x >> 6][threadIdx.x & 31] = w;
+}
+
 // Fold the partial rows of one linearisation and, when `do_step`, take one
 // Gauss-Newton step of RGBDTracking.cu:161-204.  One workgroup.  The state
 // is read from st_in; when `write`, st_out receives it with the fold's and
@@ -1152,7 +1184,7 @@ __device__ __attribute__((always_inline)) inline void gn_update(const TrackState
                                                                 const float* part_rgb, int gr, int mode,
                                                                 int first_of_level, int do_step, int record, float wrh,
                                                                 float wrb, float wih, float wib, double* est_out) {
-  __shared__ float lds[2 * 4 * 32];
+  __shared__ float lds[2][4][32];
   __shared__ float sums[2][32];
   __shared__ double s_est[16];
   __shared__ int s_good;
@@ -1163,30 +1195,17 @@ __device__ __attribute__((always_inline)) inline void gn_update(const TrackState
   if (threadIdx.x < 16) s_est[threadIdx.x] = st_in->est[threadIdx.x];
   if (threadIdx.x == 16) s_good = st_in->good;
   if (threadIdx.x == 17) s_last_err = st_in->last_err;
-  // both terms' rows are read in one pass, so their loads overlap
+  // both terms' rows are read before either is folded, so their loads overlap
   float vi[32], vr[32];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) vi[i] = vr[i] = 0.0f;
-  const int g = gi > gr ? gi : gr;
-  for (int r = threadIdx.x; r < g; r += blockDim.x) {
-    if (r < gi) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) vi[i] += part_icp[r * 32 + i];
-    }
-    if (r < gr) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) vr[i] += part_rgb[r * 32 + i];
-    }
-  }
-  if (gi && gr) {
-    const float t = block_sum32x2(vi, vr, lds);
-    if (threadIdx.x < 64) sums[threadIdx.x >> 5][threadIdx.x & 31] = t;
-  } else if (gi) {
-    const float t = block_sum32(vi, lds);
-    if (threadIdx.x < 32) sums[0][threadIdx.x] = t;
-  } else if (gr) {
-    const float t = block_sum32(vr, lds);
-    if (threadIdx.x < 32) sums[1][threadIdx.x] = t;
+  if (gi) load_rows(part_icp, gi, vi);
+  if (gr) load_rows(part_rgb, gr, vr);
+  if (gi) fold_rows(vi, lds[0]);
+  if (gr) fold_rows(vr, lds[1]);
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const float(&f)[4][32] = lds[threadIdx.x >> 5];
+    const int i = threadIdx.x & 31;
+    if (threadIdx.x < 32 ? gi : gr) sums[threadIdx.x >> 5][i] = ((f[0][i] + f[1][i]) + f[2][i]) + f[3][i];
   }
   if (write && st_out != st_in) {
     // the fields this update leaves alone carry over

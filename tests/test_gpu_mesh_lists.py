@@ -117,3 +117,29 @@ def test_random_volume(gpu, tmp_path, fmt, ofmt, observed):
     np.testing.assert_allclose(ix["vertices"][ix["triangles"]].reshape(-1, 9), soup["tris"], rtol=0,
                                atol=4 * 2.0 ** -15 * 0.02)
     m.close()
+
+
+@pytest.mark.parametrize("indexed", [False, True])
+def test_one_engine_over_volumes_of_different_size(gpu, indexed):
+    """The engine's records are sized by the volumes before: one that fits,
+    one that outgrows them, a small one after it and an empty one all give
+    what an engine of their own gives."""
+    p = synth.params(width=160, height=120, theta0=0.7)
+    K = synth.intrinsics(p).astype(np.float32)
+    gt = synth.relative_poses(p, 6)
+    maps = []
+    for n in (1, 6, 1, 0):
+        m = rf.MapStruct(K, 1 << 15, 1 << 13, 0.01, 0.04)
+        for t in range(n):
+            m.FuseU16(to_dev(synth.frame(p, 3 * t)[0]), gt[t])
+        maps.append(m)
+    nb = [m.stats().num_allocated for m in maps]
+    assert nb[1] > 1.25 * nb[0] > 0 and nb[3] == 0
+    me = rf.MeshEngine(2_000_000)
+    for m in [maps[3]] + maps:
+        own = rf.MeshEngine(2_000_000)
+        a, b = ((e.MeshifyIndexed(m) if indexed else e.Meshify(m, with_cases=True)) for e in (me, own))
+        assert a.keys() == b.keys()
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
+        own.close()

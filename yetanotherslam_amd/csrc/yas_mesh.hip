@@ -80,6 +80,14 @@ constexpr int kMcWaves = 4;
 constexpr int kMcThreads = 64 * kMcWaves;
 constexpr int kMcCube = 9 * 9 * 9;  // a block and its +1 halo, index (z*9 + y)*9 + x
 
+// The volume's blocks, or none when they are more than the records' `cap`:
+// the host launches for the capacity, without asking for the count first,
+// and repeats the extraction with more room when it did not suffice.
+__device__ inline int mc_num_blocks(const MapView& m, int cap) {
+  int n = m.ctr[kCtrAlloc];
+  n = n < m.num_blocks ? n : m.num_blocks;
+  return n <= cap ? n : 0;
+}
 // The block of this thread's wavefront.
 __device__ inline int mc_block() {
   return __builtin_amdgcn_readfirstlane((int)blockIdx.x * kMcWaves + (int)(threadIdx.x >> 6));
@@ -203,13 +211,13 @@ __device__ inline int block_excl_scan(int v, int* wsum, int& total) {
 // reading its 8 corners there; 107 us with a slice's planes as 64-bit scalar
 // masks, some 850 scalar instructions a block for a CU's one scalar unit.)
 template <class VT>
-__global__ void __launch_bounds__(kMcThreads) k_mc_count(MapView m, int nblocks, int2* counts, int16_t* cases,
+__global__ void __launch_bounds__(kMcThreads) k_mc_count(MapView m, int cap, int2* counts, int16_t* cases,
                                                          uint16_t* vinfo, int* nbr) {
   __shared__ unsigned char tri_n[256];
   if (threadIdx.x < 256) tri_n[threadIdx.x] = (unsigned char)(kTriTable[threadIdx.x] & 0xF);
   __syncthreads();
   const int blk = mc_block();
-  if (blk >= nblocks) return;
+  if (blk >= mc_num_blocks(m, cap)) return;
   const int lane = threadIdx.x & 63, a = lane & 7, b = lane >> 3;
   const typename VT::T* vox = (const typename VT::T*)m.voxels;
   typename VT::T own[8];
@@ -292,16 +300,19 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_count(MapView m, int nblocks,
 // `chunk`; block i's prefix is out[i] + chunk[i >> kMcChunkShift], which its
 // readers add.  (As three launches, local scan, chunk scan and addition, it
 // cost 14 us of a 284 us extraction.)  `done` is 0 before and after.
+struct McTotals {
+  int tri, vert, blocks;
+};
 constexpr int kMcChunkShift = 10, kMcChunk = 1 << kMcChunkShift;
 __device__ inline unsigned long long mc_pack2(int x, int y) {
   return (unsigned long long)(unsigned)x | (unsigned long long)(unsigned)y << 32;
 }
-__global__ void __launch_bounds__(kMcChunk) k_mc_scan(const int2* in, int2* out, int n, unsigned long long* chunk,
-                                                      int2* total, unsigned* done) {
+__global__ void __launch_bounds__(kMcChunk) k_mc_scan(MapView m, int cap, const int2* in, int2* out,
+                                                      unsigned long long* chunk, McTotals* total, unsigned* done) {
   __shared__ int wsum[16];
   __shared__ int carry[2];
   __shared__ int last;
-  const int i = blockIdx.x * kMcChunk + threadIdx.x, nchunks = gridDim.x;
+  const int i = blockIdx.x * kMcChunk + threadIdx.x, nchunks = gridDim.x, n = mc_num_blocks(m, cap);
   const int2 v = i < n ? in[i] : make_int2(0, 0);
   int tx, ty;
   const int ex = block_excl_scan(v.x, wsum, tx);
@@ -329,7 +340,7 @@ __global__ void __launch_bounds__(kMcChunk) k_mc_scan(const int2* in, int2* out,
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    *total = make_int2(carry[0], carry[1]);
+    *total = McTotals{carry[0], carry[1], m.ctr[kCtrAlloc] < m.num_blocks ? m.ctr[kCtrAlloc] : m.num_blocks};
     *done = 0;
   }
 }
@@ -517,13 +528,14 @@ __device__ inline void mc_soup_flush(const McSoupLds& S, const McTables& T, int 
   }
 }
 template <class VT>
-__global__ void __launch_bounds__(kMcThreads) k_mc_emit(MapView m, int nblocks, McOffsets offsets,
+__global__ void __launch_bounds__(kMcThreads) k_mc_emit(MapView m, int cap_blocks, McOffsets offsets,
                                                         const int16_t* cases, float* tris, float* normals, int cap,
                                                         const int* nbr) {
   __shared__ McTables T;
   __shared__ McSoupLds lds[kMcWaves];
   mc_fill_tables(T);
   __syncthreads();
+  const int nblocks = mc_num_blocks(m, cap_blocks);
   const int lane = threadIdx.x & 63, stride = gridDim.x * kMcWaves;
   McSoupLds& S = lds[threadIdx.x >> 6];
   int blk = mc_block(), nb = -1;
@@ -613,7 +625,7 @@ __device__ inline void mc_index_flush(const McIndexedLds& S, const McTables& T, 
   }
 }
 template <class VT>
-__global__ void __launch_bounds__(kMcThreads) k_mc_emit_indexed(MapView m, int nblocks, McOffsets offsets,
+__global__ void __launch_bounds__(kMcThreads) k_mc_emit_indexed(MapView m, int cap_blocks, McOffsets offsets,
                                                                 const int16_t* cases, const uint16_t* vinfo,
                                                                 float* verts, int vcap, int* tris, int tcap,
                                                                 const int* nbr) {
@@ -621,6 +633,7 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_emit_indexed(MapView m, int n
   __shared__ McIndexedLds lds[kMcWaves];
   mc_fill_tables(T);
   __syncthreads();
+  const int nblocks = mc_num_blocks(m, cap_blocks);
   const int lane = threadIdx.x & 63, stride = gridDim.x * kMcWaves;
   McIndexedLds& S = lds[threadIdx.x >> 6];
   int blk = mc_block(), nb = -1;
@@ -695,7 +708,7 @@ struct yas_mesher {
   int2* offsets;    // exclusive prefix of counts within a chunk
   unsigned long long* chunk;  // exclusive prefix of 1024-block chunks, {triangles, vertices}
   unsigned* done;   // the scan's finished workgroups
-  int2* total;      // {triangles, vertices}, host memory
+  McTotals* total;  // host memory
   int16_t* cases;   // per voxel cube index
   uint16_t* vinfo;  // per voxel (local vertex prefix << 3 | owned edges)
   int* nbr;         // per block, pool indices of it and its 7 +x/+y/+z neighbours (-1 absent)
@@ -708,8 +721,10 @@ struct yas_mesher {
   yas_map* map;
 };
 
-static int ensure_block_cap(yas_mesher* me, int n) {
-  if (n <= me->block_cap) return YAS_OK;
+// Records for `need` blocks and a quarter more, at most `most`.
+static int ensure_block_cap(yas_mesher* me, int need, int most) {
+  if (need <= me->block_cap) return YAS_OK;
+  const int n = (int)std::min<long long>(most, (long long)need + need / 4);
   hipFree(me->counts);
   hipFree(me->offsets);
   hipFree(me->chunk);
@@ -732,59 +747,79 @@ static int ensure_block_cap(yas_mesher* me, int n) {
   return YAS_OK;
 }
 
-// Count + scan over every allocated block of `map`; fills me->num_blocks and
-// leaves the totals on the device.
-static int count_and_scan(yas_mesher* me, yas_map* map, MapView& v) {
+// Workgroups of an emission pass: as many as the device holds at once, each
+// wavefront taking blocks in turn, for the records' capacity.
+static int emit_groups(yas_mesher* me, const void* kernel, int* groups) {
+  int per = 0;
+  YAS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, kMcThreads, 0));
+  const int all = (me->block_cap + kMcWaves - 1) / kMcWaves, fit = std::max(1, per) * me->cus;
+  *groups = std::min(all, fit);
+  return YAS_OK;
+}
+
+template <class VT>
+static int launch_extract(yas_mesher* me, const MapView& v) {
+  hipStream_t s = me->ctx->stream;
+  const int cap = me->block_cap;
+  const McOffsets off = {me->offsets, me->chunk};
+  int groups = 0, rc;
+  hipLaunchKernelGGL(k_mc_count<VT>, dim3((cap + kMcWaves - 1) / kMcWaves), dim3(kMcThreads), 0, s, v, cap, me->counts, me->cases, me->vinfo,
+                     me->nbr);
+  YAS_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_mc_scan, dim3((cap + kMcChunk - 1) / kMcChunk), dim3(kMcChunk), 0, s, v, cap,
+                     (const int2*)me->counts, me->offsets, me->chunk, me->total, me->done);
+  YAS_LAUNCH_CHECK();
+  if (me->indexed) {
+    // triangle indices in the soup buffer (3 of its 9 floats per triangle),
+    // vertices in the normal buffer (capacity max_tri * 3 vertices)
+    if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VT>, &groups))) return rc;
+    hipLaunchKernelGGL(k_mc_emit_indexed<VT>, dim3(groups), dim3(kMcThreads), 0, s, v, cap, off,
+                       (const int16_t*)me->cases, (const uint16_t*)me->vinfo, me->normals, me->max_tri * 3,
+                       (int*)me->tris, me->max_tri, (const int*)me->nbr);
+  } else {
+    if ((rc = emit_groups(me, (const void*)k_mc_emit<VT>, &groups))) return rc;
+    hipLaunchKernelGGL(k_mc_emit<VT>, dim3(groups), dim3(kMcThreads), 0, s, v, cap, off, (const int16_t*)me->cases,
+                       me->tris, me->normals, me->max_tri, (const int*)me->nbr);
+  }
+  YAS_LAUNCH_CHECK();
+  return YAS_OK;
+}
+
+// Extraction of every allocated block of `map`, waited for: num_blocks,
+// num_tri and num_vert.  The passes read the block count themselves and write
+// the totals to host memory, so one wait serves for both (asking for the
+// count first cost some 25 us); records are kept for a quarter more blocks
+// than were needed, and a volume that outgrew them is extracted again.
+static int extract(yas_mesher* me, yas_map* map, bool indexed) {
   YAS_REQUIRE(me && map, "yas_mesh_extract: null argument");
   YAS_REQUIRE_ACTIVE(map);
   YAS_REQUIRE(yas_map_ctx(map)->stream == me->ctx->stream, "yas_mesh_extract: map and mesher must share a stream");
   YAS_HIP(hipSetDevice(me->ctx->device));
-  yas_map_stats st;
-  int rc = yas_map_get_stats(map, &st);
-  if (rc) return rc;
-  const int n = st.num_allocated;
-  me->num_blocks = n;
-  me->num_tri = me->num_vert = 0;
+  me->num_blocks = me->num_tri = me->num_vert = 0;
   me->map = map;
-  if (n == 0) return YAS_OK;
-  if ((rc = ensure_block_cap(me, n))) return rc;
-  v = yas_map_view(map);
-  hipStream_t s = me->ctx->stream;
-  const int groups = (n + kMcWaves - 1) / kMcWaves;
-  switch (v.format) {
-    case YAS_VOXEL_I16_U8:
-      hipLaunchKernelGGL(k_mc_count<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
-                         me->nbr);
-      break;
-    case YAS_VOXEL_F16_U16:
-      hipLaunchKernelGGL(k_mc_count<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
-                         me->nbr);
-      break;
-    default:
-      hipLaunchKernelGGL(k_mc_count<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, me->counts, me->cases, me->vinfo,
-                         me->nbr);
+  me->indexed = indexed;
+  const MapView v = yas_map_view(map);
+  int rc;
+  if (me->block_cap == 0) {
+    yas_map_stats st;
+    if ((rc = yas_map_get_stats(map, &st))) return rc;
+    if (st.num_allocated == 0) return YAS_OK;
+    if ((rc = ensure_block_cap(me, st.num_allocated, v.num_blocks))) return rc;
   }
-  YAS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_mc_scan, dim3((n + kMcChunk - 1) / kMcChunk), dim3(kMcChunk), 0, s, (const int2*)me->counts,
-                     me->offsets, n, me->chunk, me->total, me->done);
-  YAS_LAUNCH_CHECK();
-  return YAS_OK;
-}
-
-static int read_totals(yas_mesher* me) {
-  YAS_HIP(hipStreamSynchronize(me->ctx->stream));
-  me->num_tri = me->total->x;
-  me->num_vert = me->total->y;
-  return YAS_OK;
-}
-
-// Workgroups of an emission pass: as many as the device holds at once, each
-// wavefront taking blocks in turn.
-static int emit_groups(yas_mesher* me, const void* kernel, int* groups) {
-  int per = 0;
-  YAS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, kMcThreads, 0));
-  const int all = (me->num_blocks + kMcWaves - 1) / kMcWaves, fit = std::max(1, per) * me->cus;
-  *groups = std::min(all, fit);
+  for (;;) {
+    switch (v.format) {
+      case YAS_VOXEL_I16_U8: rc = launch_extract<VoxI16>(me, v); break;
+      case YAS_VOXEL_F16_U16: rc = launch_extract<VoxF16>(me, v); break;
+      default: rc = launch_extract<VoxF32>(me, v);
+    }
+    if (rc) return rc;
+    YAS_HIP(hipStreamSynchronize(me->ctx->stream));
+    if (me->total->blocks <= me->block_cap) break;
+    if ((rc = ensure_block_cap(me, me->total->blocks, v.num_blocks))) return rc;
+  }
+  me->num_blocks = me->total->blocks;
+  me->num_tri = me->total->tri;
+  me->num_vert = me->total->vert;
   return YAS_OK;
 }
 
@@ -811,7 +846,7 @@ int yas_mesher_create(yas_ctx* ctx, int max_triangles, yas_mesher** out) {
   me->max_tri = max_triangles;
   hipError_t e = hipMalloc((void**)&me->tris, sizeof(float) * 9 * (size_t)max_triangles);
   if (e == hipSuccess) e = hipMalloc((void**)&me->normals, sizeof(float) * 9 * (size_t)max_triangles);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&me->total, sizeof(int2), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&me->total, sizeof(McTotals), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc((void**)&me->done, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(me->done, 0, sizeof(unsigned));
   if (e == hipSuccess) e = hipDeviceGetAttribute(&me->cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
@@ -845,33 +880,8 @@ int yas_mesher_destroy(yas_mesher* me) {
 
 int yas_mesh_extract(yas_mesher* me, yas_map* map, int* num_triangles) {
   if (num_triangles) *num_triangles = 0;
-  MapView v;
-  int rc = count_and_scan(me, map, v);
+  int rc = extract(me, map, false);
   if (rc) return rc;
-  me->indexed = 0;
-  const int n = me->num_blocks;
-  if (n == 0) return YAS_OK;
-  hipStream_t s = me->ctx->stream;
-  const McOffsets off = {me->offsets, me->chunk};
-  int groups = 0;
-  switch (v.format) {
-    case YAS_VOXEL_I16_U8:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxI16>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
-      break;
-    case YAS_VOXEL_F16_U16:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxF16>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
-      break;
-    default:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit<VoxF32>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         me->tris, me->normals, me->max_tri, (const int*)me->nbr);
-  }
-  YAS_LAUNCH_CHECK();
-  if ((rc = read_totals(me))) return rc;
   if (num_triangles) *num_triangles = me->num_tri;
   if (me->num_tri > me->max_tri) {
     yas_set_error("yas_mesh_extract: %d triangles exceed the capacity %d", me->num_tri, me->max_tri);
@@ -883,37 +893,9 @@ int yas_mesh_extract(yas_mesher* me, yas_map* map, int* num_triangles) {
 int yas_mesh_extract_indexed(yas_mesher* me, yas_map* map, int* num_vertices, int* num_triangles) {
   if (num_vertices) *num_vertices = 0;
   if (num_triangles) *num_triangles = 0;
-  MapView v;
-  int rc = count_and_scan(me, map, v);
+  int rc = extract(me, map, true);
   if (rc) return rc;
-  me->indexed = 1;
-  const int n = me->num_blocks;
-  if (n == 0) return YAS_OK;
-  hipStream_t s = me->ctx->stream;
-  // triangle indices in the soup buffer (3 of its 9 floats per triangle),
-  // vertices in the normal buffer (capacity max_tri * 3 vertices)
-  int* tri_idx = (int*)me->tris;
   const int vcap = me->max_tri * 3;
-  const McOffsets off = {me->offsets, me->chunk};
-  int groups = 0;
-  switch (v.format) {
-    case YAS_VOXEL_I16_U8:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxI16>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxI16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
-      break;
-    case YAS_VOXEL_F16_U16:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxF16>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF16>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
-      break;
-    default:
-      if ((rc = emit_groups(me, (const void*)k_mc_emit_indexed<VoxF32>, &groups))) return rc;
-      hipLaunchKernelGGL(k_mc_emit_indexed<VoxF32>, dim3(groups), dim3(kMcThreads), 0, s, v, n, off, (const int16_t*)me->cases,
-                         (const uint16_t*)me->vinfo, me->normals, vcap, tri_idx, me->max_tri, (const int*)me->nbr);
-  }
-  YAS_LAUNCH_CHECK();
-  if ((rc = read_totals(me))) return rc;
   if (num_vertices) *num_vertices = me->num_vert;
   if (num_triangles) *num_triangles = me->num_tri;
   if (me->num_tri > me->max_tri || me->num_vert > vcap) {

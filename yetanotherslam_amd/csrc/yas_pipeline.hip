@@ -165,8 +165,8 @@ struct yas_pipeline {
   float* depth;
   float* gray;
   double* T_last;
-  double* poses;
-  int* tracked;
+  double* poses;  // per frame, in host memory: the kernels write them, callers read them
+  int* tracked;   // likewise
   int* gate;
   int frames;
   int cap;
@@ -176,14 +176,14 @@ static int grow(yas_pipeline* p) {
   int ncap = p->cap ? p->cap * 2 : 1024;
   double* np = nullptr;
   int* nt = nullptr;
-  YAS_HIP(hipMalloc((void**)&np, sizeof(double) * 16 * (size_t)ncap));
-  YAS_HIP(hipMalloc((void**)&nt, sizeof(int) * (size_t)ncap));
+  YAS_HIP(hipHostMalloc((void**)&np, sizeof(double) * 16 * (size_t)ncap, hipHostMallocDefault));
+  YAS_HIP(hipHostMalloc((void**)&nt, sizeof(int) * (size_t)ncap, hipHostMallocDefault));
   if (p->cap) {
-    YAS_HIP(hipMemcpyAsync(np, p->poses, sizeof(double) * 16 * p->cap, hipMemcpyDeviceToDevice, p->ctx->stream));
-    YAS_HIP(hipMemcpyAsync(nt, p->tracked, sizeof(int) * p->cap, hipMemcpyDeviceToDevice, p->ctx->stream));
     YAS_HIP(hipStreamSynchronize(p->ctx->stream));
-    hipFree(p->poses);
-    hipFree(p->tracked);
+    std::memcpy(np, p->poses, sizeof(double) * 16 * (size_t)p->cap);
+    std::memcpy(nt, p->tracked, sizeof(int) * (size_t)p->cap);
+    hipHostFree(p->poses);
+    hipHostFree(p->tracked);
   }
   int* ns = nullptr;
   YAS_HIP(hipMalloc((void**)&ns, sizeof(int) * 8 * (size_t)ncap));
@@ -293,8 +293,8 @@ int yas_pipeline_destroy(yas_pipeline* p) {
   hipFree(p->depth);
   hipFree(p->gray);
   hipFree(p->T_last);
-  hipFree(p->poses);
-  hipFree(p->tracked);
+  if (p->poses) hipHostFree(p->poses);
+  if (p->tracked) hipHostFree(p->tracked);
   hipFree(p->gate);
   hipFree(p->frame_stats);
   for (auto* v : {&p->pending, &p->spare})
@@ -418,8 +418,8 @@ int yas_pipeline_pose(yas_pipeline* p, int frame, double T[16], int* tracked) {
   YAS_REQUIRE(frame >= 0 && frame < p->frames, "yas_pipeline_pose: no such frame");
   YAS_HIP(hipSetDevice(p->ctx->device));
   YAS_HIP(hipStreamSynchronize(p->ctx->stream));
-  YAS_HIP(hipMemcpy(T, p->poses + 16 * (size_t)frame, sizeof(double) * 16, hipMemcpyDeviceToHost));
-  if (tracked) YAS_HIP(hipMemcpy(tracked, p->tracked + frame, sizeof(int), hipMemcpyDeviceToHost));
+  std::memcpy(T, p->poses + 16 * (size_t)frame, sizeof(double) * 16);
+  if (tracked) *tracked = p->tracked[frame];
   return YAS_OK;
 }
 

@@ -367,11 +367,12 @@ struct MapView {
 };
 
 // Linear-probe lookup from the reference hash's home slot: the pool index
-// (-1 if absent) and the block's summary flags.
-__device__ inline int find_block(const MapView& m, uint64_t key, int home, int* flags = nullptr) {
+// (-1 if absent) and the block's summary flags.  `first`: probes already made
+// (those before `home`).
+__device__ inline int find_block(const MapView& m, uint64_t key, int home, int* flags = nullptr, int first = 0) {
   int slot = home;
   const int lim = m.num_buckets < kMaxProbe ? m.num_buckets : kMaxProbe;
-  for (int p = 0; p < lim; ++p) {
+  for (int p = first; p < lim; ++p) {
     // One 16-byte load.  The empty asm statement takes the pool index and
     // flags as register operands right after it, so the compiler cannot
     // defer their half of the slot to a second, dependent load on a match.
@@ -390,6 +391,34 @@ __device__ inline int find_block(const MapView& m, uint64_t key, int home, int* 
 __device__ inline int find_block_xyz(const MapView& m, int bx, int by, int bz, int* flags = nullptr) {
   if (!key_in_range(bx, by, bz)) return -1;
   return find_block(m, pack_key(bx, by, bz), ref_hash(bx, by, bz, m.num_buckets), flags);
+}
+// N lookups (those with `want`) whose first probes, mostly the only ones, are
+// in flight together.
+template <int N>
+__device__ inline void find_blocks(const MapView& m, const int (&b)[N][3], const bool (&want)[N], int (&idx)[N],
+                                   int (&flags)[N]) {
+  uint4 e[N];
+  int slot[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    idx[i] = -1;
+    flags[i] = 0;
+    slot[i] = want[i] && key_in_range(b[i][0], b[i][1], b[i][2]) ? ref_hash(b[i][0], b[i][1], b[i][2], m.num_buckets) : -1;
+    e[i] = reinterpret_cast<const uint4*>(m.slots)[slot[i] < 0 ? 0 : slot[i]];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    asm volatile("" : "+v"(e[i].z), "+v"(e[i].w));
+    const unsigned long long k = ((unsigned long long)e[i].y << 32) | e[i].x;
+    const uint64_t key = pack_key(b[i][0], b[i][1], b[i][2]);
+    if (slot[i] < 0 || k == kEmptyKey) continue;
+    if (k == key) {
+      idx[i] = (int)e[i].z;
+      flags[i] = (int)e[i].w;
+    } else {
+      idx[i] = find_block(m, key, slot[i] + 1 == m.num_buckets ? 0 : slot[i] + 1, &flags[i], 1);
+    }
+  }
 }
 
 // ------------------------------------------------------------------ frame outcome

@@ -288,30 +288,42 @@ struct VoxelReader {
     const int mask = (int)(bx1 != bx0) | ((int)(by1 != by0) << 1) | ((int)(bz1 != bz0) << 2);
     float sv[8];
     sv[0] = s0;
-    if ((mask & (mask - 1)) == 0) {
+    if (mask != 7) {
       const int code_a = corner_code(cblk, cflags);
-      int code_b = code_a;
-      if (mask) {
+      const int lo = mask & -mask, hi = mask ^ lo;  // the straddled axes (0: none)
+      int code_lo = code_a, code_hi = code_a, code_both = code_a;
+      if (hi) {
+        const int at[3][3] = {{(lo & 1) ? bx1 : bx0, (lo & 2) ? by1 : by0, (lo & 4) ? bz1 : bz0},
+                              {(hi & 1) ? bx1 : bx0, (hi & 2) ? by1 : by0, (hi & 4) ? bz1 : bz0},
+                              {bx1, by1, bz1}};
+        const bool want[3] = {true, true, true};
+        int idx[3], fl[3];
+        find_blocks(m, at, want, idx, fl);
+        code_lo = corner_code(idx[0], fl[0]);
+        code_hi = corner_code(idx[1], fl[1]);
+        code_both = corner_code(idx[2], fl[2]);
+      } else if (lo) {
         int fb = 0;
-        const int ib = find_block_xyz(m, (mask & 1) ? bx1 : bx0, (mask & 2) ? by1 : by0, (mask & 4) ? bz1 : bz0, &fb);
-        code_b = corner_code(ib, fb);
+        const int ib = find_block_xyz(m, bx1, by1, bz1, &fb);
+        code_lo = corner_code(ib, fb);
       }
       const int ly[2] = {vox_to_local(y0), vox_to_local(y1)};
       const int lz[2] = {vox_to_local(z0), vox_to_local(z1)};
       typename VT::T raw[8];
+      int code[8];
 #pragma unroll
       for (int c = 1; c < 8; ++c) {
-        const int code = (c & mask) ? code_b : code_a;
+        const int side = c & mask;
+        code[c] = side == 0 ? code_a : side == lo ? code_lo : side == hi ? code_hi : code_both;
         const size_t at =
-            code >= 0 ? (size_t)code * 512 + (lz[c >> 2] * 8 + ly[(c >> 1) & 1]) * 8 + ((c & 1) ? lx1 : lx0) : 0;
+            code[c] >= 0 ? (size_t)code[c] * 512 + (lz[c >> 2] * 8 + ly[(c >> 1) & 1]) * 8 + ((c & 1) ? lx1 : lx0) : 0;
         raw[c] = vox[at];
       }
 #pragma unroll
       for (int c = 1; c < 8; ++c) {
-        const int code = (c & mask) ? code_b : code_a;
-        bool v = code == -1;
+        bool v = code[c] == -1;
         sv[c] = 1.0f;
-        if (code >= 0 && VT::observed(raw[c])) {
+        if (code[c] >= 0 && VT::observed(raw[c])) {
           v = true;
           sv[c] = VT::sdf(raw[c]);
         }

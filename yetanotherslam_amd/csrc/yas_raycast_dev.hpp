@@ -292,14 +292,14 @@ struct VoxelReader {
       const int code_a = corner_code(cblk, cflags);
       const int lo = mask & -mask, hi = mask ^ lo;  // the straddled axes (0: none)
       int code_lo = code_a, code_hi = code_a, code_both = code_a;
-      if (hi) {
+      if (__any(hi)) {
         const int at[3][3] = {{(lo & 1) ? bx1 : bx0, (lo & 2) ? by1 : by0, (lo & 4) ? bz1 : bz0},
                               {(hi & 1) ? bx1 : bx0, (hi & 2) ? by1 : by0, (hi & 4) ? bz1 : bz0},
                               {bx1, by1, bz1}};
-        const bool want[3] = {true, true, true};
+        const bool want[3] = {lo != 0, hi != 0, hi != 0};
         int idx[3], fl[3];
         find_blocks(m, at, want, idx, fl);
-        code_lo = corner_code(idx[0], fl[0]);
+        if (lo) code_lo = corner_code(idx[0], fl[0]);
         code_hi = corner_code(idx[1], fl[1]);
         code_both = corner_code(idx[2], fl[2]);
       } else if (lo) {

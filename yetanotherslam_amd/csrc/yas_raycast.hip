@@ -13,6 +13,7 @@ using namespace yas;
 
 MapView yas_map_view(yas_map* map);
 const PosePair* yas_map_pose_dev(yas_map* map);
+Intr yas_map_intr(yas_map* map);
 yas_ctx* yas_map_ctx(yas_map* map);
 int yas_map_visible_async(yas_map* map, const double T[16], int W, int H);
 int yas_map_visible_prepared(yas_map* map, int W, int H);
@@ -38,11 +39,11 @@ __global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zm
 // Visibility and z-range cells (view_scan).  Workgroup b: slice b / chunks of
 // the block list, chunk b % chunks of the cell rows (rows_per each).
 template <class P>
-__global__ void __launch_bounds__(256) k_view(MapView m, P pose, Intr K, int W, int H, int cols, int rows,
+__global__ void __launch_bounds__(256) k_view(MapView m, P pose, Intr Kmap, Intr K, int W, int H, int cols, int rows,
                                               unsigned* zmin, unsigned* zmax, int slices, int chunks, int rows_per) {
   extern __shared__ unsigned lz[];
   const int chunk = blockIdx.x % chunks, r0 = chunk * rows_per;
-  view_scan(m, pose.Tinv(), K, W, H, cols, rows, zmin, zmax, lz, blockIdx.x / chunks, slices, r0,
+  view_scan(m, pose.Tinv(), Kmap, K, W, H, cols, rows, zmin, zmax, lz, blockIdx.x / chunks, slices, r0,
             min(rows, r0 + rows_per), chunk == 0);
 }
 
@@ -78,7 +79,7 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
     const int most = kViewCells / cols, chunks = (rows + most - 1) / most, rows_per = (rows + chunks - 1) / chunks;
     const int slices = chunks < kViewGroups ? kViewGroups / chunks : 1;
     hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(256), 2 * sizeof(unsigned) * (size_t)rows_per * cols, s,
-                       v, pose, K, W, H, cols, rows, zmin, zmax, slices, chunks, rows_per);
+                       v, pose, yas_map_intr(map), K, W, H, cols, rows, zmin, zmax, slices, chunks, rows_per);
   } else {
     int r = T ? yas_map_visible_async(map, T, W, H) : yas_map_visible_prepared(map, W, H);
     if (r) return r;

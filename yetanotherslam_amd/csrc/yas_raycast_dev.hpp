@@ -125,7 +125,8 @@ __device__ inline void zrange_lds_at(const MapView& m, const PosePair* pose, con
 }
 
 // What a ray cast needs of the block list in one pass: the visible blocks
-// compacted into the visible list (visible_scan's test) and their depth
+// compacted into the visible list (visible_scan's test, by the map's
+// intrinsics Kmap, which the ray caster's K may differ from) and their depth
 // ranges reduced into the cells, as zrange_lds_at does.  Workgroup (slice,
 // chunk) takes a contiguous slice of the block list and the cell rows r0 ..
 // r1 - 1 (nc cells, 2 words of LDS each); the workgroups of the first chunk
@@ -134,7 +135,7 @@ __device__ inline void zrange_lds_at(const MapView& m, const PosePair* pose, con
 // reduce in LDS too, in chunks.
 constexpr int kViewCells = 9728;  // cells of a chunk: 76 KB, two workgroups a CU
 
-__device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& K, int W, int H, int cols, int rows,
+__device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& Kmap, const Intr& K, int W, int H, int cols, int rows,
                                  unsigned* zmin, unsigned* zmax, unsigned* lds, int slice, int slices, int r0, int r1,
                                  bool list) {
   const int c0 = r0 * cols, nc = (r1 - r0) * cols;
@@ -158,7 +159,7 @@ __device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& 
       int bx, by, bz;
       key = m.block_keys[i];
       unpack_key(key, bx, by, bz);
-      vis = block_visible(bx, by, bz, Ti, K, W, H, m.voxel_size, m.depth_min, m.depth_max);
+      vis = block_visible(bx, by, bz, Ti, Kmap, W, H, m.voxel_size, m.depth_min, m.depth_max);
     }
     if (list) {
       const unsigned long long mask = __ballot(vis);

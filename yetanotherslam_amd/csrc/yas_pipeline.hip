@@ -24,7 +24,7 @@ MapView yas_map_view(yas_map* map);
 PosePair* yas_map_pose_dev_mut(yas_map* map);
 int yas_raycast_prepared(yas_raycaster* rc, yas_map* map, hipEvent_t before_march, const hipEvent_t* march_ev);
 float4* yas_raycaster_vmap_dev(yas_raycaster* rc);
-void yas_raycaster_zrange_dev(yas_raycaster* rc, unsigned** zmin, unsigned** zmax, int* ncell);
+void yas_raycaster_zrange_dev(yas_raycaster* rc, unsigned** zmin, unsigned** zmax, unsigned** occ, int* ncell);
 TrackState* yas_tracker_state_dev(yas_tracker* t);
 int yas_tracker_solve_async(yas_tracker* t);
 const double* yas_tracker_result_dev(yas_tracker* t);
@@ -59,6 +59,7 @@ struct FrameBegin {
   TrackState* st;
   unsigned* zmin;
   unsigned* zmax;
+  unsigned* occ;
   int ncell;
   int tiles_x, tiles;  // of the depth conversion
   int image_tiles, depth_tiles;  // of the levels (0 on the first frame)
@@ -76,6 +77,7 @@ __global__ void __launch_bounds__(256) k_frame_begin(FrameBegin a) {
     a.zmin[gid] = __float_as_uint(kZrangeFar);
     a.zmax[gid] = 0u;
   }
+  for (int i = gid; i < kOccWords; i += gridDim.x * blockDim.x) a.occ[i] = 0u;
   if (b == 0) {
     if (threadIdx.x == 0) {
       PosePair p;
@@ -357,7 +359,7 @@ int yas_pipeline_step(yas_pipeline* p, const uint16_t* depth, size_t dpitch, con
     a.pose = yas_map_pose_dev_mut(p->map);
     a.ctr = yas_map_view(p->map).ctr;
     a.st = yas_tracker_state_dev(p->trk);
-    yas_raycaster_zrange_dev(p->rc, &a.zmin, &a.zmax, &a.ncell);
+    yas_raycaster_zrange_dev(p->rc, &a.zmin, &a.zmax, &a.occ, &a.ncell);
     a.tiles_x = (W + 63) / 64;
     a.tiles = a.tiles_x * ((H + 3) / 4);
     a.image_tiles = a.depth_tiles = 0;

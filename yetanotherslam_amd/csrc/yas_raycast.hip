@@ -25,14 +25,16 @@ struct yas_raycaster {
   float4* vmap;
   unsigned* zmin;
   unsigned* zmax;
+  unsigned* occ;  // coarse occupancy of the map cast last
   int* host_ctr;
   yas_map* last_map;
   float* depth;  // VMapToDepth of the last vertex map (lazily allocated)
 };
 
-// The cells before a ray cast, and the map's visible counter.
-__global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zmax, int n, int* ctr) {
+// The cells and the occupancy before a ray cast, and the map's visible counter.
+__global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zmax, int n, unsigned* occ, int* ctr) {
   zrange_init_at(zmin, zmax, n, blockIdx.x, gridDim.x);
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kOccWords; i += gridDim.x * blockDim.x) occ[i] = 0u;
   if (blockIdx.x == 0 && threadIdx.x == 0) ctr[kCtrVisible] = 0;
 }
 
@@ -40,24 +42,27 @@ __global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zm
 // the block list, chunk b % chunks of the cell rows (rows_per each).
 template <class P>
 __global__ void __launch_bounds__(256) k_view(MapView m, P pose, Intr Kmap, Intr K, int W, int H, int cols, int rows,
-                                              unsigned* zmin, unsigned* zmax, int slices, int chunks, int rows_per) {
+                                              unsigned* zmin, unsigned* zmax, unsigned* occ, int slices, int chunks,
+                                              int rows_per) {
   extern __shared__ unsigned lz[];
   const int chunk = blockIdx.x % chunks, r0 = chunk * rows_per;
-  view_scan(m, pose.Tinv(), Kmap, K, W, H, cols, rows, zmin, zmax, lz, blockIdx.x / chunks, slices, r0,
+  view_scan(m, pose.Tinv(), Kmap, K, W, H, cols, rows, zmin, zmax, occ, lz, blockIdx.x / chunks, slices, r0,
             min(rows, r0 + rows_per), chunk == 0);
 }
 
 // The cells of an image too wide for k_view's chunks, straight into memory
-// (after the map's visibility pass).
+// (after the map's visibility pass), and the occupancy.
 __global__ void __launch_bounds__(256) k_zrange(MapView m, const PosePair* pose, Intr K, int cols, int rows,
-                                                unsigned* zmin, unsigned* zmax) {
+                                                unsigned* zmin, unsigned* zmax, unsigned* occ) {
   zrange_at(m, pose, K, cols, rows, zmin, zmax, blockIdx.x, gridDim.x);
+  occ_scan_at(m, occ, blockIdx.x, gridDim.x);
 }
 
 template <class VT, class P>
 __global__ void __launch_bounds__(256) k_march(MapView m, P pose, Intr K, int W, int H, int cols, const float* zmin,
-                                               const float* zmax, float4* vmap, float vsinv, float step_scale) {
-  march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, vmap, vsinv, step_scale, blockIdx.x);
+                                               const float* zmax, const unsigned* occ, float4* vmap, float vsinv,
+                                               float step_scale) {
+  march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, occ, vmap, vsinv, step_scale, blockIdx.x);
 }
 
 // Workgroups of k_view: one per CU.
@@ -69,7 +74,7 @@ constexpr int kViewGroups = 256;
 // visible counter and the cells have been reset on this stream.
 template <class P>
 static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const double* T, const Intr& K, int W, int H,
-                             unsigned* zmin, unsigned* zmax, float4* vmap, hipEvent_t before_march,
+                             unsigned* zmin, unsigned* zmax, unsigned* occ, float4* vmap, hipEvent_t before_march,
                              const hipEvent_t* march_ev) {
   MapView v = yas_map_view(map);
   const int cols = W / 8, rows = H / 8;
@@ -78,14 +83,15 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
     // workgroup a CU in all
     const int most = kViewCells / cols, chunks = (rows + most - 1) / most, rows_per = (rows + chunks - 1) / chunks;
     const int slices = chunks < kViewGroups ? kViewGroups / chunks : 1;
-    hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(256), 2 * sizeof(unsigned) * (size_t)rows_per * cols, s,
-                       v, pose, yas_map_intr(map), K, W, H, cols, rows, zmin, zmax, slices, chunks, rows_per);
+    hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(256),
+                       sizeof(unsigned) * (kOccWords + 2 * (size_t)rows_per * cols), s, v, pose, yas_map_intr(map), K, W, H,
+                       cols, rows, zmin, zmax, occ, slices, chunks, rows_per);
   } else {
     int r = T ? yas_map_visible_async(map, T, W, H) : yas_map_visible_prepared(map, W, H);
     if (r) return r;
     int g = (v.num_blocks + 255) / 256;
     if (g > 2048) g = 2048;
-    hipLaunchKernelGGL(k_zrange, dim3(g), dim3(256), 0, s, v, yas_map_pose_dev(map), K, cols, rows, zmin, zmax);
+    hipLaunchKernelGGL(k_zrange, dim3(g), dim3(256), 0, s, v, yas_map_pose_dev(map), K, cols, rows, zmin, zmax, occ);
   }
   YAS_LAUNCH_CHECK();
   if (before_march) YAS_HIP(hipEventRecord(before_march, s));
@@ -96,15 +102,15 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
   const float* zf = (const float*)zmax;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
-      launch_timed(k_march<VoxI16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxI16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
                    step_scale);
       break;
     case YAS_VOXEL_F16_U16:
-      launch_timed(k_march<VoxF16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxF16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
                    step_scale);
       break;
     default:
-      launch_timed(k_march<VoxF32, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, vmap, vsinv,
+      launch_timed(k_march<VoxF32, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
                    step_scale);
   }
   YAS_LAUNCH_CHECK();
@@ -114,26 +120,26 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
 // A whole ray cast at pose T: the cells and the visible counter reset, then
 // launch_view_march.
 static int launch_raycast_to(yas_map* map, const double T[16], const Intr& K, int W, int H, unsigned* zmin,
-                             unsigned* zmax, float4* vmap) {
+                             unsigned* zmax, unsigned* occ, float4* vmap) {
   hipStream_t s = yas_map_ctx(map)->stream;
   const int ncell = (W / 8) * (H / 8);
-  hipLaunchKernelGGL(k_cells_init, dim3((ncell + 255) / 256), dim3(256), 0, s, zmin, zmax, ncell,
+  hipLaunchKernelGGL(k_cells_init, dim3((ncell + 255) / 256), dim3(256), 0, s, zmin, zmax, ncell, occ,
                      yas_map_view(map).ctr);
   YAS_LAUNCH_CHECK();
   PoseVal pose;
   pose_pair_from(T, pose.p);
-  return launch_view_march(s, map, pose, T, K, W, H, zmin, zmax, vmap, nullptr, nullptr);
+  return launch_view_march(s, map, pose, T, K, W, H, zmin, zmax, occ, vmap, nullptr, nullptr);
 }
 
 // ------------------------------------------------------------------ ray cast without allocation
-// yas_raycast_into keeps its only scratch, the two z-range maps, in this
-// file-scope device array: zmin in the first kScratchCells words, zmax in
-// the next (256 KiB, held on every device the library runs on until the
+// yas_raycast_into keeps its only scratch, the two z-range maps and the coarse
+// occupancy, in this file-scope device array: zmin in the first kScratchCells
+// words, zmax in the next, then the occupancy (268 KiB, held on every device the library runs on until the
 // process ends).  The kernels get its device address, looked up once per
 // device with that device current; the array's name itself is a host-side
 // stand-in and is never passed to a kernel.
 constexpr int kScratchCells = 32768;
-static __device__ __align__(256) unsigned scratch[2 * kScratchCells];
+static __device__ __align__(256) unsigned scratch[2 * kScratchCells + kOccWords];
 
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -161,14 +167,15 @@ static int scratch_on_device(int device, unsigned** out) {
 // `before_march` (optional) is recorded between the view and march kernels.
 int yas_raycast_prepared(yas_raycaster* rc, yas_map* map, hipEvent_t before_march, const hipEvent_t* march_ev) {
   int r = launch_view_march(rc->ctx->stream, map, PoseDev{yas_map_pose_dev(map)}, (const double*)nullptr, rc->K, rc->W,
-                            rc->H, rc->zmin, rc->zmax, rc->vmap, before_march, march_ev);
+                            rc->H, rc->zmin, rc->zmax, rc->occ, rc->vmap, before_march, march_ev);
   if (r) return r;
   rc->last_map = map;
   return YAS_OK;
 }
 
 float4* yas_raycaster_vmap_dev(yas_raycaster* rc) { return rc->vmap; }
-void yas_raycaster_zrange_dev(yas_raycaster* rc, unsigned** zmin, unsigned** zmax, int* ncell) {
+void yas_raycaster_zrange_dev(yas_raycaster* rc, unsigned** zmin, unsigned** zmax, unsigned** occ, int* ncell) {
+  *occ = rc->occ;
   *zmin = rc->zmin;
   *zmax = rc->zmax;
   *ncell = rc->cols * rc->rows;
@@ -205,6 +212,7 @@ int yas_raycaster_create(yas_ctx* ctx, int W, int H, const float K[4], yas_rayca
   hipError_t e = hipMalloc((void**)&rc->vmap, sizeof(float4) * (size_t)W * H);
   if (e == hipSuccess) e = hipMalloc((void**)&rc->zmin, sizeof(unsigned) * rc->cols * rc->rows);
   if (e == hipSuccess) e = hipMalloc((void**)&rc->zmax, sizeof(unsigned) * rc->cols * rc->rows);
+  if (e == hipSuccess) e = hipMalloc((void**)&rc->occ, sizeof(unsigned) * kOccWords);
   if (e == hipSuccess) e = hipHostMalloc((void**)&rc->host_ctr, sizeof(int) * kCtrCount, hipHostMallocDefault);
   if (e != hipSuccess) {
     yas_set_error("yas_raycaster_create: %s", hipGetErrorString(e));
@@ -224,6 +232,7 @@ int yas_raycaster_destroy(yas_raycaster* rc) {
   hipFree(rc->vmap);
   hipFree(rc->zmin);
   hipFree(rc->zmax);
+  hipFree(rc->occ);
   hipFree(rc->depth);
   if (rc->host_ctr) hipHostFree(rc->host_ctr);
   yas_ctx_release(rc->ctx);
@@ -236,7 +245,7 @@ int yas_raycast(yas_raycaster* rc, yas_map* map, const double T[16]) {
   YAS_REQUIRE_ACTIVE(map);
   YAS_HIP(hipSetDevice(rc->ctx->device));
   YAS_REQUIRE(yas_map_ctx(map)->stream == rc->ctx->stream, "yas_raycast: map and ray caster must share a stream");
-  int r = launch_raycast_to(map, T, rc->K, rc->W, rc->H, rc->zmin, rc->zmax, rc->vmap);
+  int r = launch_raycast_to(map, T, rc->K, rc->W, rc->H, rc->zmin, rc->zmax, rc->occ, rc->vmap);
   if (r) return r;
   rc->last_map = map;
   return YAS_OK;
@@ -256,7 +265,8 @@ int yas_raycast_into(yas_map* map, const double T[16], const float K[4], int W, 
   unsigned* zr = nullptr;
   int r = scratch_on_device(ctx->device, &zr);
   if (r) return r;
-  return launch_raycast_to(map, T, make_intr(K), W, H, zr, zr + kScratchCells, (float4*)vmap);
+  return launch_raycast_to(map, T, make_intr(K), W, H, zr, zr + kScratchCells, zr + 2 * kScratchCells,
+                            (float4*)vmap);
 }
 
 int yas_raycaster_vmap(yas_raycaster* rc, float** vmap, size_t* pitch) {

@@ -39,9 +39,11 @@ __global__ void __launch_bounds__(256) k_cells_init(unsigned* zmin, unsigned* zm
 }
 
 // Visibility and z-range cells (view_scan).  Workgroup b: slice b / chunks of
-// the block list, chunk b % chunks of the cell rows (rows_per each).
+// the block list, chunk b % chunks of the cell rows (rows_per each).  A slice
+// has a few hundred blocks at most; the threads are for the cells, cleared and
+// merged (1280x960: 14.7 us with 256, 11.9 us with 1024).
 template <class P>
-__global__ void __launch_bounds__(256) k_view(MapView m, P pose, Intr Kmap, Intr K, int W, int H, int cols, int rows,
+__global__ void __launch_bounds__(1024) k_view(MapView m, P pose, Intr Kmap, Intr K, int W, int H, int cols, int rows,
                                               unsigned* zmin, unsigned* zmax, unsigned* occ, int slices, int chunks,
                                               int rows_per) {
   extern __shared__ unsigned lz[];
@@ -83,7 +85,7 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
     // workgroup a CU in all
     const int most = kViewCells / cols, chunks = (rows + most - 1) / most, rows_per = (rows + chunks - 1) / chunks;
     const int slices = chunks < kViewGroups ? kViewGroups / chunks : 1;
-    hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(256),
+    hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(1024),
                        sizeof(unsigned) * (kOccWords + 2 * (size_t)rows_per * cols), s, v, pose, yas_map_intr(map), K, W, H,
                        cols, rows, zmin, zmax, occ, slices, chunks, rows_per);
   } else {

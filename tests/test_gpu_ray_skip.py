@@ -44,6 +44,7 @@ def _with_intrinsics(m, K, Kr, tmp_path):
     (160, 120, 0.01, 0.03, "f32", (0, 0, 0), 0.1, 900.0),         # 90000 voxels from the origin
     (160, 120, 0.01, 0.03, "f32", (0, 0, 0), 0.1, 9000.0),        # 900000 voxels
     (1280, 960, 0.01, 0.03, "f32", (0.2, 0, -0.3), -0.2, 0.0),    # two chunks of cells
+    (480, 360, 0.01, 0.03, "i16", (-0.2, 0, -0.2), 0.3, 0.0),     # 32 rays a wavefront (64, 16 and 8 above)
     (77832, 8, 0.02, 0.06, "f32", (0, 0, -0.3), 0.0, 0.0),        # 9729 columns of cells
 ])
 def test_ray_cast_equals_the_oracle(gpu, w, h, voxel, trunc, fmt, shift, yaw, origin, tmp_path):

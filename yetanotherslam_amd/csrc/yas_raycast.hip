@@ -63,8 +63,8 @@ __global__ void __launch_bounds__(256) k_zrange(MapView m, const PosePair* pose,
 template <class VT, class P>
 __global__ void __launch_bounds__(256) k_march(MapView m, P pose, Intr K, int W, int H, int cols, const float* zmin,
                                                const float* zmax, const unsigned* occ, float4* vmap, float vsinv,
-                                               float step_scale) {
-  march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, occ, vmap, vsinv, step_scale, blockIdx.x);
+                                               float step_scale, int rows) {
+  march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, occ, vmap, vsinv, step_scale, rows, blockIdx.x);
 }
 
 // Workgroups of k_view: one per CU.
@@ -99,21 +99,22 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
   if (before_march) YAS_HIP(hipEventRecord(before_march, s));
   const float vsinv = (float)(1.0 / (double)v.voxel_size);
   const float step_scale = v.trunc / v.voxel_size;
-  dim3 grid(((W + 15) / 16) * ((H + 15) / 16));
+  const int mr = march_rows(W, H);
+  dim3 grid(march_tiles(W, H, mr));
   const float* zn = (const float*)zmin;
   const float* zf = (const float*)zmax;
   switch (v.format) {
     case YAS_VOXEL_I16_U8:
       launch_timed(k_march<VoxI16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
-                   step_scale);
+                   step_scale, mr);
       break;
     case YAS_VOXEL_F16_U16:
       launch_timed(k_march<VoxF16, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
-                   step_scale);
+                   step_scale, mr);
       break;
     default:
       launch_timed(k_march<VoxF32, P>, grid, dim3(256), s, march_ev, v, pose, K, W, H, cols, zn, zf, occ, vmap, vsinv,
-                   step_scale);
+                   step_scale, mr);
   }
   YAS_LAUNCH_CHECK();
   return YAS_OK;

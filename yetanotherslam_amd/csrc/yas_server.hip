@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(256) k_s_march(const StreamDev* streams, const
   const YAS_CONSTANT Slot& sl = ctab.slot[slot];
   const YAS_CONSTANT StreamDev& S = ((const YAS_CONSTANT StreamDev*)streams)[sl.stream];
   march_tile_at<VT>(S.m, S.pose->T, S.pose->Tinv, S.K, S.W, S.H, S.cols, (const float*)S.zmin, (const float*)S.zmax, nullptr, S.vmap,
-                    S.vsinv, S.step_scale, tile);
+                    S.vsinv, S.step_scale, 8, tile);
 }
 
 // Tracker inputs, two launches per pyramid level (the per-pixel functions

@@ -87,15 +87,15 @@ def cpu_baseline(p, K, depth, rgb, budget_s=12.0, all_cores=False):
 # carried here, keyed by the run they were measured on: (warmup, steps),
 # i.e. the timed frames warmup+1 .. warmup+steps of the sequence.  Other runs
 # report no traffic figure.
-TRAFFIC_BYTES = {(10, 290): {"k_march": 54.42e6, "k_integrate": 108.93e6, "k_alloc": 4.45e6},
-                 (5, 20): {"k_march": 38.42e6, "k_integrate": 87.36e6, "k_alloc": 4.42e6}}
+TRAFFIC_BYTES = {(10, 290): {"k_march": 53.07e6, "k_integrate": 107.68e6, "k_alloc": 3.23e6},
+                 (5, 20): {"k_march": 38.00e6, "k_integrate": 85.43e6, "k_alloc": 3.18e6}}
 
 # VALU instructions (wavefront instructions summed over the GPU) per launch
 # of the ray march, from a rocprofv3 SQ_INSTS_VALU pass over this script's
 # own run (profiles/k_march_640x480_sq_counters.md), keyed as above.  The
 # march is bound by the latency of its slowest rays' dependent reads, so
 # neither HBM nor VALU issue saturates; both fractions are reported.
-VALU_INSTS = {(10, 290): {"k_march": 22.68e6}, (5, 20): {"k_march": 16.21e6}}
+VALU_INSTS = {(10, 290): {"k_march": 20.18e6}, (5, 20): {"k_march": 15.21e6}}
 # one wave64 VALU instruction per SIMD every 4 cycles: 256 CUs x 4 SIMDs x 2.4 GHz / 4
 VALU_PEAK_G = 614.4
 

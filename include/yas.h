@@ -337,9 +337,10 @@ int yas_raycast(yas_raycaster* rc, yas_map* map, const double T_map_cam[16]);
  * harnesses that forbid hipMalloc.  The map (its visible-block list and
  * pose) and the dense W*H float4 vertex map `vmap` (pitch = 16*W) are the
  * caller's; intrinsics K = {fx, fy, cx, cy} as yas_raycaster_create.  The
- * only scratch, the two 1/8-resolution z-range maps, is a static device
- * array of 32768 cells per map (256 KiB per device, held until the process
- * ends): (W/8)*(H/8) > 32768 is rejected with YAS_E_INVALID.  Every call on a
+ * only scratch, the two 1/8-resolution z-range maps of 32768 cells each and
+ * the blocks' coarse occupancy, is a static device array (260 KiB per device,
+ * held until the process ends): (W/8)*(H/8) > 32768 is rejected with
+ * YAS_E_INVALID.  Every call on a
  * device shares that array, so calls that overlap on one GPU (on different
  * streams) race.  Asynchronous on the map's stream; results are those of
  * yas_raycast with a ray caster of the same size and intrinsics. */

@@ -137,10 +137,10 @@ static int launch_raycast_to(yas_map* map, const double T[16], const Intr& K, in
 // ------------------------------------------------------------------ ray cast without allocation
 // yas_raycast_into keeps its only scratch, the two z-range maps and the coarse
 // occupancy, in this file-scope device array: zmin in the first kScratchCells
-// words, zmax in the next, then the occupancy (268 KiB, held on every device the library runs on until the
-// process ends).  The kernels get its device address, looked up once per
-// device with that device current; the array's name itself is a host-side
-// stand-in and is never passed to a kernel.
+// words, zmax in the next, then the occupancy (260 KiB, held on every device
+// the library runs on until the process ends).  The kernels get its device
+// address, looked up once per device with that device current; the array's
+// name itself is a host-side stand-in and is never passed to a kernel.
 constexpr int kScratchCells = 32768;
 static __device__ __align__(256) unsigned scratch[2 * kScratchCells + kOccWords];
 

@@ -153,9 +153,9 @@ __device__ inline void zrange_lds_at(const MapView& m, const PosePair* pose, con
 // reduce in LDS too, in chunks.
 constexpr int kViewCells = 9728;  // cells of a chunk: 76 KB and 4 KB, two workgroups a CU
 
-__device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& Kmap, const Intr& K, int W, int H, int cols, int rows,
-                                 unsigned* zmin, unsigned* zmax, unsigned* occ, unsigned* lds, int slice, int slices,
-                                 int r0, int r1, bool list) {
+__device__ inline void view_scan(const MapView& m, const PoseF& Ti, const Intr& Kmap, const Intr& K, int W, int H,
+                                 int cols, int rows, unsigned* zmin, unsigned* zmax, unsigned* occ, unsigned* lds,
+                                 int slice, int slices, int r0, int r1, bool list) {
   const int c0 = r0 * cols, nc = (r1 - r0) * cols;
   unsigned* locc = lds;
   unsigned* lmin = lds + kOccWords;

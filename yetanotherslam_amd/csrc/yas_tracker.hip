@@ -112,10 +112,10 @@ __global__ void __launch_bounds__(256) k_step_pass1(Level L, TrackBufs B, StepAr
 }
 // The whole solve in one launch (yas_solve_dev.hpp).  1024 threads a
 // workgroup, so 128 registers a lane; one workgroup per CU.  Bound by the
-// chain of an iteration (20 us at 640x480, 16.5 us at any small size): pixel
-// terms 3-5 us (VALU issue, four wavefronts a SIMD), statistics 1.5 us, three
-// messages between workgroups of about 1.3 us each, the step 4.3 us.  The
-// launch-per-pass iteration took 27 us (24 us at small sizes).
+// chain of an iteration (15.8 us at 640x480 with both terms, 7.4 us at 320x240
+// with depth alone): the pixels' gathers, the wavefronts' sums and the fold,
+// two or three messages between workgroups of about 1.4 us each, the step
+// 2.4 us.  The launch-per-pass iteration took 27 us (24 us at small sizes).
 template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(kSolveThreads) k_solve(SolveArgs a) {
   solve_body<ICP, RGB>(solve_lds(), a);

@@ -283,7 +283,8 @@ __device__ inline void integrate_waves(const MapView& m, const PoseF& Ti, const 
     const unsigned long long un = __ballot(unobserved), fr = __ballot(free_space);
     if (lane == 0) {
       const int f = (un == ~0ull ? kBlockUnobserved : 0) | (fr == ~0ull ? kBlockFree : 0);
-      m.slots[m.block_slot[blk]].flags = f;
+      const int slot = m.block_slot[blk];
+      if (slot >= 0) m.slots[slot].flags = f;
     }
   }
 }

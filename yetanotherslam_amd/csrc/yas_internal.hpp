@@ -352,7 +352,7 @@ enum : int { kBlockUnobserved = 1, kBlockFree = 2 };  // all w == 0 / all w > 0 
 
 struct MapView {
   HashSlot* slots;                 // [num_buckets]
-  int* block_slot;                 // [num_blocks] hash slot of each pool block
+  int* block_slot;                 // [num_blocks] hash slot of each pool block, -1 for one that the table had no room for
   unsigned long long* block_keys;  // [num_blocks]
   void* voxels;                    // [num_blocks * 512] of the storage type
   int* visible;                    // [num_blocks] pool indices of visible blocks

@@ -151,7 +151,10 @@ __global__ void __launch_bounds__(256) k_reset_used(MapView m, int words16 /* 16
   if (na > m.num_blocks) {
     for (int i = t; i < m.num_buckets; i += nt) m.slots[i] = e;
   } else {
-    for (int i = t; i < n; i += nt) m.slots[m.block_slot[i]] = e;
+    for (int i = t; i < n; i += nt) {
+      const int slot = m.block_slot[i];
+      if (slot >= 0) m.slots[slot] = e;
+    }
   }
   uint4* v = (uint4*)m.voxels;
   for (size_t i = t; i < (size_t)n * words16; i += nt) v[i] = make_uint4(0u, 0u, 0u, 0u);

@@ -39,11 +39,12 @@ __global__ void __launch_bounds__(256) k_zero_words(uint32_t* p, size_t n) {
 // Gather each pool block's summary flags from its hash slot.
 __global__ void __launch_bounds__(256) k_gather_flags(const HashSlot* slots, const int* block_slot, int n, int* flags) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) flags[i] = slots[block_slot[i]].flags;
+  if (i < n) flags[i] = block_slot[i] >= 0 ? slots[block_slot[i]].flags : 0;
 }
 
 // Insert pool blocks [0, n) (distinct keys) into an empty table: slot =
-// first free slot probing from the reference hash's home slot.
+// first free slot probing from the reference hash's home slot; -1 where there
+// is none within the probe limit (a file with fewer buckets than blocks).
 __global__ void __launch_bounds__(256) k_rehash(MapView m, const int* flags, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -62,6 +63,7 @@ __global__ void __launch_bounds__(256) k_rehash(MapView m, const int* flags, int
     }
     slot = slot + 1 == m.num_buckets ? 0 : slot + 1;
   }
+  m.block_slot[i] = -1;
   atomicOr(&m.ctr[kCtrFlags], kFlagProbeLimit);
 }
 
@@ -188,7 +190,8 @@ __global__ void __launch_bounds__(256) k_merge_fuse(MapView dst, MapView src, Po
     const unsigned long long un = __ballot(unobserved), fr = __ballot(free_space);
     if (lane == 0) {
       const int f = (un == ~0ull ? kBlockUnobserved : 0) | (fr == ~0ull ? kBlockFree : 0);
-      dst.slots[dst.block_slot[w]].flags = f;
+      const int slot = dst.block_slot[w];
+      if (slot >= 0) dst.slots[slot].flags = f;
     }
   }
 }

@@ -848,13 +848,15 @@ int yas_mesher_create(yas_ctx* ctx, int max_triangles, yas_mesher** out) {
   if (e == hipSuccess) e = hipMalloc((void**)&me->normals, sizeof(float) * 9 * (size_t)max_triangles);
   if (e == hipSuccess) e = hipHostMalloc((void**)&me->total, sizeof(McTotals), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc((void**)&me->done, sizeof(unsigned));
-  if (e == hipSuccess) e = hipMemset(me->done, 0, sizeof(unsigned));
+  // on the context's stream, which the null stream need not be in order with
+  if (e == hipSuccess) e = hipMemsetAsync(me->done, 0, sizeof(unsigned), ctx->stream);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&me->cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
   if (e != hipSuccess) {
     yas_set_error("yas_mesher_create: %s", hipGetErrorString(e));
     yas_mesher_destroy(me);
     return YAS_E_HIP;
   }
+  *me->total = McTotals{0, 0, 0};
   *out = me;
   return YAS_OK;
 }

@@ -107,13 +107,10 @@ yas_ctx* yas_ctx_retain(yas_ctx* c) {
   return c;
 }
 
-void yas_solve_forget_stream(int device, hipStream_t s);
-
 void yas_ctx_release(yas_ctx* c) {
   if (!c || c->refs.fetch_sub(1) != 1) return;
   hipSetDevice(c->device);
   hipStreamSynchronize(c->stream);
-  yas_solve_forget_stream(c->device, c->stream);
   if (c->own_stream) hipStreamDestroy(c->stream);
   delete c;
 }

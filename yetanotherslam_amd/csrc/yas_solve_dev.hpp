@@ -59,7 +59,8 @@ struct SolveXchg {
 // A solve's result in host memory, for the caller that waits for it.
 struct HostState {
   TrackState s;
-  int ok;  // the solve completed
+  int ok;          // the solve completed
+  unsigned ended;  // number of the tracker's last one-launch solve that has ended
 };
 
 struct SolveArgs {

@@ -120,9 +120,11 @@ template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(kSolveThreads) k_solve(SolveArgs a) {
   solve_body<ICP, RGB>(solve_lds(), a);
 }
-// Takes a solve whose workgroups did not meet; nothing to do otherwise.
+// Takes a solve whose workgroups did not meet; nothing to do otherwise, but to
+// say in host memory that solve `number` has ended.
 template <bool ICP, bool RGB>
-__global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a) {
+__global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a, HostState* host, unsigned number) {
+  if (threadIdx.x == 0) __hip_atomic_store(&host->ended, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   solve_rescue<ICP, RGB>(a);
 }
 // All levels of an image, a depth image or a model in one launch (yas_frame_dev.hpp).
@@ -160,6 +162,7 @@ struct yas_tracker {
   HostState* host_st;
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
+  unsigned solves;               // one-launch solves launched
   float sin2_max, dist2_max;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
   float* raw_image;  // intensity uploaded by the host-image setters
@@ -302,19 +305,24 @@ static int solve_by_passes(yas_tracker* t) {
 
 // Whether this solve may run as one launch (k_solve): every workgroup must
 // find a CU at once, so only one stream's solves do at a time.  A stream
-// other than the last one's takes over once that one is idle; until then its
-// solves run as separate passes.  So do solves recorded into a graph, whose
-// replays nothing here orders.
+// other than the last one's takes over once that solve has ended, which its
+// tracker's host memory says; until then its solves run as separate passes.
+// (Asking the runtime whether the other stream is idle breaks a capture in the
+// global mode that any thread may have begun.)  Solves recorded into a graph,
+// whose replays nothing here orders, run as separate passes too.
 static std::mutex g_solve_mu;
 static struct {
-  bool used;
-  hipStream_t stream;
+  yas_tracker* owner;  // of the last one-launch solve; null when it is gone
+  hipStream_t stream;  // only compared
 } g_solve_last[kMaxSolveDevices];
 
-void yas_solve_forget_stream(int device, hipStream_t s) {
+static bool solve_ended(const yas_tracker* t) {
+  return __atomic_load_n(&t->host_st->ended, __ATOMIC_ACQUIRE) == t->solves;
+}
+static void forget_solves(const yas_tracker* t) {
   std::lock_guard<std::mutex> lk(g_solve_mu);
-  if (device >= 0 && device < kMaxSolveDevices && g_solve_last[device].used && g_solve_last[device].stream == s)
-    g_solve_last[device].used = false;
+  for (auto& last : g_solve_last)
+    if (last.owner == t) last.owner = nullptr;
 }
 
 static bool solve_fits(int device, const void* kernel, int grid) {
@@ -364,11 +372,15 @@ static SolveArgs solve_args(yas_tracker* t) {
   a.wait_ticks = t->wait_ticks;
   return a;
 }
-static void launch_rescue(const SolveArgs& a, hipStream_t s) {
+static void launch_rescue(yas_tracker* t) {
+  const SolveArgs a = solve_args(t);
+  HostState* h = t->host_st;
+  hipStream_t s = t->ctx->stream;
   const dim3 one(1), threads(256);
-  if (a.mode == YAS_TRACK_RGBD) hipLaunchKernelGGL((k_solve_rescue<true, true>), one, threads, 0, s, a);
-  else if (a.mode == YAS_TRACK_DEPTH) hipLaunchKernelGGL((k_solve_rescue<true, false>), one, threads, 0, s, a);
-  else hipLaunchKernelGGL((k_solve_rescue<false, true>), one, threads, 0, s, a);
+  if (a.mode == YAS_TRACK_RGBD) hipLaunchKernelGGL((k_solve_rescue<true, true>), one, threads, 0, s, a, h, t->solves);
+  else if (a.mode == YAS_TRACK_DEPTH)
+    hipLaunchKernelGGL((k_solve_rescue<true, false>), one, threads, 0, s, a, h, t->solves);
+  else hipLaunchKernelGGL((k_solve_rescue<false, true>), one, threads, 0, s, a, h, t->solves);
 }
 
 // The solve in one launch from `init` (null: the state's pose), its result to
@@ -389,12 +401,8 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
       !solve_fits(device, kernel, grid)) return YAS_OK;
   std::lock_guard<std::mutex> lk(g_solve_mu);
   auto& last = g_solve_last[device];
-  if (last.used && last.stream != s && (is_capturing(last.stream) || hipStreamQuery(last.stream) != hipSuccess)) {
-    (void)hipGetLastError();  // hipErrorNotReady is no failure
-    return YAS_OK;
-  }
-  last.used = true;
-  last.stream = s;
+  // (the per-thread stream's handle is not one stream)
+  if (last.owner && (last.stream != s || s == hipStreamPerThread) && !solve_ended(last.owner)) return YAS_OK;
   SolveArgs a = solve_args(t);
   if (init) a.init = *init;
   a.has_init = init != nullptr;
@@ -404,6 +412,9 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
   else if (mode == YAS_TRACK_DEPTH) hipLaunchKernelGGL((k_solve<true, false>), dim3(grid), threads, 0, s, a);
   else hipLaunchKernelGGL((k_solve<false, true>), dim3(grid), threads, 0, s, a);
   YAS_LAUNCH_CHECK();
+  last.owner = t;
+  last.stream = s;
+  t->solves++;
   done = true;
   return YAS_OK;
 }
@@ -413,7 +424,7 @@ int yas_tracker_solve_async(yas_tracker* t) {
   int rc = solve_in_one(t, nullptr, nullptr, done);
   if (rc) return rc;
   if (!done) return solve_by_passes(t);
-  launch_rescue(solve_args(t), t->ctx->stream);
+  launch_rescue(t);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
@@ -430,12 +441,13 @@ static int solve_and_wait(yas_tracker* t, const Mat44& init) {
   if (rc) return rc;
   if (done) {
     YAS_HIP(hipStreamSynchronize(s));
+    __atomic_store_n(&t->host_st->ended, t->solves, __ATOMIC_RELEASE);
     if (t->host_st->ok) return YAS_OK;
   }
   hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, s, t->st, init);
   YAS_LAUNCH_CHECK();
   if (done) {
-    launch_rescue(solve_args(t), s);
+    launch_rescue(t);
     YAS_LAUNCH_CHECK();
   } else if ((rc = solve_by_passes(t))) {
     return rc;
@@ -597,6 +609,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   YAS_HIP(hipMemsetAsync(t->st, 0, sizeof(TrackState), ctx->stream));
   YAS_HIP(hipMemsetAsync(t->st2, 0, sizeof(TrackState), ctx->stream));
   YAS_HIP(hipMemsetAsync(t->xchg, 0, sizeof(SolveXchg), ctx->stream));
+  std::memset(t->host_st, 0, sizeof(HostState));
   int rc = yas_tracker_init_identity_async(t);
   if (rc) {
     yas_tracker_destroy(t);
@@ -610,6 +623,7 @@ int yas_tracker_destroy(yas_tracker* t) {
   if (!t) return YAS_OK;
   hipSetDevice(t->ctx->device);
   hipStreamSynchronize(t->ctx->stream);
+  forget_solves(t);
   for (int l = 0; l < kMaxLevels; ++l) {
     for (float* p : {t->cur_int[l], t->ref_int[l], t->gx[l], t->gy[l], t->cur_inv[l], t->ref_inv[l]}) hipFree(p);
     for (float4* p : {t->cur_v[l], t->cur_n[l], t->ref_v[l], t->ref_n[l]}) hipFree(p);

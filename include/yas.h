@@ -457,6 +457,10 @@ int yas_tracker_step_sums(yas_tracker* trk, int level, const double T[16], int k
  * row-major 6x6 float matrices, b n float 6-vectors, x receives n double
  * 6-vectors (host arrays). Synchronous. */
 int yas_tracker_solve6(yas_ctx* ctx, const float* H, const float* b, double* x, int n);
+/* The bound of the waits inside a one-launch solve, in ticks of the device's
+ * 100 MHz clock (test access; 2000000 by default).  0 makes every wait that
+ * finds its words missing at the first look give up. */
+int yas_tracker_set_wait_ticks(yas_tracker* trk, unsigned long long ticks);
 /* Device pointer and pitch of one pyramid image (test access):
  * which = 0 current intensity, 1 reference intensity, 2 gx, 3 gy,
  * 4 current inverse depth, 5 reference inverse depth (float);

@@ -461,6 +461,11 @@ int yas_tracker_solve6(yas_ctx* ctx, const float* H, const float* b, double* x, 
  * 100 MHz clock (test access; 2000000 by default).  0 makes every wait that
  * finds its words missing at the first look give up. */
 int yas_tracker_set_wait_ticks(yas_tracker* trk, unsigned long long ticks);
+/* How many of this tracker's solves (GetTransform, pipeline frames) ran as
+ * one launch, ran out of a wait as one launch and were taken again, and ran as
+ * separate passes from the start; the result is the same either way.
+ * Synchronous. */
+int yas_tracker_solve_routes(yas_tracker* trk, int routes[3]);
 /* Device pointer and pitch of one pyramid image (test access):
  * which = 0 current intensity, 1 reference intensity, 2 gx, 3 gy,
  * 4 current inverse depth, 5 reference inverse depth (float);

@@ -58,3 +58,97 @@ def test_steps_beside_a_capture(gpu):
         assert float(x[0]) == 2.0 * (k + 1)
     for pl, _ in pls:
         assert np.array_equal(_poses(pl), want)
+
+
+DEFAULT_TICKS = 2000000
+
+
+def _ticks(h, ticks):
+    native.call("yas_tracker_set_wait_ticks", h, ticks)
+
+
+def _routes(h):
+    r = (ctypes.c_int * 3)()
+    native.call("yas_tracker_solve_routes", h, r)
+    return list(r)  # in one launch, lost, passes
+
+
+def _tracker(w, h, mode, iters=(10, 5, 3), ctx=None):
+    p = synth.params(width=w, height=h, theta0=0.7)
+    p.noise_k, p.step = 0.0002, 0.004
+    trk = rf.RGBDTracking(w, h, synth.intrinsics(p), len(iters), iters, mode, (0.1, 0.1, 1.0, 1.0), ctx=ctx)
+    keep = []
+    for t in range(2):
+        d, c = synth.frame(p, t)[:2]
+        z = to_dev(d.astype(np.float32) * np.float32(0.001))
+        g = to_dev(c.astype(np.float32) @ np.array([0.299, 0.587, 0.114], np.float32))
+        keep.append((z, g))
+        (trk.SetReferenceDepth, trk.SetTrackingDepth)[t](z)
+        (trk.SetReferenceImage, trk.SetTrackingImage)[t](g)
+    trk._keep = keep
+    return trk
+
+
+def _solve(trk):
+    T, st = trk.GetTransform(swap=False)
+    return T, (st.good, st.icp_inliers, st.rgb_inliers, np.float32(st.last_error).tobytes())
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("w,h,iters", [(32, 24, (4,)), (164, 124, (4, 2, 2)), (644, 484, (3, 2, 1)), (1280, 968, (2, 1))])
+def test_a_solve_is_one_launch_and_a_lost_one_is_taken_again(gpu, w, h, iters, mode):
+    trk = _tracker(w, h, mode, iters)
+    T, st = _solve(trk)
+    assert _routes(trk.h) == [1, 0, 0]
+    if w == 32:  # one workgroup waits for itself alone
+        return
+    _ticks(trk.h, 0)
+    Tl, sl = _solve(trk)
+    assert _routes(trk.h) == [1, 1, 0]
+    _ticks(trk.h, DEFAULT_TICKS)
+    T2, s2 = _solve(trk)
+    assert _routes(trk.h) == [2, 1, 0]
+    assert np.array_equal(T, Tl) and np.array_equal(T, T2) and st == sl == s2
+
+
+def test_a_stream_beside_a_busy_one_takes_the_passes(gpu):
+    import torch
+    s = [torch.cuda.Stream() for _ in range(2)]
+    trks = []
+    for q in s:
+        with torch.cuda.stream(q):
+            trks.append(_tracker(320, 240, 2, ctx=rf.Context()))
+    with torch.cuda.stream(s[0]):
+        pl, fr = _pipeline(ctx=trks[0].ctx)
+    want = _solve(trks[1])
+    x = torch.zeros(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+    pl.step(*fr[0])
+    with torch.cuda.stream(s[0]):
+        for _ in range(200):  # some 20 ms, then a solve
+            x.add_(1.0)
+    pl.step(*fr[1])
+    got = _solve(trks[1])
+    assert _routes(trks[1].h) == [1, 0, 1]
+    torch.cuda.synchronize()
+    again = _solve(trks[1])
+    assert _routes(trks[1].h) == [2, 0, 1]
+    for g in (got, again):
+        assert np.array_equal(g[0], want[0]) and g[1] == want[1]
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_queued_solves_that_are_lost_are_rescued(gpu, mode):
+    """A pipeline with the bound at 0 in some frames: the rescue that follows
+    each queued solve takes those, with the same bits, and no others."""
+    lost = (2, 3, 6)
+    ref, frames = _pipeline(mode=mode)
+    pl, _ = _pipeline(mode=mode, n=1)
+    h = ctypes.c_void_p()
+    native.call("yas_pipeline_tracker", pl.h, ctypes.byref(h))
+    for i, f in enumerate(frames):
+        ref.step(*f)
+        _ticks(h, 0 if i in lost else DEFAULT_TICKS)
+        pl.step(*f)
+        assert np.array_equal(pl.pose(i)[0], ref.pose(i)[0]) and pl.pose(i)[1] == ref.pose(i)[1], i
+    assert _routes(h) == [len(frames) - 1 - len(lost), len(lost), 0]

@@ -49,7 +49,8 @@ constexpr int kSolveBatch = 2;                    // slots of a thread whose row
 struct SolveXchg {
   unsigned epoch;  // of the last iteration of the last solve
   int ok;          // set when a solve completes, cleared by k_solve_rescue
-  int pad[30];
+  unsigned lost;   // solves that k_solve_rescue took
+  int pad[29];
   unsigned long long pose[32];  // float pose (12) and warp (12) of the next iteration
   unsigned long long stat[kRedGroups][4];
   unsigned long long icp[kRedGroups][32];
@@ -61,6 +62,7 @@ struct HostState {
   TrackState s;
   int ok;          // the solve completed
   unsigned ended;  // number of the tracker's last one-launch solve that has ended
+  unsigned lost;   // its one-launch solves whose workgroups did not meet
 };
 
 struct SolveArgs {

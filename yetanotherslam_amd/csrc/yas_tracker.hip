@@ -121,10 +121,16 @@ __global__ void __launch_bounds__(kSolveThreads) k_solve(SolveArgs a) {
   solve_body<ICP, RGB>(solve_lds(), a);
 }
 // Takes a solve whose workgroups did not meet; nothing to do otherwise, but to
-// say in host memory that solve `number` has ended.
+// say in host memory that solve `number` has ended (and how many were lost).
 template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a, HostState* host, unsigned number) {
-  if (threadIdx.x == 0) __hip_atomic_store(&host->ended, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) {
+    if (!a.x->ok) {
+      a.x->lost++;
+      __hip_atomic_store(&host->lost, a.x->lost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __hip_atomic_store(&host->ended, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
   solve_rescue<ICP, RGB>(a);
 }
 // All levels of an image, a depth image or a model in one launch (yas_frame_dev.hpp).
@@ -163,6 +169,7 @@ struct yas_tracker {
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
   unsigned solves;               // one-launch solves launched
+  unsigned by_passes;            // solves that were separate passes from the start
   float sin2_max, dist2_max;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
   float* raw_image;  // intensity uploaded by the host-image setters
@@ -250,6 +257,7 @@ static int launch_iteration(yas_tracker* t, int l, bool icp, bool rgb, bool do_s
 // i - 1 and writes the other one, and the ICP partial rows alternate the
 // same way, since that pass 1 reads the previous rows while writing its own.
 static int solve_by_passes(yas_tracker* t) {
+  t->by_passes++;
   const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
   hipStream_t s = t->ctx->stream;
   TrackState* S[2] = {t->st, t->st2};
@@ -457,14 +465,26 @@ static int solve_and_wait(yas_tracker* t, const Mat44& init) {
   return YAS_OK;
 }
 
-// The bound of the one-launch solve's waits, for tests that want one to run
-// out: 0 makes every wait that finds its words missing at the first look
-// give up.
-extern "C" int yas_tracker_set_wait_ticks(yas_tracker* t, unsigned long long ticks) {
+extern "C" {
+
+int yas_tracker_set_wait_ticks(yas_tracker* t, unsigned long long ticks) {
   YAS_REQUIRE(t, "null tracker");
   t->wait_ticks = ticks;
   return YAS_OK;
 }
+
+int yas_tracker_solve_routes(yas_tracker* t, int routes[3]) {
+  YAS_REQUIRE(t && routes, "yas_tracker_solve_routes: null argument");
+  YAS_HIP(hipSetDevice(t->ctx->device));
+  YAS_HIP(hipStreamSynchronize(t->ctx->stream));
+  const unsigned lost = __atomic_load_n(&t->host_st->lost, __ATOMIC_ACQUIRE);
+  routes[0] = (int)(t->solves - lost);
+  routes[1] = (int)lost;
+  routes[2] = (int)t->by_passes;
+  return YAS_OK;
+}
+
+}  // extern "C"
 
 int yas_tracker_init_identity_async(yas_tracker* t) {
   hipLaunchKernelGGL(k_track_init_identity, dim3(1), dim3(64), 0, t->ctx->stream, t->st);

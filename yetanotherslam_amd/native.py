@@ -145,6 +145,7 @@ SIGNATURES = {
     "yas_tracker_step_sums": (I, [P, I, P, I, P, P]),
     "yas_tracker_solve6": (I, [P, P, P, P, I]),
     "yas_tracker_set_wait_ticks": (I, [P, ctypes.c_ulonglong]),
+    "yas_tracker_solve_routes": (I, [P, P]),
     "yas_tracker_level": (I, [P, I, I, PP, ctypes.POINTER(SZ), PI, PI]),
     "yas_depth_u16_to_f32": (I, [P, P, SZ, P, SZ, I, I, F]),
     "yas_rgb_to_intensity": (I, [P, P, SZ, P, SZ, I, I, I]),

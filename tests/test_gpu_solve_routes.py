@@ -152,3 +152,15 @@ def test_queued_solves_that_are_lost_are_rescued(gpu, mode):
         pl.step(*f)
         assert np.array_equal(pl.pose(i)[0], ref.pose(i)[0]) and pl.pose(i)[1] == ref.pose(i)[1], i
     assert _routes(h) == [len(frames) - 1 - len(lost), len(lost), 0]
+
+
+def test_many_coarse_iterations_are_no_time_out(gpu):
+    """Workgroups without work on the coarse level wait for all of its
+    iterations together, far longer than the bound that holds for one."""
+    trk = _tracker(320, 240, 2, (1, 6000))
+    T, st = _solve(trk)
+    assert _routes(trk.h) == [1, 0, 0]
+    _ticks(trk.h, 0)
+    Tl, sl = _solve(trk)
+    assert _routes(trk.h) == [1, 1, 0]
+    assert np.array_equal(T, Tl) and st == sl

@@ -162,11 +162,14 @@ __device__ inline float word_value(unsigned long long w) { return __builtin_bit_
 // The values of the N words at byte offsets at(i) from `base` (those with
 // want(i), 0 for the others, which must be readable too) once all carry
 // `epoch`; false when the wait's bound passes first.  All words are loaded
-// together.
-template <int N, class P, class W>
+// together.  STEPS (one word): the bound begins again whenever the word's epoch
+// has changed, for a workgroup that waits for a level's iterations together.
+template <int N, bool STEPS = false, class P, class W>
 __device__ inline bool wait_words(const void* base, P at, W want, unsigned epoch, unsigned long long ticks,
                                   float (&out)[N]) {
+  static_assert(!STEPS || N == 1, "the epoch of one word");
   unsigned long long t0 = 0;
+  unsigned seen = 0;
   for (unsigned looks = 0;; ++looks) {
     unsigned long long w[N];
 #pragma unroll
@@ -182,7 +185,8 @@ __device__ inline bool wait_words(const void* base, P at, W want, unsigned epoch
     const unsigned every = ticks ? 31u : 0u;
     if ((looks & every) == every) {  // the clock is read at every 32nd look
       const unsigned long long now = wall_clock64();
-      if (looks == every) t0 = now;
+      if (looks == every || (STEPS && (unsigned)(w[0] >> 32) != seen)) t0 = now;
+      if (STEPS) seen = (unsigned)(w[0] >> 32);
       if (now - t0 >= ticks) return false;
     }
   }
@@ -727,7 +731,7 @@ __device__ inline void solve_body(SolveLds& S, const SolveArgs& a) {
         const int w = fresh_tid();
         if (w < 64) {
           float v[1];
-          const bool ok = wait_words<1>(a.x->pose, [&](int) { return (w & 31) * 8; }, [&](int) { return w < (RGB ? 24 : 12); },
+          const bool ok = wait_words<1, true>(a.x->pose, [&](int) { return (w & 31) * 8; }, [&](int) { return w < (RGB ? 24 : 12); },
                                         epoch, a.wait_ticks, v);
           if (!ok) S.lost = 1;
           if (w < 12) S.pose[w] = v[0];

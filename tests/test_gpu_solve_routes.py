@@ -164,3 +164,54 @@ def test_many_coarse_iterations_are_no_time_out(gpu):
     Tl, sl = _solve(trk)
     assert _routes(trk.h) == [1, 1, 0]
     assert np.array_equal(T, Tl) and st == sl
+
+
+def test_after_a_lost_solve_come_passes(gpu):
+    """A solve that waits in vain is not tried again each time: 64 solves are
+    separate passes, 128 after the next loss, and 64 again once one completes."""
+    trk = _tracker(164, 124, 0, (2, 1, 1))
+    T, st = _solve(trk)
+    done, lost, passes = 1, 0, 0
+
+    def solve(n=1):
+        for _ in range(n):
+            got = _solve(trk)
+            assert np.array_equal(got[0], T) and got[1] == st
+
+    _ticks(trk.h, 0)
+    for n in (64, 128):
+        solve(1 + n)
+        lost, passes = lost + 1, passes + n
+        assert _routes(trk.h) == [done, lost, passes]
+    _ticks(trk.h, DEFAULT_TICKS)
+    solve(3)
+    done += 3
+    assert _routes(trk.h) == [done, lost, passes]
+    _ticks(trk.h, 0)
+    solve(1 + 64 + 1)
+    assert _routes(trk.h) == [done, lost + 2, passes + 64]
+
+
+@pytest.mark.parametrize("wait", [True, False])
+def test_after_a_rescued_frame_come_passes(gpu, wait):
+    """The same where the solves are queued: the loss is known once the frame
+    has run, and frames queued before that are rescued too."""
+    ref, frames = _pipeline()
+    pl, _ = _pipeline(n=1)
+    h = ctypes.c_void_p()
+    native.call("yas_pipeline_tracker", pl.h, ctypes.byref(h))
+    _ticks(h, 0)
+    for i, f in enumerate(frames):
+        ref.step(*f)
+        pl.step(*f)
+        if wait:
+            pl.pose(i)
+    assert np.array_equal(_poses(pl), _poses(ref))
+    done, lost, passes = _routes(h)
+    assert done == 0 and lost + passes == len(frames) - 1 and lost >= 1
+    if wait:
+        assert lost == 1
+    for i in range(8):
+        pl.step(*frames[6 - i % 2])
+        pl.pose(len(frames) + i)
+    assert _routes(h)[1] == lost  # still by passes, once, however many were lost together

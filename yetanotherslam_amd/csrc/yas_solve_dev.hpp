@@ -31,8 +31,9 @@
 // leaves, the tracker's state stays as it was before the solve, and
 // k_solve_rescue takes the whole solve in one workgroup with the
 // launch-per-pass code (the same sums, so the same bits).  It follows each
-// solve on the stream, except where the caller waits for the solve: that one
-// sees in host memory whether it completed and launches the rescue only then.
+// queued solve on the stream.  A caller that waits for the solve sees in host
+// memory whether it completed, and else takes the separate passes.  After a
+// lost solve the tracker takes the passes for a while.
 #pragma once
 
 #include <type_traits>
@@ -49,7 +50,7 @@ constexpr int kSolveBatch = 2;                    // slots of a thread whose row
 struct SolveXchg {
   unsigned epoch;  // of the last iteration of the last solve
   int ok;          // set when a solve completes, cleared by k_solve_rescue
-  unsigned lost;   // solves that k_solve_rescue took
+  unsigned rescued;  // solves that k_solve_rescue took
   int pad[29];
   unsigned long long pose[32];  // float pose (12) and warp (12) of the next iteration
   unsigned long long stat[kRedGroups][4];
@@ -62,7 +63,7 @@ struct HostState {
   TrackState s;
   int ok;          // the solve completed
   unsigned ended;  // number of the tracker's last one-launch solve that has ended
-  unsigned lost;   // its one-launch solves whose workgroups did not meet
+  unsigned rescued;  // its queued solves that the rescue took
 };
 
 struct SolveArgs {

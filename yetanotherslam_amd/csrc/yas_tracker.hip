@@ -43,9 +43,16 @@ using namespace yas;
 
 constexpr int kMaxSolveDevices = 64;
 constexpr long long kSolveMaxPixels = 1 << 26;  // 32-bit byte offsets in yas_solve_dev.hpp
-// 20 ms: a solve takes under 0.5 ms, and its workgroups wait for a CU at
-// most as long as other streams' kernels hold one.
+// 20 ms: between two words that a workgroup waits for lies at most an
+// iteration (16 us at 640x480, 0.8 ms at 4096x3072, 4 ms at kSolveMaxPixels),
+// and its workgroups wait for a CU at most as long as other kernels hold one.
 constexpr unsigned long long kSolveWaitTicks = 2000000ull;
+// Solves that are separate passes after one that was lost, twice as many after
+// the next loss, up to kMaxPasses; a solve in one launch begins anew.  A lost
+// solve costs its wait and, queued, the rescue (3.4 ms at 320x240 with depth
+// alone, 65 ms at 640x480 with both terms); the passes cost 0.03 to 0.11 ms a
+// solve more than the one launch (150 / 180 us and 306 / 415 us waited for).
+constexpr int kFirstPasses = 64, kMaxPasses = 8192;
 
 namespace {
 
@@ -121,17 +128,21 @@ __global__ void __launch_bounds__(kSolveThreads) k_solve(SolveArgs a) {
   solve_body<ICP, RGB>(solve_lds(), a);
 }
 // Takes a solve whose workgroups did not meet; nothing to do otherwise, but to
-// say in host memory that solve `number` has ended (and how many were lost).
+// say in host memory that solve `number` has ended (and how many it took).
 template <bool ICP, bool RGB>
 __global__ void __launch_bounds__(256) k_solve_rescue(SolveArgs a, HostState* host, unsigned number) {
   if (threadIdx.x == 0) {
     if (!a.x->ok) {
-      a.x->lost++;
-      __hip_atomic_store(&host->lost, a.x->lost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      a.x->rescued++;
+      __hip_atomic_store(&host->rescued, a.x->rescued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __hip_atomic_store(&host->ended, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   solve_rescue<ICP, RGB>(a);
+}
+// The epochs that a lost solve may have used are skipped.
+__global__ void k_solve_skip(SolveXchg* x, unsigned iterations) {
+  if (threadIdx.x == 0) x->epoch += iterations;
 }
 // All levels of an image, a depth image or a model in one launch (yas_frame_dev.hpp).
 __global__ void __launch_bounds__(256) k_image_levels(ImageArgs<SrcF32> a) {
@@ -169,7 +180,10 @@ struct yas_tracker {
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
   unsigned solves;               // one-launch solves launched
+  unsigned lost_waited;          // those lost that were waited for (the others: host_st->rescued)
   unsigned by_passes;            // solves that were separate passes from the start
+  unsigned lost_seen, solves_seen;  // lost solves known, and solves launched when the last was found
+  int passes_left, passes_next;  // solves to take by passes, and after the next loss
   float sin2_max, dist2_max;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
   float* raw_image;  // intensity uploaded by the host-image setters
@@ -257,7 +271,6 @@ static int launch_iteration(yas_tracker* t, int l, bool icp, bool rgb, bool do_s
 // i - 1 and writes the other one, and the ICP partial rows alternate the
 // same way, since that pass 1 reads the previous rows while writing its own.
 static int solve_by_passes(yas_tracker* t) {
-  t->by_passes++;
   const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
   hipStream_t s = t->ctx->stream;
   TrackState* S[2] = {t->st, t->st2};
@@ -391,6 +404,32 @@ static void launch_rescue(yas_tracker* t) {
   else hipLaunchKernelGGL((k_solve_rescue<false, true>), one, threads, 0, s, a, h, t->solves);
 }
 
+static unsigned lost_solves(const yas_tracker* t) {
+  return t->lost_waited + __atomic_load_n(&t->host_st->rescued, __ATOMIC_ACQUIRE);
+}
+// Whether the tracker's last solves let the next one be tried as one launch.
+// Its workgroups do not meet while something keeps them off a CU that nothing
+// here can ask for (another process, an application's kernels), and then the
+// next solve's mostly don't either.  Queued solves are found lost when their
+// rescue has run.
+static bool may_try(yas_tracker* t) {
+  const bool ended = solve_ended(t);
+  const unsigned lost = lost_solves(t);
+  if (lost != t->lost_seen) {
+    t->lost_seen = lost;
+    if (t->solves != t->solves_seen) {  // else of the solves queued behind one found before
+      t->solves_seen = t->solves;
+      t->passes_left = t->passes_next;
+      t->passes_next = std::min(2 * t->passes_next, kMaxPasses);
+    }
+  } else if (ended && t->solves != t->solves_seen) {
+    t->passes_next = kFirstPasses;
+  }
+  if (t->passes_left == 0) return true;
+  t->passes_left--;
+  return false;
+}
+
 // The solve in one launch from `init` (null: the state's pose), its result to
 // `host` too when not null; `done` tells whether this solve may run so (else
 // nothing is launched).
@@ -406,7 +445,7 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
                                                                         : (const void*)k_solve<false, true>;
   if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels ||
       t->H > kFastRows || is_capturing(s) ||
-      !solve_fits(device, kernel, grid)) return YAS_OK;
+      !solve_fits(device, kernel, grid) || !may_try(t)) return YAS_OK;
   std::lock_guard<std::mutex> lk(g_solve_mu);
   auto& last = g_solve_last[device];
   // (the per-thread stream's handle is not one stream)
@@ -431,7 +470,10 @@ int yas_tracker_solve_async(yas_tracker* t) {
   bool done;
   int rc = solve_in_one(t, nullptr, nullptr, done);
   if (rc) return rc;
-  if (!done) return solve_by_passes(t);
+  if (!done) {
+    t->by_passes++;
+    return solve_by_passes(t);
+  }
   launch_rescue(t);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
@@ -439,8 +481,9 @@ int yas_tracker_solve_async(yas_tracker* t) {
 
 // A solve from `init`, waited for; its state is left in host_st->s.  The one
 // launch takes the pose as an argument and leaves its result in host memory,
-// so the state's initialisation, the rescue and the result's copy, 4 to 5 us
-// each, are launched only where it did not run or did not complete.
+// so the state's initialisation and the result's copy, 4 to 5 us each, are
+// launched only where it did not run or did not complete, and then with the
+// separate passes.
 static int solve_and_wait(yas_tracker* t, const Mat44& init) {
   hipStream_t s = t->ctx->stream;
   t->host_st->ok = 0;
@@ -452,14 +495,17 @@ static int solve_and_wait(yas_tracker* t, const Mat44& init) {
     __atomic_store_n(&t->host_st->ended, t->solves, __ATOMIC_RELEASE);
     if (t->host_st->ok) return YAS_OK;
   }
+  if (done) {
+    unsigned iterations = 0;
+    for (int l = 0; l < t->P.levels; ++l) iterations += t->P.iters[l] > 0 ? t->P.iters[l] : 0;
+    hipLaunchKernelGGL(k_solve_skip, dim3(1), dim3(64), 0, s, t->xchg, iterations);
+    t->lost_waited++;
+  } else {
+    t->by_passes++;
+  }
   hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, s, t->st, init);
   YAS_LAUNCH_CHECK();
-  if (done) {
-    launch_rescue(t);
-    YAS_LAUNCH_CHECK();
-  } else if ((rc = solve_by_passes(t))) {
-    return rc;
-  }
+  if ((rc = solve_by_passes(t))) return rc;
   YAS_HIP(hipMemcpyAsync(&t->host_st->s, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, s));
   YAS_HIP(hipStreamSynchronize(s));
   return YAS_OK;
@@ -470,6 +516,11 @@ extern "C" {
 int yas_tracker_set_wait_ticks(yas_tracker* t, unsigned long long ticks) {
   YAS_REQUIRE(t, "null tracker");
   t->wait_ticks = ticks;
+  // the next solve is tried as if none had been lost
+  t->lost_seen = lost_solves(t);
+  t->solves_seen = t->solves;
+  t->passes_left = 0;
+  t->passes_next = kFirstPasses;
   return YAS_OK;
 }
 
@@ -477,7 +528,7 @@ int yas_tracker_solve_routes(yas_tracker* t, int routes[3]) {
   YAS_REQUIRE(t && routes, "yas_tracker_solve_routes: null argument");
   YAS_HIP(hipSetDevice(t->ctx->device));
   YAS_HIP(hipStreamSynchronize(t->ctx->stream));
-  const unsigned lost = __atomic_load_n(&t->host_st->lost, __ATOMIC_ACQUIRE);
+  const unsigned lost = lost_solves(t);
   routes[0] = (int)(t->solves - lost);
   routes[1] = (int)lost;
   routes[2] = (int)t->by_passes;
@@ -579,6 +630,7 @@ int yas_tracker_create(yas_ctx* ctx, int W, int H, const double K[4], const yas_
   t->sin2_max = largest_square((float)std::sin(20.f * 3.14159254f / 180.f), false);
   t->dist2_max = largest_square(0.01f, true);
   t->wait_ticks = kSolveWaitTicks;
+  t->passes_next = kFirstPasses;
   hipError_t e = hipSuccess;
   auto alloc = [&](void** p, size_t bytes) {
     if (e == hipSuccess) e = hipMalloc(p, bytes);

@@ -71,6 +71,7 @@ inline void launch_timed(F kernel, dim3 grid, dim3 block, hipStream_t s, const h
 
 struct yas_ctx {
   int device;
+  int cus;  // compute units that the stream's kernels run on
   hipStream_t stream;
   bool own_stream;
   std::atomic<int> refs;  // the creator's reference plus one per object built on it

@@ -40,6 +40,21 @@ void yas_set_error(const char* fmt, ...) {
   g_last_error = buf;
 }
 
+// The CUs that a stream's kernels run on: those of its mask (of all bits, where
+// it was made without one), of the device's or its partition's.
+static int stream_cus(int device, hipStream_t s, int* out) {
+  int all = 0;
+  YAS_HIP(hipDeviceGetAttribute(&all, hipDeviceAttributeMultiprocessorCount, device));
+  uint32_t mask[32] = {};
+  int n = 0;
+  if (hipExtStreamGetCUMask(s, 32, mask) == hipSuccess)
+    for (uint32_t w : mask) n += __builtin_popcount(w);
+  else
+    (void)hipGetLastError();
+  *out = n > 0 && n < all ? n : all;
+  return YAS_OK;
+}
+
 extern "C" {
 
 const char* yas_version(void) { return "yas-mi355x 0.1.0 (gfx950)"; }
@@ -66,6 +81,11 @@ int yas_ctx_create(int device, void* stream, yas_ctx** out) {
     }
     c->own_stream = true;
   }
+  const int rc = stream_cus(device, c->stream, &c->cus);
+  if (rc) {
+    yas_ctx_release(c);
+    return rc;
+  }
   *out = c;
   return YAS_OK;
 }
@@ -81,6 +101,11 @@ int yas_ctx_create_null_stream(int device, yas_ctx** out) {
   c->refs.store(1);
   c->stream = nullptr;  // the device's null stream
   c->own_stream = false;
+  const int rc = stream_cus(device, c->stream, &c->cus);
+  if (rc) {
+    delete c;
+    return rc;
+  }
   *out = c;
   return YAS_OK;
 }

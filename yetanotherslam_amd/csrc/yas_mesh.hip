@@ -713,7 +713,6 @@ struct yas_mesher {
   uint16_t* vinfo;  // per voxel (local vertex prefix << 3 | owned edges)
   int* nbr;         // per block, pool indices of it and its 7 +x/+y/+z neighbours (-1 absent)
   int block_cap;
-  int cus;
   int num_blocks;
   int num_tri;
   int num_vert;
@@ -752,7 +751,7 @@ static int ensure_block_cap(yas_mesher* me, int need, int most) {
 static int emit_groups(yas_mesher* me, const void* kernel, int* groups) {
   int per = 0;
   YAS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, kMcThreads, 0));
-  const int all = (me->block_cap + kMcWaves - 1) / kMcWaves, fit = std::max(1, per) * me->cus;
+  const int all = (me->block_cap + kMcWaves - 1) / kMcWaves, fit = std::max(1, per) * me->ctx->cus;
   *groups = std::min(all, fit);
   return YAS_OK;
 }
@@ -850,7 +849,6 @@ int yas_mesher_create(yas_ctx* ctx, int max_triangles, yas_mesher** out) {
   if (e == hipSuccess) e = hipMalloc((void**)&me->done, sizeof(unsigned));
   // on the context's stream, which the null stream need not be in order with
   if (e == hipSuccess) e = hipMemsetAsync(me->done, 0, sizeof(unsigned), ctx->stream);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&me->cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
   if (e != hipSuccess) {
     yas_set_error("yas_mesher_create: %s", hipGetErrorString(e));
     yas_mesher_destroy(me);

@@ -67,9 +67,6 @@ __global__ void __launch_bounds__(256) k_march(MapView m, P pose, Intr K, int W,
   march_at<VT>(m, pose.T(), pose.Tinv(), K, W, H, cols, zmin, zmax, occ, vmap, vsinv, step_scale, rows, blockIdx.x);
 }
 
-// Workgroups of k_view: one per CU.
-constexpr int kViewGroups = 256;
-
 // Visibility and z-range cells, then the march (RayTraceEngine.cu:412-450):
 // cells zmin/zmax of (W/8)*(H/8), vertex map `vmap` dense W*H float4.  The
 // pose is T's, or with T null the map's pose pair on the device; the map's
@@ -79,12 +76,12 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
                              unsigned* zmin, unsigned* zmax, unsigned* occ, float4* vmap, hipEvent_t before_march,
                              const hipEvent_t* march_ev) {
   MapView v = yas_map_view(map);
-  const int cols = W / 8, rows = H / 8;
+  const int cols = W / 8, rows = H / 8, cus = yas_map_ctx(map)->cus;
   if (cols <= kViewCells) {
     // equal chunks of whole cell rows; the block list in slices, one
     // workgroup a CU in all
     const int most = kViewCells / cols, chunks = (rows + most - 1) / most, rows_per = (rows + chunks - 1) / chunks;
-    const int slices = chunks < kViewGroups ? kViewGroups / chunks : 1;
+    const int slices = chunks < cus ? cus / chunks : 1;
     hipLaunchKernelGGL(k_view<P>, dim3(slices * chunks), dim3(1024),
                        sizeof(unsigned) * (kOccWords + 2 * (size_t)rows_per * cols), s, v, pose, yas_map_intr(map), K, W, H,
                        cols, rows, zmin, zmax, occ, slices, chunks, rows_per);
@@ -99,7 +96,7 @@ static int launch_view_march(hipStream_t s, yas_map* map, const P& pose, const d
   if (before_march) YAS_HIP(hipEventRecord(before_march, s));
   const float vsinv = (float)(1.0 / (double)v.voxel_size);
   const float step_scale = v.trunc / v.voxel_size;
-  const int mr = march_rows(W, H);
+  const int mr = march_rows(W, H, cus);
   dim3 grid(march_tiles(W, H, mr));
   const float* zn = (const float*)zmin;
   const float* zf = (const float*)zmax;

@@ -561,14 +561,14 @@ __device__ inline void march_tile_at(const MapView& m, const PoseF& T, const Pos
 }
 
 // Rays of a wavefront, in rows of 8: as few as leave no wavefront waiting for
-// a place (6 a SIMD).  A wavefront pays at each iteration for whatever any of
+// a place (6 a SIMD, 24 a CU).  A wavefront pays at each iteration for whatever any of
 // its rays does, and the launch's time is its longest wavefront's: 16 rays
 // instead of 64 take 12 to 17 % off a 320x240 ray cast.  At 640x480, 32 rays
 // are from 12 % faster to 21 % slower, and at 1280x960 40 % slower.
-constexpr int kMarchWaves = 6 * 1024;
-inline int march_rows(int W, int H) {
+constexpr int kMarchWaves = 24;
+inline int march_rows(int W, int H, int cus) {
   int rows = 8;
-  while (rows > 1 && (long long)W * H <= (long long)kMarchWaves * 4 * rows) rows >>= 1;
+  while (rows > 1 && (long long)W * H <= (long long)kMarchWaves * cus * 4 * rows) rows >>= 1;
   return rows;
 }
 inline int march_tiles(int W, int H, int rows) { return ((W + 15) / 16) * ((H + 2 * rows - 1) / (2 * rows)); }

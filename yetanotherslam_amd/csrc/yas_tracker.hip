@@ -346,22 +346,21 @@ static void forget_solves(const yas_tracker* t) {
     if (last.owner == t) last.owner = nullptr;
 }
 
-static bool solve_fits(int device, const void* kernel, int grid) {
+static bool solve_fits(const yas_ctx* ctx, const void* kernel, int grid) {
   static std::mutex mu;
-  static int room[kMaxSolveDevices][3];  // workgroups that fit at once, + 1; 0 = not asked yet
-  int per_cu = 0, cus = 0;
+  static int room[kMaxSolveDevices][3];  // workgroups that fit on a CU at once, + 1; 0 = not asked yet
+  int per_cu = 0;
   const int k = kernel == (const void*)k_solve<true, true> ? 0 : kernel == (const void*)k_solve<true, false> ? 1 : 2;
   std::lock_guard<std::mutex> lk(mu);
-  int& r = room[device][k];
+  int& r = room[ctx->device][k];
   if (r == 0) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kSolveThreads, 0) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kSolveThreads, 0) != hipSuccess) {
       (void)hipGetLastError();
-      per_cu = cus = 0;
+      per_cu = 0;
     }
-    r = per_cu * cus + 1;
+    r = per_cu + 1;
   }
-  return grid <= r - 1;
+  return grid <= (r - 1) * ctx->cus;
 }
 
 static bool is_capturing(hipStream_t s) {
@@ -445,7 +444,7 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
                                                                         : (const void*)k_solve<false, true>;
   if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels ||
       t->H > kFastRows || is_capturing(s) ||
-      !solve_fits(device, kernel, grid) || !may_try(t)) return YAS_OK;
+      !solve_fits(t->ctx, kernel, grid) || !may_try(t)) return YAS_OK;
   std::lock_guard<std::mutex> lk(g_solve_mu);
   auto& last = g_solve_last[device];
   // (the per-thread stream's handle is not one stream)

@@ -478,6 +478,8 @@ int yas_map_fuse_u16(yas_map* m, const uint16_t* depth, size_t pitch, int W, int
   YAS_REQUIRE_ACTIVE(m);
   YAS_REQUIRE(W > 0 && H > 0 && pitch >= (size_t)W * sizeof(uint16_t), "yas_map_fuse_u16: bad image size");
   YAS_REQUIRE(depth_scale > 0.f, "yas_map_fuse_u16: depth_scale must be > 0");
+  // the limit of float images, which the conversion below makes of some
+  YAS_REQUIRE(depth_span_fits((size_t)W * sizeof(float), W, H), "depth image spans 4 GiB or more");
   YAS_HIP(hipSetDevice(m->ctx->device));
   // the kernels convert what they read, as (float)raw * (float)(1 / scale)
   if (depth_span_fits(pitch, W, H, 2u))

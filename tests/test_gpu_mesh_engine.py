@@ -42,3 +42,29 @@ def test_engine_made_while_the_null_stream_is_busy(gpu):
             for _ in range(2):
                 _same(e.MeshifyIndexed(m), want)
         torch.cuda.synchronize()
+
+
+def test_first_extraction_takes_the_records_it_needs(gpu):
+    """Device memory of an engine's first extraction: 2096 bytes a block and
+    little more; an engine that outgrows its records gets the same mesh."""
+    import torch
+    p = synth.params(width=320, height=240, theta0=0.7)
+    K = synth.intrinsics(p).astype(np.float32)
+    big = rf.MapStruct(K, 1 << 18, 1 << 17, 0.004, 0.3)
+    big.FuseU16(to_dev(synth.frame(p, 0)[0]), np.eye(4))
+    n = big.stats().num_allocated
+    assert n > 40000 and big.stats().flags == 0
+    small = _room()
+    used = []
+    for _ in range(2):
+        e = rf.MeshEngine(1 << 21)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        mesh = e.MeshifyIndexed(big)
+        used.append(free - torch.cuda.mem_get_info()[0])
+        e.close()
+    assert min(used) <= 2096 * n + (6 << 20), (used, n)
+    e = rf.MeshEngine(1 << 21)
+    _same(e.MeshifyIndexed(small), rf.MeshEngine(1 << 21).MeshifyIndexed(small))
+    _same(e.MeshifyIndexed(big), mesh)
+    _same(e.MeshifyIndexed(small), rf.MeshEngine(1 << 21).MeshifyIndexed(small))

@@ -108,9 +108,9 @@ __device__ inline float block_sum32(float (&v)[32], float* lds /* [nwaves * 32] 
 
 // a / d and b / d, correctly rounded, by one reciprocal: the refinement that
 // the division expands to, without the scaling that it does first, which these
-// positive counts (and their products) are far from needing.
-__device__ inline float2 count_quotients(float a, float b, float d) {
-  const float r0 = __builtin_amdgcn_rcpf(d);
+// positive counts (and their products) are far from needing.  `r0` is the
+// reciprocal to within an ulp.
+__host__ __device__ inline float2 count_quotients_from(float r0, float a, float b, float d) {
   const float r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
   auto quotient = [&](float x) {
     float q = x * r;
@@ -118,6 +118,9 @@ __device__ inline float2 count_quotients(float a, float b, float d) {
     return fmaf(fmaf(-d, q, x), r, q);
   };
   return make_float2(quotient(a), quotient(b));
+}
+__device__ inline float2 count_quotients(float a, float b, float d) {
+  return count_quotients_from(__builtin_amdgcn_rcpf(d), a, b, d);
 }
 // Chan et al.'s pairwise update of (count, mean, M2) statistics.  By selects:
 // a merge is a link of the solve's serial chain, some 18 to an iteration, and

@@ -460,7 +460,7 @@ int yas_tracker_solve6(yas_ctx* ctx, const float* H, const float* b, double* x, 
 /* The bound of the waits inside a one-launch solve, in ticks of the device's
  * 100 MHz clock (test access; 2000000 by default).  0 makes every wait that
  * finds its words missing at the first look give up.  A call also lets the
- * next solve be tried as one launch, whatever became of those before. */
+ * next solve be tried as one launch, whatever became of those before it. */
 int yas_tracker_set_wait_ticks(yas_tracker* trk, unsigned long long ticks);
 /* How many of this tracker's solves (GetTransform, pipeline frames) ran as
  * one launch, ran out of a wait as one launch and were taken again, and ran as

@@ -86,6 +86,7 @@ def _tracker(w, h, mode, iters=(10, 5, 3), ctx=None):
         (trk.SetReferenceDepth, trk.SetTrackingDepth)[t](z)
         (trk.SetReferenceImage, trk.SetTrackingImage)[t](g)
     trk._keep = keep
+    _ticks(trk.h, DEFAULT_TICKS)  # whatever other tests left
     return trk
 
 
@@ -215,3 +216,51 @@ def test_after_a_rescued_frame_come_passes(gpu, wait):
         pl.step(*frames[6 - i % 2])
         pl.pose(len(frames) + i)
     assert _routes(h)[1] == lost  # still by passes, once, however many were lost together
+
+
+def test_overlapping_solves_of_large_images_take_the_passes(gpu):
+    """Two cameras whose frames are enqueued without waiting: a one-launch
+    solve on every CU would hold up the other camera, so neither takes it while
+    their solves overlap, nor for 32 solves after; the poses are the same."""
+    import torch
+    size = dict(w=640, h=480)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    ref, frames = _pipeline(**size)
+    pls, hs = [], []
+    for q in streams:
+        with torch.cuda.stream(q):
+            pls.append(_pipeline(n=1, ctx=rf.Context(), **size)[0])
+        h = ctypes.c_void_p()
+        native.call("yas_pipeline_tracker", pls[-1].h, ctypes.byref(h))
+        hs.append(h)
+    for f in frames:
+        ref.step(*f)
+    want = _poses(ref)
+    _ticks(hs[0], DEFAULT_TICKS)  # whatever other tests left
+    x = torch.zeros(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+    for pl in pls:
+        pl.step(*frames[0])
+    for i in (1, 2):  # waited for one after the other: no overlap
+        for pl in pls:
+            pl.step(*frames[i])
+            pl.pose(i)
+    assert [_routes(h) for h in hs] == [[2, 0, 0]] * 2
+    for q in streams:
+        with torch.cuda.stream(q):
+            for _ in range(200):  # some 20 ms
+                x.add_(1.0)
+    for f in frames[3:]:
+        for pl in pls:
+            pl.step(*f)
+    torch.cuda.synchronize()
+    n = len(frames) - 3
+    # the first of all finds no other solve
+    assert [_routes(h) for h in hs] == [[3, 0, n - 1], [2, 0, n]]
+    for pl in pls:
+        assert np.array_equal(_poses(pl), want)
+    for i in range(33):  # alone again
+        assert _routes(hs[0]) == [3, 0, n - 1 + i]
+        pls[0].step(*frames[(6, 7)[i % 2]])
+        pls[0].pose(len(frames) + i)
+    assert _routes(hs[0]) == [4, 0, n - 1 + 32]

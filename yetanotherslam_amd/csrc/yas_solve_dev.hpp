@@ -26,7 +26,7 @@
 // before their first level.
 //
 // All workgroups must be resident at once.  The host takes this path only
-// when the device holds the grid, and for one stream at a time.  Every wait
+// when the device holds the grid, and for one solve at a time.  Every wait
 // is bounded by the clock all the same: a workgroup whose wait runs out
 // leaves, the tracker's state stays as it was before the solve, and
 // k_solve_rescue takes the whole solve in one workgroup with the
@@ -62,7 +62,7 @@ struct SolveXchg {
 struct HostState {
   TrackState s;
   int ok;          // the solve completed
-  unsigned ended;  // number of the tracker's last one-launch solve that has ended
+  unsigned ended;  // number of the tracker's last solve that has ended
   unsigned rescued;  // its queued solves that the rescue took
 };
 

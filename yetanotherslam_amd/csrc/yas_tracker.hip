@@ -106,8 +106,12 @@ __global__ void __launch_bounds__(256) k_update(TrackState* st, const float* par
                                                 float wrh, float wrb, float wih, float wib) {
   update_at(st, part_icp, gi, part_rgb, gr, mode, first_of_level, do_step, record, wrh, wrb, wih, wib);
 }
-// The last step of a solve, from the state buffer the last pass used into the tracker's state.
-__global__ void __launch_bounds__(256) k_update_into(const TrackState* st_in, TrackState* st_out, StepArgs a) {
+// The last step of a solve, from the state buffer the last pass used into the
+// tracker's state; in host memory (if `host`), that solve `number` has ended.
+__global__ void __launch_bounds__(256) k_update_into(const TrackState* st_in, TrackState* st_out, StepArgs a,
+                                                     HostState* host, unsigned number) {
+  if (host && threadIdx.x == 0)
+    __hip_atomic_store(&host->ended, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   gn_update(st_in, st_out, true, a.part_icp, a.gi, a.part_rgb, a.gr, a.mode, a.first_of_level, 1, a.record, a.wrh,
             a.wrb, a.wih, a.wib, nullptr);
 }
@@ -179,10 +183,13 @@ struct yas_tracker {
   HostState* host_st;
   SolveXchg* xchg;               // words the one-launch solve's workgroups exchange
   unsigned long long wait_ticks; // bound of its waits (100 MHz clock)
-  unsigned solves;               // one-launch solves launched
+  unsigned solves;               // number of the last solve enqueued (but those recorded into graphs)
+  bool listed, one;              // in its device's list (g_solves); the last solve is a one-launch solve
+  yas_tracker* next;             // in that list
+  unsigned tried, last_tried;    // one-launch solves launched, and the last one's number
   unsigned lost_waited;          // those lost that were waited for (the others: host_st->rescued)
   unsigned by_passes;            // solves that were separate passes from the start
-  unsigned lost_seen, solves_seen;  // lost solves known, and solves launched when the last was found
+  unsigned lost_seen, tried_seen;  // lost solves known, and solves tried when the last was found
   int passes_left, passes_next;  // solves to take by passes, and after the next loss
   float sin2_max, dist2_max;
   float* raw_depth;  // depth uploaded by the host-image setters (W*H, lazily allocated)
@@ -270,7 +277,7 @@ static int launch_iteration(yas_tracker* t, int l, bool icp, bool rgb, bool do_s
 // saves one launch per iteration.  Step i reads the state buffer of step
 // i - 1 and writes the other one, and the ICP partial rows alternate the
 // same way, since that pass 1 reads the previous rows while writing its own.
-static int solve_by_passes(yas_tracker* t) {
+static int solve_by_passes(yas_tracker* t, bool numbered) {
   const bool icp = t->P.mode != YAS_TRACK_RGB, rgb = t->P.mode != YAS_TRACK_DEPTH;
   hipStream_t s = t->ctx->stream;
   TrackState* S[2] = {t->st, t->st2};
@@ -319,31 +326,56 @@ static int solve_by_passes(yas_tracker* t) {
       a.record = l == 0 ? 1 : 0;
       a.wrh = t->P.w_rgb_h; a.wrb = t->P.w_rgb_b; a.wih = t->P.w_icp_h; a.wib = t->P.w_icp_b;
     }
-  if (i > 0) hipLaunchKernelGGL(k_update_into, dim3(1), dim3(256), 0, s, (const TrackState*)S[(i - 1) & 1], t->st, a);
+  if (i > 0)
+    hipLaunchKernelGGL(k_update_into, dim3(1), dim3(256), 0, s, (const TrackState*)S[(i - 1) & 1], t->st, a,
+                       numbered ? t->host_st : (HostState*)nullptr, t->solves);
   YAS_LAUNCH_CHECK();
   return YAS_OK;
 }
 
-// Whether this solve may run as one launch (k_solve): every workgroup must
-// find a CU at once, so only one stream's solves do at a time.  A stream
-// other than the last one's takes over once that solve has ended, which its
-// tracker's host memory says; until then its solves run as separate passes.
-// (Asking the runtime whether the other stream is idle breaks a capture in the
-// global mode that any thread may have begun.)  Solves recorded into a graph,
-// whose replays nothing here orders, run as separate passes too.
+// The solves of a device that have not ended, by tracker, as each tracker's
+// host memory says.  (Asking the runtime whether another stream is idle breaks
+// a capture in the global mode that any thread may have begun.)
 static std::mutex g_solve_mu;
 static struct {
-  yas_tracker* owner;  // of the last one-launch solve; null when it is gone
-  hipStream_t stream;  // only compared
-} g_solve_last[kMaxSolveDevices];
+  yas_tracker* head;
+  int crowded;  // solves since two streams' overlapped, counted down from kCrowd
+} g_solves[kMaxSolveDevices];
+constexpr int kCrowd = 32;
 
-static bool solve_ended(const yas_tracker* t) {
-  return __atomic_load_n(&t->host_st->ended, __ATOMIC_ACQUIRE) == t->solves;
+static void list_solve(yas_tracker* t, yas_tracker*& head) {
+  if (!t->listed) {
+    t->next = head;
+    head = t;
+    t->listed = true;
+  }
 }
 static void forget_solves(const yas_tracker* t) {
   std::lock_guard<std::mutex> lk(g_solve_mu);
-  for (auto& last : g_solve_last)
-    if (last.owner == t) last.owner = nullptr;
+  for (auto& d : g_solves)
+    for (yas_tracker** p = &d.head; *p; p = &(*p)->next)
+      if (*p == t) {
+        *p = t->next;
+        break;
+      }
+}
+// Whether solves of other streams than s are there, and one-launch solves among
+// them; those that have ended leave the list.
+static void other_solves(yas_tracker*& head, hipStream_t s, bool& any, bool& one) {
+  any = one = false;
+  for (yas_tracker** p = &head; *p;) {
+    yas_tracker* q = *p;
+    if (__atomic_load_n(&q->host_st->ended, __ATOMIC_ACQUIRE) == q->solves) {
+      *p = q->next;
+      q->listed = false;
+      continue;
+    }
+    if (q->ctx->stream != s || s == hipStreamPerThread) {  // (whose handle is not one stream)
+      any = true;
+      one |= q->one;
+    }
+    p = &q->next;
+  }
 }
 
 static bool solve_fits(const yas_ctx* ctx, const void* kernel, int grid) {
@@ -412,16 +444,16 @@ static unsigned lost_solves(const yas_tracker* t) {
 // next solve's mostly don't either.  Queued solves are found lost when their
 // rescue has run.
 static bool may_try(yas_tracker* t) {
-  const bool ended = solve_ended(t);
+  const bool ended = (int)(__atomic_load_n(&t->host_st->ended, __ATOMIC_ACQUIRE) - t->last_tried) >= 0;
   const unsigned lost = lost_solves(t);
   if (lost != t->lost_seen) {
     t->lost_seen = lost;
-    if (t->solves != t->solves_seen) {  // else of the solves queued behind one found before
-      t->solves_seen = t->solves;
+    if (t->tried != t->tried_seen) {  // else of the solves queued behind one found before
+      t->tried_seen = t->tried;
       t->passes_left = t->passes_next;
       t->passes_next = std::min(2 * t->passes_next, kMaxPasses);
     }
-  } else if (ended && t->solves != t->solves_seen) {
+  } else if (ended && t->tried != t->tried_seen) {
     t->passes_next = kFirstPasses;
   }
   if (t->passes_left == 0) return true;
@@ -430,25 +462,44 @@ static bool may_try(yas_tracker* t) {
 }
 
 // The solve in one launch from `init` (null: the state's pose), its result to
-// `host` too when not null; `done` tells whether this solve may run so (else
-// nothing is launched).
-static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool& done) {
+// `host` too when not null, where it may run so (`one`, else nothing is
+// launched).  Solves recorded into a graph, whose replays nothing here orders,
+// may not; the others are numbered.
+//
+// All workgroups must find a CU at once, so no two one-launch solves run
+// together.  One that takes more than half of the CUs also keeps other streams'
+// kernels waiting (k_view, which needs half of a CU's LDS, above all), so while
+// solves of several streams overlap they all take the passes: two cameras of
+// 640x480 with both terms 3076 frames/s, four 4820; with one of the streams in
+// one launch 2590 and 3830, and one camera alone 2080 against 1695 by passes.
+// At 320x240 (75 workgroups) two cameras take 3850 against 3970 frames/s, but
+// four that one thread enqueues 6900 against 5550.
+static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool& one, bool& numbered) {
   hipStream_t s = t->ctx->stream;
   const int device = t->ctx->device, mode = t->P.mode;
   int grid = 0;
   for (int l = t->P.levels - 1; l >= 0; --l)
     if (t->P.iters[l] > 0) grid = groups_for(t->lv[l]);
-  done = false;
+  one = numbered = false;
+  if (grid == 0 || device >= kMaxSolveDevices || is_capturing(s)) return YAS_OK;
   const void* kernel = mode == YAS_TRACK_RGBD ? (const void*)k_solve<true, true>
                                               : mode == YAS_TRACK_DEPTH ? (const void*)k_solve<true, false>
                                                                         : (const void*)k_solve<false, true>;
-  if (grid == 0 || device >= kMaxSolveDevices || (long long)t->W * t->H > kSolveMaxPixels ||
-      t->H > kFastRows || is_capturing(s) ||
-      !solve_fits(t->ctx, kernel, grid) || !may_try(t)) return YAS_OK;
+  bool may = (long long)t->W * t->H <= kSolveMaxPixels && t->H <= kFastRows && solve_fits(t->ctx, kernel, grid) &&
+             may_try(t);
   std::lock_guard<std::mutex> lk(g_solve_mu);
-  auto& last = g_solve_last[device];
-  // (the per-thread stream's handle is not one stream)
-  if (last.owner && (last.stream != s || s == hipStreamPerThread) && !solve_ended(last.owner)) return YAS_OK;
+  auto& d = g_solves[device];
+  bool others, other_one;
+  other_solves(d.head, s, others, other_one);
+  if (2 * grid <= t->ctx->cus) may &= !other_one;
+  else may &= !others && d.crowded == 0;
+  if (others) d.crowded = kCrowd;
+  else if (d.crowded > 0) d.crowded--;
+  t->solves++;
+  t->one = may;
+  list_solve(t, d.head);
+  numbered = true;
+  if (!may) return YAS_OK;
   SolveArgs a = solve_args(t);
   if (init) a.init = *init;
   a.has_init = init != nullptr;
@@ -458,20 +509,19 @@ static int solve_in_one(yas_tracker* t, const Mat44* init, HostState* host, bool
   else if (mode == YAS_TRACK_DEPTH) hipLaunchKernelGGL((k_solve<true, false>), dim3(grid), threads, 0, s, a);
   else hipLaunchKernelGGL((k_solve<false, true>), dim3(grid), threads, 0, s, a);
   YAS_LAUNCH_CHECK();
-  last.owner = t;
-  last.stream = s;
-  t->solves++;
-  done = true;
+  t->tried++;
+  t->last_tried = t->solves;
+  one = true;
   return YAS_OK;
 }
 
 int yas_tracker_solve_async(yas_tracker* t) {
-  bool done;
-  int rc = solve_in_one(t, nullptr, nullptr, done);
+  bool one, numbered;
+  int rc = solve_in_one(t, nullptr, nullptr, one, numbered);
   if (rc) return rc;
-  if (!done) {
+  if (!one) {
     t->by_passes++;
-    return solve_by_passes(t);
+    return solve_by_passes(t, numbered);
   }
   launch_rescue(t);
   YAS_LAUNCH_CHECK();
@@ -486,15 +536,15 @@ int yas_tracker_solve_async(yas_tracker* t) {
 static int solve_and_wait(yas_tracker* t, const Mat44& init) {
   hipStream_t s = t->ctx->stream;
   t->host_st->ok = 0;
-  bool done;
-  int rc = solve_in_one(t, &init, t->host_st, done);
+  bool one, numbered;
+  int rc = solve_in_one(t, &init, t->host_st, one, numbered);
   if (rc) return rc;
-  if (done) {
+  if (one) {
     YAS_HIP(hipStreamSynchronize(s));
-    __atomic_store_n(&t->host_st->ended, t->solves, __ATOMIC_RELEASE);
-    if (t->host_st->ok) return YAS_OK;
-  }
-  if (done) {
+    if (t->host_st->ok) {
+      __atomic_store_n(&t->host_st->ended, t->solves, __ATOMIC_RELEASE);
+      return YAS_OK;
+    }
     unsigned iterations = 0;
     for (int l = 0; l < t->P.levels; ++l) iterations += t->P.iters[l] > 0 ? t->P.iters[l] : 0;
     hipLaunchKernelGGL(k_solve_skip, dim3(1), dim3(64), 0, s, t->xchg, iterations);
@@ -504,7 +554,7 @@ static int solve_and_wait(yas_tracker* t, const Mat44& init) {
   }
   hipLaunchKernelGGL(k_track_init, dim3(1), dim3(64), 0, s, t->st, init);
   YAS_LAUNCH_CHECK();
-  if ((rc = solve_by_passes(t))) return rc;
+  if ((rc = solve_by_passes(t, numbered))) return rc;
   YAS_HIP(hipMemcpyAsync(&t->host_st->s, t->st, sizeof(TrackState), hipMemcpyDeviceToHost, s));
   YAS_HIP(hipStreamSynchronize(s));
   return YAS_OK;
@@ -515,9 +565,13 @@ extern "C" {
 int yas_tracker_set_wait_ticks(yas_tracker* t, unsigned long long ticks) {
   YAS_REQUIRE(t, "null tracker");
   t->wait_ticks = ticks;
-  // the next solve is tried as if none had been lost
+  // the next solve is tried as if none had been lost or had overlapped another
+  if (t->ctx->device < kMaxSolveDevices) {
+    std::lock_guard<std::mutex> lk(g_solve_mu);
+    g_solves[t->ctx->device].crowded = 0;
+  }
   t->lost_seen = lost_solves(t);
-  t->solves_seen = t->solves;
+  t->tried_seen = t->tried;
   t->passes_left = 0;
   t->passes_next = kFirstPasses;
   return YAS_OK;
@@ -528,7 +582,7 @@ int yas_tracker_solve_routes(yas_tracker* t, int routes[3]) {
   YAS_HIP(hipSetDevice(t->ctx->device));
   YAS_HIP(hipStreamSynchronize(t->ctx->stream));
   const unsigned lost = lost_solves(t);
-  routes[0] = (int)(t->solves - lost);
+  routes[0] = (int)(t->tried - lost);
   routes[1] = (int)lost;
   routes[2] = (int)t->by_passes;
   return YAS_OK;

@@ -174,30 +174,38 @@ struct yas_pipeline {
   int cap;
 };
 
+// Room for twice the frames; the arrays there are stay until all new ones are
+// filled.
 static int grow(yas_pipeline* p) {
-  int ncap = p->cap ? p->cap * 2 : 1024;
+  const int ncap = p->cap ? p->cap * 2 : 1024;
+  hipStream_t s = p->ctx->stream;
   double* np = nullptr;
-  int* nt = nullptr;
-  YAS_HIP(hipHostMalloc((void**)&np, sizeof(double) * 16 * (size_t)ncap, hipHostMallocDefault));
-  YAS_HIP(hipHostMalloc((void**)&nt, sizeof(int) * (size_t)ncap, hipHostMallocDefault));
+  int *nt = nullptr, *ns = nullptr;
+  hipError_t e = hipHostMalloc((void**)&np, sizeof(double) * 16 * (size_t)ncap, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&nt, sizeof(int) * (size_t)ncap, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipMalloc((void**)&ns, sizeof(int) * 8 * (size_t)ncap);
+  if (e == hipSuccess) e = hipMemsetAsync(ns, 0, sizeof(int) * 8 * (size_t)ncap, s);
+  if (e == hipSuccess && p->cap) {
+    e = hipMemcpyAsync(ns, p->frame_stats, sizeof(int) * 8 * (size_t)p->cap, hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+  }
+  if (e != hipSuccess) {
+    if (np) hipHostFree(np);
+    if (nt) hipHostFree(nt);
+    hipFree(ns);
+    yas_set_error("yas_pipeline: room for %d frames: %s", ncap, hipGetErrorString(e));
+    return YAS_E_HIP;
+  }
   if (p->cap) {
-    YAS_HIP(hipStreamSynchronize(p->ctx->stream));
     std::memcpy(np, p->poses, sizeof(double) * 16 * (size_t)p->cap);
     std::memcpy(nt, p->tracked, sizeof(int) * (size_t)p->cap);
     hipHostFree(p->poses);
     hipHostFree(p->tracked);
-  }
-  int* ns = nullptr;
-  YAS_HIP(hipMalloc((void**)&ns, sizeof(int) * 8 * (size_t)ncap));
-  YAS_HIP(hipMemsetAsync(ns, 0, sizeof(int) * 8 * (size_t)ncap, p->ctx->stream));
-  if (p->cap) {
-    YAS_HIP(hipMemcpyAsync(ns, p->frame_stats, sizeof(int) * 8 * p->cap, hipMemcpyDeviceToDevice, p->ctx->stream));
-    YAS_HIP(hipStreamSynchronize(p->ctx->stream));
     hipFree(p->frame_stats);
   }
-  p->frame_stats = ns;
   p->poses = np;
   p->tracked = nt;
+  p->frame_stats = ns;
   p->cap = ncap;
   return YAS_OK;
 }

@@ -15,9 +15,9 @@
 // The hash is open addressing with linear probing from the reference hash's
 // home slot.  Insertion is lock-free: a 64-bit compare-and-swap claims a free
 // slot for a key; within a wavefront, lanes carrying the same block key are
-// reduced to one leader with ballots before any memory traffic, and new
-// blocks take pool indices from one atomic per wavefront.  The resulting set
-// of allocated blocks does not depend on the order of insertion.
+// reduced to one leader with ballots before any memory traffic, and the new
+// blocks of a workgroup take their pool indices from one atomic.  The resulting
+// set of allocated blocks does not depend on the order of insertion.
 #include <cstdarg>
 #include <cstring>
 #include <mutex>

@@ -310,14 +310,15 @@ struct VoxelReader {
     return flags == kBlockFree ? -1 : blk;
   }
   // The 7 remaining corners: corner c is (c&1 ? x1 : x0, c&2 ? y1 : y0,
-  // c&4 ? z1 : z0).  When at most one axis's two corners straddle a block
-  // face (nearly every call), the corners lie in corner 0's block, which is
-  // cached, and at most one other, looked up once; then the voxel loads of
-  // all 7 corners are issued before any is used.  Read one by one through
-  // the one-entry cache they made a chain of dependent loads, with a lookup
-  // per read when the corners alternate between two blocks.  Corners
-  // spread over more blocks take the reads in turn.  The values and the
-  // arithmetic order are those of 8 reads in the reference's order.
+  // c&4 ? z1 : z0).  When the corners straddle a block face along at most two
+  // axes (nearly every call), they lie in corner 0's block, which is cached,
+  // and one other, looked up once, or three others, looked up with their first
+  // probes in flight together; then the voxel loads of all 7 corners are issued
+  // before any is used.  Read one by one through the one-entry cache they made
+  // a chain of dependent loads, with a lookup per read when the corners
+  // alternate between blocks.  Corners over three faces take the reads in turn.
+  // The values and the arithmetic order are those of 8 reads in the
+  // reference's order.
   __device__ inline float interp_rest(float x, float y, float z, int x0, int y0, int z0, float s0, bool vp,
                                       bool& valid) {
     const float fx = x - floorf(x), fy = y - floorf(y), fz = z - floorf(z);

@@ -3,9 +3,10 @@
 // image operations it uses (RGBDFusion/src/ImageProc.cu).
 //
 // MI355X design: the whole Gauss-Newton loop stays on the device, with no
-// host round trip and no grid-wide synchronisation inside a kernel (on the
-// multi-XCD gfx950 an agent-scope fence writes back the L2, so kernel
-// boundaries are the cheaper barrier).  One iteration is:
+// host round trip and no fence inside a kernel (on the multi-XCD gfx950 an
+// agent-scope fence writes back the L2): the separate passes meet at kernel
+// boundaries, and the workgroups of the one-launch solve wait for each other's
+// words, which carry their iteration.  One iteration is:
 //   pass 1   grid-stride over the level's pixels: ICP point-to-plane rows
 //            (28 upper-triangle products + count) and photometric residuals
 //            with per-thread Welford statistics; each workgroup reduces its
@@ -18,10 +19,11 @@
 //            the 6x6 system in FP64 (the reference's Eigen LDLT, restated),
 //            applies T <- exp(xi) T in FP64 and keeps the best pose.
 // A full solve runs all of its iterations in one launch (k_solve,
-// yas_solve_dev.hpp) where its workgroups can be resident at once; otherwise
-// it takes each update but the last at the start of the next pass 1: every
-// workgroup of that pass folds the same rows and takes the same step, one
-// launch fewer per iteration.  The values are the same either way.
+// yas_solve_dev.hpp) where its workgroups can be resident at once
+// (solve_in_one says when); otherwise it takes each update but the last at the
+// start of the next pass 1: every workgroup of that pass folds the same rows
+// and takes the same step, one launch fewer per iteration.  The values are the
+// same either way.
 // Results are deterministic run to run.
 #include <algorithm>
 #include <cfloat>

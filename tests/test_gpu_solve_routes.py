@@ -126,7 +126,7 @@ def test_a_stream_beside_a_busy_one_takes_the_passes(gpu):
     torch.cuda.synchronize()
     pl.step(*fr[0])
     with torch.cuda.stream(s[0]):
-        for _ in range(200):  # some 20 ms, then a solve
+        for _ in range(600):  # some 60 ms, then a solve
             x.add_(1.0)
     pl.step(*fr[1])
     got = _solve(trks[1])
@@ -248,7 +248,7 @@ def test_overlapping_solves_of_large_images_take_the_passes(gpu):
     assert [_routes(h) for h in hs] == [[2, 0, 0]] * 2
     for q in streams:
         with torch.cuda.stream(q):
-            for _ in range(200):  # some 20 ms
+            for _ in range(600):  # some 60 ms
                 x.add_(1.0)
     for f in frames[3:]:
         for pl in pls:
